@@ -235,7 +235,20 @@ struct afq_job {
   // three bf16 planes (k_split_e1_bf16)
   uint16_t* e1s[2] = {nullptr, nullptr};
   uint16_t* vsplit = nullptr;             // (W, 4, 16 ceil(N/16), 32 ceil(N/32)) split VHS planes
-  // nocc > 64: stored f blocks of the wide exchange path (k_exchange_wide)
+  // FP64 exchange over the trial's unoccupied orbitals (exchange_f64.hip), per
+  // spin: Q, P from the trial; packed rot_chol Q, tr f0, M^T and K0 from
+  // rot_chol.  Null where another exchange runs (x_f64).
+  double* xq_q[2] = {nullptr, nullptr};   // (N, N - nocc)
+  double* xq_p[2] = {nullptr, nullptr};   // (N, nocc)
+  double* xq_a[2] = {nullptr, nullptr};
+  double* xq_c0[2] = {nullptr, nullptr};  // (G,)
+  double* xq_mt[2] = {nullptr, nullptr};  // (nocc, N - nocc)
+  double* xq_k0[2] = {nullptr, nullptr};  // (1,)
+  double2* xq_b[2] = {nullptr, nullptr};  // packed theta (one buffer for both spins unless the job is small)
+  double* xq_kg = nullptr;                // (G,) setup scratch
+  double* xq_tmp = nullptr;               // setup scratch
+  bool rc_set[2] = {false, false};        // rot_chol has been built or supplied
+  // nocc > 128: stored f blocks of the wide exchange path (k_exchange_wide)
   double2* xwide = nullptr;
   long xwide_elems = 0;
   // symmetric Cholesky vectors: the VHS product over block-packed columns

@@ -5,6 +5,7 @@
 #include <cstring>
 #include <string>
 
+#include "exchange_f64.h"
 #include "gemm_bf3.h"
 #include "group.h"
 #include "kernels.h"
@@ -85,6 +86,18 @@ void release(afq_job* j) {
   fr(j->e1s[0]);
   fr(j->e1s[1]);
   fr(j->vsplit);
+  for (int s = 0; s < (j->rhf ? 1 : 2); ++s) {
+    fr(j->xq_q[s]);
+    fr(j->xq_p[s]);
+    fr(j->xq_a[s]);
+    fr(j->xq_c0[s]);
+    fr(j->xq_mt[s]);
+    fr(j->xq_k0[s]);
+  }
+  fr(j->xq_b[0]);
+  if (j->xq_b[1] != j->xq_b[0]) fr(j->xq_b[1]);
+  fr(j->xq_kg);
+  fr(j->xq_tmp);
   fr(j->xwide);
   fr(j->t32[0]);
   fr(j->t32[1]);
@@ -295,6 +308,24 @@ int force_bias_gemm(afq_job* j, double2* out, hipStream_t st) {
   return AFQ_OK;
 }
 
+// Spins whose exchange runs in FP64 over the unoccupied orbitals: FP64 jobs,
+// and above 64 occupied orbitals the reduced-precision ones too.
+bool x_f64(const afq_job* j, int s) {
+  return j->nocc[s] <= kExchangeF64MaxO && (!j->lp || j->nocc[s] > kExchangeRegMaxO);
+}
+
+// Rebuilds the parts of that exchange that follow from the trial, and from
+// rot_chol once there is one.
+int x_f64_trial(afq_job* j, int s, hipStream_t st) {
+  return exchange_f64_set_trial(j->mo[s], j->N, j->nocc[s], j->xq_q[s], j->xq_p[s], j->xq_tmp, j->gemm_ws,
+                                j->gemm_ws_elems, st);
+}
+int x_f64_chol(afq_job* j, int s, hipStream_t st) {
+  return exchange_f64_set_chol(j->rot_chol[s], j->xq_q[s], j->xq_p[s], j->N, j->nocc[s], j->G, j->xq_a[s],
+                               j->xq_c0[s], j->xq_mt[s], j->xq_k0[s], j->xq_kg, j->xq_tmp, j->gemm_ws,
+                               j->gemm_ws_elems, st);
+}
+
 int energy_pipeline(afq_job* j, const void* up, const void* dn, double2* out, hipStream_t st, bool have_green) {
   if (!have_green) AFQ_TRY(green_pipeline(j, up, dn, true, true, st));
   const bool two = !j->one_spin;
@@ -327,11 +358,13 @@ int energy_pipeline(afq_job* j, const void* up, const void* dn, double2* out, hi
       continue;
     }
     ProfScope ps(j, AFQ_K_EXCHANGE, st);
-    if (j->nocc[s] > kExchangeRegMaxO)
+    if (x_f64(j, s))  // theta in the SR gather buffer
+      AFQ_TRY(k_exchange_f64(j->xq_a[s], j->xq_q[s], j->xq_c0[s], j->xq_mt[s], j->xq_k0[s],
+                             j->green[s], j->wgather,
+                             j->xq_b[s], j->nocc[s], j->N, j->G, j->W, coul, kpart, &nch[s], st));
+    else
       AFQ_TRY(k_exchange_wide(j->rot_chol[s], j->green[s], j->nocc[s], j->N, j->G, j->W, j->xwide, j->xwide_elems,
                               coul, kpart, &nch[s], st));
-    else
-      AFQ_TRY(k_exchange(j->rot_chol[s], j->green[s], j->nocc[s], j->N, j->G, j->W, coul, kpart, &nch[s], st));
   }
   ProfScope ps(j, AFQ_K_ENERGY_MISC, st);
   return k_energy_finalize(j->ene1, j->coul, two ? j->coul + (long)j->W * j->G : nullptr, j->kpart,
@@ -877,6 +910,8 @@ void init_job(afq_job* j, const afq_job_desc* d) {
   j->lp = d->precision != AFQ_PREC_FP64;
   j->bf16x3 = d->precision == AFQ_PREC_BF16X3;
   j->kchunk_max = exchange_nchunk(j->G);
+  for (int s = 0; s < 2; ++s)
+    if (x_f64(j, s)) j->kchunk_max = std::max(j->kchunk_max, exchange_f64_nchunk(j->nocc[s], j->G) + 1);
 }
 
 // Allocates every device buffer of the job (dry: only sums the bytes).
@@ -915,7 +950,27 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
     A_(j->green[s], W * O * N);
   }
   const int omax = std::max(j->nocc[0], j->nocc[1]);
-  if (omax > kExchangeRegMaxO) {
+  {
+    long tmp = 0, nb = 0;
+    for (int s = 0; s < (j->rhf ? 1 : 2); ++s) {
+      const int O = j->nocc[s];
+      if (!x_f64(j, s)) continue;
+      A_(j->xq_q[s], N * (N - O));
+      A_(j->xq_p[s], N * O);
+      A_(j->xq_a[s], exchange_f64_a_elems(O, (int)N, (int)G));
+      A_(j->xq_c0[s], G);
+      A_(j->xq_mt[s], (N - O) * O);
+      A_(j->xq_k0[s], 1);
+      tmp = std::max(tmp, exchange_f64_tmp_elems(O, (int)N, (int)G));
+      nb = std::max(nb, exchange_f64_b_elems(O, (int)N, (int)W));
+    }
+    if (tmp > 0) {
+      A_(j->xq_b[0], nb);
+      A_(j->xq_kg, G);
+      A_(j->xq_tmp, tmp);
+    }
+  }
+  if (omax > kExchangeF64MaxO) {
     j->xwide_elems = exchange_wide_ws_elems(omax, (int)G, (int)W);
     A_(j->xwide, j->xwide_elems);
   }
@@ -1007,7 +1062,8 @@ int64_t afq_job_footprint(const afq_job_desc* d, int32_t n_prop_steps) {
   init_job(&j, d);
   int64_t total = 0;
   alloc_job(&j, true, &total);
-  if (n_prop_steps > 0) total += (int64_t)sizeof(double) * n_prop_steps * j.W * j.G;
+  if (n_prop_steps > 0)
+    total += (int64_t)sizeof(double) * n_prop_steps * j.W * j.G;
   return total;
 }
 
@@ -1033,6 +1089,7 @@ int afq_job_create(afq_job_t* out, const afq_job_desc* d) {
       return fail(AFQ_E_HIP, std::string("hipMemset: ") + hipGetErrorString(e));
     }
   }
+  if (!j->xq_b[1]) j->xq_b[1] = j->xq_b[0];
   if (j->rhf) {
     j->mo[1] = j->mo[0];
     j->rot_h1[1] = j->rot_h1[0];
@@ -1041,6 +1098,12 @@ int afq_job_create(afq_job_t* out, const afq_job_desc* d) {
     j->rcs[1] = j->rcs[0];
     j->rcs_fb[1] = j->rcs_fb[0];
     j->rct32[1] = j->rct32[0];
+    j->xq_q[1] = j->xq_q[0];
+    j->xq_p[1] = j->xq_p[0];
+    j->xq_a[1] = j->xq_a[0];
+    j->xq_c0[1] = j->xq_c0[0];
+    j->xq_mt[1] = j->xq_mt[0];
+    j->xq_k0[1] = j->xq_k0[0];
   } else if (j->rcs_fb[0]) {
     j->rcs_fb[1] = j->rcs_fb[0] + 2 * fb_kspin(j, 0);
   }
@@ -1111,6 +1174,11 @@ int afq_job_set_trial(afq_job_t j, const double* mo_up, const double* mo_dn, con
   if (!j->rhf)
     AFQ_HIP(hipMemcpyAsync(j->mo[1], mo_dn, sizeof(double) * N * j->nocc[1], hipMemcpyDefault, S(stream)));
   AFQ_HIP(hipMemcpyAsync(j->rdm1, rdm1, sizeof(double) * 2 * N * N, hipMemcpyDefault, S(stream)));
+  for (int s = 0; s < (j->rhf ? 1 : 2); ++s)
+    if (x_f64(j, s)) {
+      AFQ_TRY(x_f64_trial(j, s, S(stream)));
+      if (j->rc_set[s]) AFQ_TRY(x_f64_chol(j, s, S(stream)));
+    }
   j->have_trial = true;
   j->have_meas = j->have_prop = false;
   return AFQ_OK;
@@ -1161,6 +1229,8 @@ int afq_build_measurement_intermediates(afq_job_t j, void* stream) {
     r.ldc = N;
     r.sC = (long)O * N;
     AFQ_TRY(gemm_f64(r, st));
+    j->rc_set[s] = true;
+    if (x_f64(j, s)) AFQ_TRY(x_f64_chol(j, s, st));
   }
   if (j->lp)
     for (int s = 0; s < nsp; ++s) {
@@ -1288,6 +1358,8 @@ int afq_set_intermediate(afq_job_t j, int which, int spin, const void* src, void
     case AFQ_INT_ROT_H1: j->have_rot_h1[spin] = true; break;
     case AFQ_INT_ROT_CHOL:
       j->have_rot_chol[spin] = true;
+      j->rc_set[spin] = true;
+      if (x_f64(j, spin) && j->have_trial) AFQ_TRY(x_f64_chol(j, spin, S(stream)));
       if (j->lp) AFQ_TRY(k_to_f32(j->rot_chol[spin], j->rot_chol32[spin], G * O * N, S(stream)));
       if (j->rct32[spin])
         AFQ_TRY(k_split_f32(j->rot_chol[spin], false, (int)O, (int)N, G, j->rct32[spin], S(stream)));

@@ -9,18 +9,14 @@
 // are reduced in FP64 in every mode.
 //
 // Arithmetic of f:
-//   FP64   : v_mfma_f64_16x16x4f64 (exchange_kernel, exchange_split_kernel)
 //   FP32   : v_mfma_f32_16x16x4f32 on pre-converted FP32 planes
 //            (exchange_f32_kernel)
 //   BF16X3 : v_mfma_f32_16x16x32_bf16 on pre-split hi/lo bf16 planes,
 //            hi*hi + hi*lo + lo*hi (exchange_bf16_kernel)
 //
-// In the FP64 kernels fragments go straight from global memory to registers
-// in MFMA layout.  The K dimension (orbital index p) is permuted within each
-// chunk so that every lane reads consecutive elements of one row: lane l of
-// slab s reads p = c + KS*(l/16) + s (KS slabs per chunk), and the next chunk
-// is loaded while the current one is multiplied.  The FP32 and bf16 kernels
-// take 8 consecutive k per lane from planes laid out for it.
+// Both take 8 consecutive k per lane from planes laid out for it.  The FP64
+// exchange is exchange_f64.hip's up to nocc = 128; above, the f blocks are
+// stored (k_exchange_wide).
 //
 // Work-group order is XCD-aware: work-groups are handed to the eight XCDs
 // round-robin, so the logical index L = xcd * (T/8) + (bid/8) gives each XCD a
@@ -77,345 +73,6 @@ __device__ inline double wave_sum(double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
   return v;
-}
-
-// FP64 fragment of one chunk: NB row blocks of A (rot_chol rows) and of B
-// (Green's function rows), KS elements per lane.
-template <int NB, int KS>
-struct Frag {
-  double a[NB][KS];
-  double br[NB][KS];
-  double bi[NB][KS];
-};
-
-// One chunk as loaded: raw values at clamped (always valid) addresses, rows
-// >= O and columns >= N included.  take() converts it to the MFMA type and
-// zeroes A (rot_chol) there; that alone makes every padded product vanish:
-// f_ij = 0 for i >= O, so f_ij f_ji and f_ii vanish whenever i or j >= O, and
-// the clamped B values stay finite.  No loaded value is consumed before the
-// MFMAs of the current chunk are issued, so the next chunk's loads overlap them
-// (masking or converting at load time made the compiler wait for every load
-// first).
-template <int NB, int KS>
-struct Raw {
-  double a[NB][KS];
-  double2 b[NB][KS];
-};
-
-template <int NB, int KS>
-__device__ inline void load_raw(Raw<NB, KS>& X, const double* __restrict__ A, const double2* __restrict__ B, int O,
-                                int N, int c, int lane) {
-  const int kb = c + KS * (lane >> 4);
-  const int r16 = lane & 15;
-#pragma unroll
-  for (int bi = 0; bi < NB; ++bi) {
-    const long roff = (long)min(bi * 16 + r16, O - 1) * N;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const int col = min(kb + s, N - 1);
-      X.a[bi][s] = A[roff + col];
-      X.b[bi][s] = B[roff + col];
-    }
-  }
-}
-
-template <int NB, int KS>
-__device__ inline void take(Frag<NB, KS>& F, const Raw<NB, KS>& X, int O, int N, int c, int lane) {
-  const int kb = c + KS * (lane >> 4);
-#pragma unroll
-  for (int bi = 0; bi < NB; ++bi) {
-    const bool rok = bi * 16 + (lane & 15) < O;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      F.a[bi][s] = (rok && kb + s < N) ? X.a[bi][s] : 0.0;
-      F.br[bi][s] = X.b[bi][s].x;
-      F.bi[bi][s] = X.b[bi][s].y;
-    }
-  }
-}
-
-// NB <= 3 fits two work-groups per CU (<= 256 VGPRs per lane); NB = 4 would
-// need the whole register file (exchange_split_kernel serves 48 < O <= 64).
-template <int NB, int KS>
-__global__ __launch_bounds__(256, 2) void exchange_kernel(const double* __restrict__ rc, const double2* __restrict__ Gm, int O,
-                                                       int N, int Gn, int W, int nchunk, int cpg, long T8,
-                                                       double2* __restrict__ coul, double2* __restrict__ kpart) {
-  static_assert(NB <= 3, "48 < O <= 64 runs in exchange_split_kernel");
-  using Acc = v4d;
-  __shared__ double2 scr[4][16 * 17];
-  __shared__ double2 kred[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-
-  // XCD-aware logical index -> (gamma group, walker, chunk in group)
-  const long bid = blockIdx.x;
-  const long L = (bid & 7) * T8 + (bid >> 3);
-  const long per_group = (long)W * cpg;
-  const long grp = L / per_group;
-  const long rem = L - grp * per_group;
-  const int w = (int)(rem / cpg);
-  const int chunk = (int)(grp * cpg + rem % cpg);
-  if (chunk >= nchunk) return;  // uniform for the whole work-group
-  const int g = chunk * 4 + wave;
-  const bool valid = g < Gn;
-  const int gg = valid ? g : Gn - 1;
-
-  const double* A = rc + (long)gg * O * N;
-  const double2* B = Gm + (long)w * O * N;
-
-  Acc accR[NB][NB], accI[NB][NB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i)
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      accR[i][j] = Acc{0, 0, 0, 0};
-      accI[i][j] = Acc{0, 0, 0, 0};
-    }
-
-  constexpr int CW = 4 * KS;
-  Frag<NB, KS> cur;
-  Raw<NB, KS> nxt;
-  load_raw<NB, KS>(nxt, A, B, O, N, 0, lane);
-  take<NB, KS>(cur, nxt, O, N, 0, lane);
-  for (int c = 0; c < N; c += CW) {
-    if (c + CW < N) load_raw<NB, KS>(nxt, A, B, O, N, c + CW, lane);
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int bi = 0; bi < NB; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < NB; ++bj) {
-          accR[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(cur.a[bi][s], cur.br[bj][s], accR[bi][bj], 0, 0, 0);
-          accI[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(cur.a[bi][s], cur.bi[bj][s], accI[bi][bj], 0, 0, 0);
-        }
-    if (c + CW < N) take<NB, KS>(cur, nxt, O, N, c + CW, lane);
-  }
-
-  // element v of lane l sits at (row, col) = (l/16 + 4v, l%16)
-  const int cc = lane & 15;
-  double kr = 0.0, ki = 0.0, cr = 0.0, ci = 0.0;
-  double2* S = scr[wave];
-#pragma unroll
-  for (int bi = 0; bi < NB; ++bi)
-#pragma unroll
-    for (int bj = bi; bj < NB; ++bj) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = (lane >> 4) + 4 * v;
-        S[r * 17 + cc] = double2{(double)accR[bj][bi][v], (double)accI[bj][bi][v]};
-      }
-      wave_lds_sync();
-      const double wgt = (bi == bj) ? 1.0 : 2.0;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = (lane >> 4) + 4 * v;
-        const int gi = bi * 16 + r, gj = bj * 16 + cc;
-        if (gi < O && gj < O) {
-          const double xr = accR[bi][bj][v], xi = accI[bi][bj][v];
-          const double2 y = S[cc * 17 + r];
-          kr += wgt * (xr * y.x - xi * y.y);
-          ki += wgt * (xr * y.y + xi * y.x);
-          if (bi == bj && r == cc) {
-            cr += xr;
-            ci += xi;
-          }
-        }
-      }
-      wave_lds_sync();
-    }
-  kr = wave_sum(kr);
-  ki = wave_sum(ki);
-  cr = wave_sum(cr);
-  ci = wave_sum(ci);
-  if (lane == 0) {
-    if (valid) coul[(long)w * Gn + g] = double2{cr, ci};
-    kred[wave] = valid ? double2{kr, ki} : double2{0.0, 0.0};
-  }
-  __syncthreads();
-  if (tid == 0) {
-    double2 s = {0.0, 0.0};
-    for (int i = 0; i < 4; ++i) {
-      s.x += kred[i].x;
-      s.y += kred[i].y;
-    }
-    kpart[(long)w * nchunk + chunk] = s;
-  }
-}
-
-// FP64 exchange for 48 < O <= 64: a 64 x 64 complex f-block takes 256
-// accumulator registers, which leaves one wave per SIMD.  Here two waves share
-// one (walker, gamma): wave half h holds the block rows 2h, 2h + 1 (2 x 4 blocks,
-// 128 registers), so two waves fit per SIMD.  The eight waves of a work-group
-// take four consecutive gamma of one walker, as in exchange_kernel.  For
-// sum_ij f_ij f_ji, a block whose transposed partner lies in the other half is
-// exchanged through LDS (each wave publishes its four cross blocks), and the
-// pairs inside a half are matched through a per-wave LDS tile afterwards.
-template <int KS>
-__global__ __launch_bounds__(512, 1) void exchange_split_kernel(const double* __restrict__ rc,
-                                                                const double2* __restrict__ Gm, int O, int N, int Gn,
-                                                                int W, int nchunk, int cpg, long T8,
-                                                                double2* __restrict__ coul, double2* __restrict__ kpart) {
-  constexpr int TS = 16 * 17;  // one padded 16 x 16 tile
-  extern __shared__ double2 xsh[];  // [8 waves][4 tiles][TS]
-  __shared__ double2 kred[8], cred[8];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int gi = wave >> 1, h = wave & 1;
-  const long bid = blockIdx.x;
-  const long L = (bid & 7) * T8 + (bid >> 3);
-  const long per_group = (long)W * cpg;
-  const long grp = L / per_group;
-  const long rem = L - grp * per_group;
-  const int w = (int)(rem / cpg);
-  const int chunk = (int)(grp * cpg + rem % cpg);
-  if (chunk >= nchunk) return;  // uniform for the whole work-group
-  const int g = chunk * 4 + gi;
-  const bool valid = g < Gn;
-  const int gg = valid ? g : Gn - 1;
-  const double* A = rc + (long)gg * O * N;
-  const double2* B = Gm + (long)w * O * N;
-  const int r16 = lane & 15, q4 = lane >> 4;
-
-  long ra[2], rb[4];
-  bool oka[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int row = 16 * (2 * h + i) + r16;
-    oka[i] = row < O;
-    ra[i] = (long)min(row, O - 1) * N;
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    rb[j] = (long)min(16 * j + r16, O - 1) * N;
-  }
-  v4d accR[2][4], accI[2][4];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) accR[i][j] = accI[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
-
-  struct Fr {
-    double a[2][KS], br[4][KS], bi[4][KS];
-  };
-  // raw values at clamped addresses; mask() zeroes A at rows >= O and
-  // columns >= N once the chunk is about to be used, which makes every padded
-  // product vanish (f_ij = 0 for i >= O) while the clamped B values stay finite
-  auto load = [&](Fr& F, int c) {
-    const int kb = c + KS * q4;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const int pc = min(kb + s, N - 1);
-#pragma unroll
-      for (int i = 0; i < 2; ++i) F.a[i][s] = A[ra[i] + pc];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const double2 bv = B[rb[j] + pc];
-        F.br[j][s] = bv.x;
-        F.bi[j][s] = bv.y;
-      }
-    }
-  };
-  auto mask = [&](Fr& F, int c) {
-    const int kb = c + KS * q4;
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) F.a[i][s] = (oka[i] && kb + s < N) ? F.a[i][s] : 0.0;
-  };
-  constexpr int CW = 4 * KS;
-  Fr cur, nxt;
-  load(cur, 0);
-  mask(cur, 0);
-  for (int c = 0; c < N; c += CW) {
-    if (c + CW < N) load(nxt, c + CW);
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(cur.a[i][s], cur.br[j][s], accR[i][j], 0, 0, 0);
-          accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(cur.a[i][s], cur.bi[j][s], accI[i][j], 0, 0, 0);
-        }
-    if (c + CW < N) {
-      cur = nxt;
-      mask(cur, c + CW);
-    }
-  }
-
-  // element v of lane l is (row, col) = (l/16 + 4v, l%16) of its 16 x 16 block
-  const int cc = lane & 15;
-  double kr = 0.0, ki = 0.0, cr = 0.0, ci = 0.0;
-  double2* mine = xsh + (long)wave * 4 * TS;
-  const double2* other = xsh + (long)(wave ^ 1) * 4 * TS;
-  const int ho = 1 - h;
-  // cross blocks (2h + i, 2ho + jj): publish, then pair with the partner's (2ho + jj, 2h + i)
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        mine[(i * 2 + jj) * TS + (q4 + 4 * v) * 17 + cc] =
-            double2{accR[i][2 * ho + jj][v], accI[i][2 * ho + jj][v]};
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = q4 + 4 * v;
-        const double xr = accR[i][2 * ho + jj][v], xi = accI[i][2 * ho + jj][v];
-        const double2 y = other[(jj * 2 + i) * TS + cc * 17 + r];
-        kr += xr * y.x - xi * y.y;
-        ki += xr * y.y + xi * y.x;
-      }
-  __syncthreads();
-  // pairs inside the half: blocks (2h + i, 2h + j), i <= j, through the first tile
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = i; j < 2; ++j) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        mine[(q4 + 4 * v) * 17 + cc] = double2{accR[j][2 * h + i][v], accI[j][2 * h + i][v]};
-      __syncthreads();
-      const double wgt = (i == j) ? 1.0 : 2.0;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = q4 + 4 * v;
-        const double xr = accR[i][2 * h + j][v], xi = accI[i][2 * h + j][v];
-        const double2 y = mine[cc * 17 + r];
-        kr += wgt * (xr * y.x - xi * y.y);
-        ki += wgt * (xr * y.y + xi * y.x);
-        if (i == j && r == cc) {
-          cr += xr;
-          ci += xi;
-        }
-      }
-      __syncthreads();
-    }
-  kr = wave_sum(kr);
-  ki = wave_sum(ki);
-  cr = wave_sum(cr);
-  ci = wave_sum(ci);
-  if (lane == 0) {
-    kred[wave] = valid ? double2{kr, ki} : double2{0.0, 0.0};
-    cred[wave] = double2{cr, ci};
-  }
-  __syncthreads();
-  if (tid < 4) {
-    const int gq = chunk * 4 + tid;
-    if (gq < Gn)
-      coul[(long)w * Gn + gq] = double2{cred[2 * tid].x + cred[2 * tid + 1].x, cred[2 * tid].y + cred[2 * tid + 1].y};
-  }
-  if (tid == 0) {
-    double2 sum = {0.0, 0.0};
-    for (int q = 0; q < 8; ++q) {
-      sum.x += kred[q].x;
-      sum.y += kred[q].y;
-    }
-    kpart[(long)w * nchunk + chunk] = sum;
-  }
 }
 
 // Exchange epilogue of one wave: c_g = tr f_g and K_g = sum_ab f_ab f_ba from
@@ -931,69 +588,9 @@ __global__ __launch_bounds__(256) void exchange_wide_reduce_kernel(const double2
   if (tid == 0) kpart[(long)w * nchunk + g0 / 4 + c] = double2{ksr, ksi};
 }
 
-template <int NB, int KS>
-int launch_nb(const double* rc, const double2* Gm, int O, int N, int Gn, int W, int nchunk, double2* coul,
-              double2* kpart, hipStream_t s) {
-  // gamma chunks per group: a group's rot_chol slice ~2.5 MB of L2
-  const long chunk_bytes = 4L * O * N * (long)sizeof(double);
-  const int cpg = (int)std::max(1L, std::min((long)nchunk, (kGroupSliceBytes) / std::max(1L, chunk_bytes)));
-  const long ngroups = (nchunk + cpg - 1) / cpg;
-  const long T = ngroups * cpg * (long)W;
-  const long T8 = (T + 7) / 8;
-  const long grid = T8 * 8;
-  if (grid > 0x7fffffffL) return fail(AFQ_E_UNSUPPORTED, "exchange grid too large");
-  hipLaunchKernelGGL((exchange_kernel<NB, KS>), dim3((unsigned)grid), dim3(256), 0, s, rc, Gm, O, N, Gn, W, nchunk,
-                     cpg, T8, coul, kpart);
-  return launch_status("exchange_kernel");
-}
-
-template <int KS>
-int launch_split(const double* rc, const double2* Gm, int O, int N, int Gn, int W, int nchunk, double2* coul,
-                 double2* kpart, hipStream_t s) {
-  const long chunk_bytes = 4L * O * N * (long)sizeof(double);
-  const int cpg = (int)std::max(1L, std::min((long)nchunk, (kGroupSliceBytes) / std::max(1L, chunk_bytes)));
-  const long ngroups = (nchunk + cpg - 1) / cpg;
-  const long T = ngroups * cpg * (long)W;
-  const long T8 = (T + 7) / 8;
-  const long grid = T8 * 8;
-  if (grid > 0x7fffffffL) return fail(AFQ_E_UNSUPPORTED, "exchange grid too large");
-  const size_t lds = sizeof(double2) * 8 * 4 * 16 * 17;
-  static bool raised = false;
-  if (!raised) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(exchange_split_kernel<KS>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return fail(AFQ_E_HIP, std::string("exchange LDS attribute: ") + hipGetErrorString(e));
-    raised = true;
-  }
-  hipLaunchKernelGGL((exchange_split_kernel<KS>), dim3((unsigned)grid), dim3(512), lds, s, rc, Gm, O, N, Gn, W,
-                     nchunk, cpg, T8, coul, kpart);
-  return launch_status("exchange_split_kernel");
-}
-
-// O <= 48; chunk widths chosen so the fragments fit next to the accumulators
-// (NB = 3: 8-wide chunks, two work-groups per CU)
-int launch_f64(const double* rc, const double2* Gm, int O, int N, int Gn, int W, int nchunk, double2* coul,
-               double2* kpart, hipStream_t s) {
-  switch ((O + 15) / 16) {
-    case 1: return launch_nb<1, 4>(rc, Gm, O, N, Gn, W, nchunk, coul, kpart, s);
-    case 2: return launch_nb<2, 4>(rc, Gm, O, N, Gn, W, nchunk, coul, kpart, s);
-    default: return launch_nb<3, 2>(rc, Gm, O, N, Gn, W, nchunk, coul, kpart, s);
-  }
-}
-
 }  // namespace
 
 int exchange_nchunk(int Gn) { return (Gn + 3) / 4; }
-
-int k_exchange(const double* rc, const double2* Gm, int O, int N, int Gn, int W, double2* coul, double2* kpart,
-               int* nchunk_out, hipStream_t s) {
-  if (O < 1 || O > 64) return fail(AFQ_E_UNSUPPORTED, "exchange kernel supports 1 <= nocc <= 64");
-  const int nchunk = exchange_nchunk(Gn);
-  *nchunk_out = nchunk;
-  // 48 < O <= 64: two waves per f-block (the 64 x 64 block alone would take 256 registers)
-  if (O > 48) return launch_split<2>(rc, Gm, O, N, Gn, W, nchunk, coul, kpart, s);
-  return launch_f64(rc, Gm, O, N, Gn, W, nchunk, coul, kpart, s);
-}
 
 long exchange_wide_ws_elems(int O, int Gn, int W) {
   // a pass of gc g's (a multiple of 4, at least one chunk) within 256 MB

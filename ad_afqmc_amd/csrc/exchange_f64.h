@@ -1,0 +1,47 @@
+// FP64 exchange over the unoccupied orbitals of the trial (exchange_f64.hip).
+#pragma once
+#include "afq_internal.h"
+
+namespace afq {
+
+constexpr int kExchangeF64MaxO = 128;
+
+// Work-group tile: WR x WC waves of MB x NB MFMA blocks hold gw g's of wn walkers.
+struct ExF64Tile {
+  int MB, NB, WR, WC, gw, wn;
+};
+ExF64Tile exchange_f64_tile(int O);
+int exchange_f64_nchunk(int O, int G);
+
+struct ExF64 {
+  const double* a;        // packed rot_chol Q
+  const double2* theta;   // packed slabs of B (pack_b_kernel)
+  const double* c0;       // (G,) tr f0_g
+  int O, Nv, n8, G, W, gw, wn, nwg, nchunk, cpg, gp, strip;
+  long T8, lds_elems;
+  double2* coul;          // (W, G)
+  double2* kpart;         // (W, nchunk + 1)
+};
+
+// Sizes of the packed rot_chol Q (doubles), of the packed theta (complex) and
+// of the setup workspace (doubles).
+long exchange_f64_a_elems(int O, int N, int G);
+long exchange_f64_b_elems(int O, int N, int W);
+long exchange_f64_tmp_elems(int O, int N, int G);
+// Q (N, N - O): orthonormal complement of span(mo); P (N, O) = mo (mo^T mo)^-1.
+int exchange_f64_set_trial(const double* mo, int N, int O, double* Q, double* P, double* tmp, double* ws,
+                           long ws_elems, hipStream_t st);
+// From rot_chol (G, O, N): a, c0 (G,), mt (O, N - O), k0 (1,); kg (G,) scratch.
+int exchange_f64_set_chol(const double* rc, const double* Q, const double* P, int N, int O, int G, double* a,
+                          double* c0, double* mt, double* k0, double* kg, double* tmp, double* ws, long ws_elems,
+                          hipStream_t st);
+// Rows (k pairs) of the packed theta of one walker group.
+int exchange_f64_npairs(int Nv);
+// green null: the caller has filled thetap and the last partial K already.
+// c_g (W, G) and the *nch_out partial K's of every walker; theta (W, O, N - O) and
+// thetap (exchange_f64_b_elems) are scratch.
+int k_exchange_f64(const double* a, const double* Q, const double* c0, const double* mt, const double* k0,
+                   const double2* green, double2* theta, double2* thetap, int O, int N, int G, int W, double2* coul,
+                   double2* kpart, int* nch_out, hipStream_t st);
+
+}  // namespace afq

@@ -17,9 +17,7 @@ int k_overlap_combine(const double2* d0, const double2* d1, double2* out, int W,
 int k_ene1(const double2* G0, const double* rh0, int n0, const double2* G1, const double* rh1, int n1, int N, double f0,
            double2* out, int W, hipStream_t s);
 int exchange_nchunk(int Gn);
-int k_exchange(const double* rc, const double2* Gm, int O, int N, int Gn, int W, double2* coul, double2* kpart,
-               int* nchunk_out, hipStream_t s);
-// nocc > 64 (any precision, FP64 arithmetic): f_g of a pass of g's for all
+// nocc > 128 (any precision, FP64 arithmetic): f_g of a pass of g's for all
 // walkers by the batched FP64 product into ws, then c_g and the K_g of each
 // 4-g chunk; ws holds exchange_wide_ws_elems(O, Gn, W) complex elements.
 long exchange_wide_ws_elems(int O, int Gn, int W);
