@@ -9,6 +9,7 @@
 #include "gemm_bf3.h"
 #include "group.h"
 #include "kernels.h"
+#include "small.h"
 #include "trot_fused.h"
 #include "pipeline.h"
 
@@ -96,6 +97,9 @@ void release(afq_job* j) {
   }
   fr(j->xq_b[0]);
   if (j->xq_b[1] != j->xq_b[0]) fr(j->xq_b[1]);
+  fr(j->h_step);
+  fr(j->small_l);
+  fr(j->small_rc);
   fr(j->xq_kg);
   fr(j->xq_tmp);
   fr(j->xwide);
@@ -139,12 +143,18 @@ int check_walkers(const afq_job* j, const void* up, const void* dn) {
   return AFQ_OK;
 }
 
+bool small_meas(const afq_job* j);
+int measure_small(afq_job* j, const void* up, const void* dn, bool qr, bool inverse, double2* energies,
+                  double2* overlaps, hipStream_t st);
+
 // S_s = T_s^H W_s ; det_s ; optionally S_s^-1 and G_s = (W_s S_s^-1)^T.  With
 // have_inv the caller guarantees that S_s^-1 and det_s already belong to these
 // walkers (computed by the previous call on them), and only G_s is formed.
 int green_pipeline(afq_job* j, const void* up, const void* dn, bool want_inv, bool want_green, hipStream_t st,
                    bool have_inv) {
   const int N = j->N, W = j->W;
+  if (!have_inv && want_inv && want_green && small_meas(j))
+    return measure_small(j, up, dn, false, true, nullptr, nullptr, st);
   if (!have_inv) {
     DetInvSet sets[2];
     Gemm gs[2];
@@ -326,10 +336,124 @@ int x_f64_chol(afq_job* j, int s, hipStream_t st) {
                                j->gemm_ws_elems, st);
 }
 
-int energy_pipeline(afq_job* j, const void* up, const void* dn, double2* out, hipStream_t st, bool have_green) {
-  if (!have_green) AFQ_TRY(green_pipeline(j, up, dn, true, true, st));
-  const bool two = !j->one_spin;
+// FP64 jobs whose walkers fit one work-group each (small.hip): for the
+// measurement, and for the step (small_steps: with buffers for it; small_step:
+// and better off so with the walkers and L at hand).
+int small_osum(const afq_job* j) { return j->nocc[0] + (j->nspin_meas > 1 ? j->nocc[1] : 0); }
+int small_cols(const afq_job* j) { return j->restricted ? j->wcols : j->nocc[0] + j->nocc[1]; }
+bool small_occ(const afq_job* j) {
+  return !j->lp && std::max(j->nocc[0], j->nocc[1]) <= kSmallMaxO && j->wcols <= kSmallMaxO;
+}
+bool small_meas(const afq_job* j) { return small_occ(j) && small_measure_lds(j->N, small_cols(j), small_osum(j)) > 0; }
+bool small_whole(const afq_job* j) {
+  return small_energy_whole(j->N, j->G, j->nocc[0], j->nspin_meas > 1 ? j->nocc[1] : 0);
+}
+bool small_steps(const afq_job* j) {
+  return small_occ(j) && small_step_lds(j->N, j->G, small_cols(j), small_osum(j), j->nspin_prop) > 0;
+}
+bool small_step(const afq_job* j) {
+  return small_steps(j) && small_step_pays(j->N, j->G, small_osum(j), j->W, j->sym_chol);
+}
+
+int small_pack_rc(afq_job* j, hipStream_t st) {
+  if (!j->small_rc) return AFQ_OK;
+  return k_small_pack_rc(j->rot_chol[0], j->N * j->nocc[0], j->rot_chol[1], j->nspin_meas > 1 ? j->N * j->nocc[1] : 0,
+                         j->G, j->small_rc, st);
+}
+
+SmallJob small_args(afq_job* j, const void* up, const void* dn) {
+  SmallJob b{};
+  b.N = j->N;
+  b.G = j->G;
+  b.W = j->W;
+  b.nspin = j->nspin_meas;
+  b.nbuf = j->nspin_prop;
+  for (int s = 0; s < 2; ++s) {
+    b.occ[s] = j->nocc[s];
+    b.off[s] = j->restricted || s == 0 ? 0 : j->nocc[0];
+    b.cb[s] = j->restricted ? j->wcols : j->nocc[s];
+    b.wbuf[s] = static_cast<double2*>(const_cast<void*>(s == 0 ? up : dn));
+    b.mo[s] = j->mo[s];
+    b.Sinv[s] = j->Sinv[s];
+    b.det[s] = j->det[s];
+  }
+  b.c = b.cb[0] + (b.nbuf > 1 ? b.cb[1] : 0);
+  return b;
+}
+
+// nsteps phaseless steps of a small job; j->h_step holds nsteps rows.
+int propagate_small(afq_job* j, void* up, void* dn, const double* fields, int nsteps, double* weights,
+                    double2* overlaps, double* scalars, hipStream_t st) {
+  SmallStep p{};
+  p.b = small_args(j, up, dn);
+  for (int s = 0; s < 2; ++s) p.ex[s] = j->exp_h1[s];
+  p.lt = j->small_l;
+  p.rcp = j->small_rc;
+  p.sym = j->sym_chol;
+  p.nterms = j->d.n_exp_terms;
+  p.nsteps = nsteps;
+  p.fac = j->one_spin ? 2.0 : 1.0;
+  p.dt = j->d.dt;
+  p.mf = j->mf_shifts;
+  p.fields = fields;
+  p.h0p = j->h0_prop;
+  p.scalars = scalars;
+  p.h = j->h_step;
+  p.overlaps = overlaps;
+  p.fb = j->fb;
+  p.xs = j->xs;
+  p.terms = j->terms;
+  p.ov_new = j->ov_new;
   {
+    ProfScope ps(j, AFQ_K_TAYLOR, st);
+    AFQ_TRY(k_small_step(p, st));
+  }
+  ProfScope ps(j, AFQ_K_WEIGHT, st);
+  return k_small_weights(j->h_step, nsteps, j->W, j->d.dt, weights, scalars, st);
+}
+
+// With qr, re-orthonormalises the walkers; overlaps (may be null); with inverse
+// also S^-1 and the Green's functions, and with energies (of a small_whole job)
+// the energies, or else everything they need before the exchange.
+int measure_small(afq_job* j, const void* up, const void* dn, bool qr, bool inverse, double2* energies,
+                  double2* overlaps, hipStream_t st) {
+  SmallMeasure p{};
+  p.b = small_args(j, up, dn);
+  p.qr = qr;
+  p.inverse = inverse;
+  p.energy = energies != nullptr;
+  p.whole = small_whole(j);
+  p.h0 = j->h0;
+  p.energies = energies;
+  p.fac = j->one_spin ? 2.0 : 1.0;
+  p.overlaps = overlaps;
+  p.ene1 = j->ene1;
+  for (int s = 0; s < j->nspin_meas; ++s) {
+    const ExF64Tile t = exchange_f64_tile(j->nocc[s]);
+    p.green[s] = j->green[s];
+    p.rh1[s] = j->rot_h1[s];
+    p.rc[s] = j->rot_chol[s];
+    p.q[s] = j->xq_q[s];
+    p.mt[s] = j->xq_mt[s];
+    p.k0[s] = j->xq_k0[s];
+    p.thetap[s] = j->xq_b[s];
+    p.kpart[s] = j->kpart + (long)s * j->W * j->kchunk_max;
+    p.wn[s] = t.wn;
+    p.c2[s] = 8 * t.NB * t.WC;
+    p.npr[s] = exchange_f64_npairs(j->N - j->nocc[s]);
+    p.nchunk[s] = exchange_f64_nchunk(j->nocc[s], j->G);
+  }
+  ProfScope ps(j, inverse ? AFQ_K_GREEN : AFQ_K_OVLP_GEMM, st);
+  return k_small_measure(p, st);
+}
+
+int energy_pipeline(afq_job* j, const void* up, const void* dn, double2* out, hipStream_t st, bool have_green) {
+  const bool small = small_meas(j);
+  if (small && !have_green) AFQ_TRY(measure_small(j, up, dn, false, true, out, nullptr, st));
+  if (small && small_whole(j)) return AFQ_OK;  // the energies are in out already
+  if (!small && !have_green) AFQ_TRY(green_pipeline(j, up, dn, true, true, st));
+  const bool two = !j->one_spin;
+  if (!small) {
     ProfScope ps(j, AFQ_K_ENERGY_MISC, st);
     AFQ_TRY(k_ene1(j->green[0], j->rot_h1[0], j->nocc[0], two ? j->green[1] : nullptr, two ? j->rot_h1[1] : nullptr,
                    j->nocc[1], j->N, two ? 1.0 : 2.0, j->ene1, j->W, st));
@@ -360,7 +484,7 @@ int energy_pipeline(afq_job* j, const void* up, const void* dn, double2* out, hi
     ProfScope ps(j, AFQ_K_EXCHANGE, st);
     if (x_f64(j, s))  // theta in the SR gather buffer
       AFQ_TRY(k_exchange_f64(j->xq_a[s], j->xq_q[s], j->xq_c0[s], j->xq_mt[s], j->xq_k0[s],
-                             j->green[s], j->wgather,
+                             small ? nullptr : j->green[s], j->wgather,
                              j->xq_b[s], j->nocc[s], j->N, j->G, j->W, coul, kpart, &nch[s], st));
     else
       AFQ_TRY(k_exchange_wide(j->rot_chol[s], j->green[s], j->nocc[s], j->N, j->G, j->W, j->xwide, j->xwide_elems,
@@ -635,6 +759,7 @@ int trotprop(afq_job* j, void* up, void* dn, const double2* xs, hipStream_t st) 
 
 int propagate(afq_job* j, void* up, void* dn, const double* fields, double* weights, double2* overlaps,
               double* scalars, hipStream_t st, bool inv_ready, bool keep_inv) {
+  if (small_step(j)) return propagate_small(j, up, dn, fields, 1, weights, overlaps, scalars, st);
   AFQ_TRY(green_pipeline(j, up, dn, true, true, st, inv_ready));
   AFQ_TRY(force_bias_gemm(j, j->fb, st));
   {
@@ -966,6 +1091,7 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
     }
     if (tmp > 0) {
       A_(j->xq_b[0], nb);
+      if (small_meas(j) && j->nspin_meas > 1) A_(j->xq_b[1], nb);
       A_(j->xq_kg, G);
       A_(j->xq_tmp, tmp);
     }
@@ -1048,6 +1174,12 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
   j->gemm_ws_elems = 16 * std::max(2 * W * G, N * N);
   A_(j->gemm_ws, j->gemm_ws_elems);
   A_(j->dscratch, 8);
+  if (small_steps(j)) {
+    j->h_cap = W;
+    A_(j->h_step, j->h_cap);
+    A_(j->small_l, G * small_l_pairs((int)N, false));
+    A_(j->small_rc, G * small_rc_pairs((int)N, small_osum(j)));
+  }
 #undef A_
   return rc;
 }
@@ -1063,7 +1195,7 @@ int64_t afq_job_footprint(const afq_job_desc* d, int32_t n_prop_steps) {
   int64_t total = 0;
   alloc_job(&j, true, &total);
   if (n_prop_steps > 0)
-    total += (int64_t)sizeof(double) * n_prop_steps * j.W * j.G;
+    total += (int64_t)sizeof(double) * n_prop_steps * j.W * (j.G + (small_steps(&j) ? 1 : 0));
   return total;
 }
 
@@ -1161,6 +1293,7 @@ int afq_job_set_hamiltonian(afq_job_t j, double h0, const double* h1, const doub
   } else if (j->sym_chol) {
     AFQ_TRY(k_sym_pack(j->chol, j->G, (int)N, j->cholp, nullptr, S(stream)));
   }
+  if (j->small_l) AFQ_TRY(k_small_pack_l(j->chol, (int)N, j->G, j->sym_chol, j->small_l, S(stream)));
   j->have_ham = true;
   j->have_meas = j->have_prop = false;
   return AFQ_OK;
@@ -1232,6 +1365,7 @@ int afq_build_measurement_intermediates(afq_job_t j, void* stream) {
     j->rc_set[s] = true;
     if (x_f64(j, s)) AFQ_TRY(x_f64_chol(j, s, st));
   }
+  AFQ_TRY(small_pack_rc(j, st));
   if (j->lp)
     for (int s = 0; s < nsp; ++s) {
       AFQ_TRY(k_to_f32(j->rot_chol[s], j->rot_chol32[s], (long)j->G * j->nocc[s] * N, st));
@@ -1360,6 +1494,7 @@ int afq_set_intermediate(afq_job_t j, int which, int spin, const void* src, void
       j->have_rot_chol[spin] = true;
       j->rc_set[spin] = true;
       if (x_f64(j, spin) && j->have_trial) AFQ_TRY(x_f64_chol(j, spin, S(stream)));
+      AFQ_TRY(small_pack_rc(j, S(stream)));
       if (j->lp) AFQ_TRY(k_to_f32(j->rot_chol[spin], j->rot_chol32[spin], G * O * N, S(stream)));
       if (j->rct32[spin])
         AFQ_TRY(k_split_f32(j->rot_chol[spin], false, (int)O, (int)N, G, j->rct32[spin], S(stream)));
@@ -1391,6 +1526,7 @@ int afq_calc_overlap(afq_job_t j, const void* up, const void* dn, void* ov, void
   AFQ_TRY(require(j, false, false));
   AFQ_TRY(check_walkers(j, up, dn));
   if (!ov) return fail(AFQ_E_INVALID, "overlaps is NULL");
+  if (small_meas(j)) return measure_small(j, up, dn, false, false, nullptr, static_cast<double2*>(ov), S(stream));
   AFQ_TRY(green_pipeline(j, up, dn, false, false, S(stream)));
   return overlap_from_dets(j, static_cast<double2*>(ov), S(stream));
 }
@@ -1482,14 +1618,25 @@ int afq_sr_zeta(double* out, uint64_t seed, uint64_t counter, void* stream) {
 
 namespace afq {
 
+// Room for `need` fields, and the phaseless factors of as many steps.
 int reserve_fields(afq_job* j, long need, hipStream_t st) {
-  if (need <= j->fields_cap) return AFQ_OK;
+  const long hneed = j->h_step ? (need + j->G - 1) / j->G : 0;
+  if (need <= j->fields_cap && hneed <= j->h_cap) return AFQ_OK;
   AFQ_HIP(hipStreamSynchronize(st));
-  if (j->fields) (void)hipFree(j->fields);
-  j->fields = nullptr;
-  j->fields_cap = 0;
-  AFQ_TRY(dalloc_n(&j->fields, (size_t)need));
-  j->fields_cap = need;
+  if (need > j->fields_cap) {
+    if (j->fields) (void)hipFree(j->fields);
+    j->fields = nullptr;
+    j->fields_cap = 0;
+    AFQ_TRY(dalloc_n(&j->fields, (size_t)need));
+    j->fields_cap = need;
+  }
+  if (hneed > j->h_cap) {
+    double* h = nullptr;
+    AFQ_TRY(dalloc_n(&h, (size_t)hneed));
+    (void)hipFree(j->h_step);
+    j->h_step = h;
+    j->h_cap = hneed;
+  }
   return AFQ_OK;
 }
 
@@ -1502,11 +1649,19 @@ int reserve_fields(afq_job* j, long need, hipStream_t st) {
 int block_body(afq_job* j, void* up, void* dn, double* weights, double2* ov, double* scalars, int n_prop_steps,
                double* block_out, hipStream_t st) {
   const long per_step = (long)j->W * j->G;
-  for (int i = 0; i < n_prop_steps; ++i)
-    AFQ_TRY(propagate(j, up, dn, j->fields + i * per_step, weights, ov, scalars, st, i > 0, i + 1 < n_prop_steps));
-  AFQ_TRY(orthonormalize(j, up, dn, st));
-  AFQ_TRY(green_pipeline(j, up, dn, true, true, st));
-  AFQ_TRY(overlap_from_dets(j, ov, st));
+  if (small_step(j)) {
+    AFQ_TRY(propagate_small(j, up, dn, j->fields, n_prop_steps, weights, ov, scalars, st));
+  } else {
+    for (int i = 0; i < n_prop_steps; ++i)
+      AFQ_TRY(propagate(j, up, dn, j->fields + i * per_step, weights, ov, scalars, st, i > 0, i + 1 < n_prop_steps));
+  }
+  if (small_meas(j)) {
+    AFQ_TRY(measure_small(j, up, dn, true, true, j->energies, ov, st));
+  } else {
+    AFQ_TRY(orthonormalize(j, up, dn, st));
+    AFQ_TRY(green_pipeline(j, up, dn, true, true, st));
+    AFQ_TRY(overlap_from_dets(j, ov, st));
+  }
   AFQ_TRY(energy_pipeline(j, up, dn, j->energies, st, true));
   ProfScope ps(j, AFQ_K_ENERGY_MISC, st);
   return k_block_finalize(j->energies, weights, scalars, std::sqrt(2.0 / j->d.dt), j->W, block_out, st);
@@ -1525,6 +1680,7 @@ int sr_and_overlap(afq_job* j, void* up, void* dn, double* weights, const double
       AFQ_HIP(hipMemcpyAsync(Wp, j->wgather, sizeof(double2) * per * j->W, hipMemcpyDeviceToDevice, st));
     }
   }
+  if (small_meas(j)) return measure_small(j, up, dn, false, false, nullptr, ov, st);
   AFQ_TRY(green_pipeline(j, up, dn, false, false, st));
   return overlap_from_dets(j, ov, st);
 }

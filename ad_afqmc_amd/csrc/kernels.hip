@@ -2,33 +2,15 @@
 // exchange-energy kernel.  Launch helpers are declared in kernels.h.
 #include "kernels.h"
 #include "group.h"
+#include "wave_math.h"
 
 namespace afq {
 namespace {
 
-__device__ inline double2 cmul(double2 a, double2 b) { return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
-__device__ inline double2 cadd(double2 a, double2 b) { return {a.x + b.x, a.y + b.y}; }
-__device__ inline double2 cdiv(double2 a, double2 b) {
-  // Smith's algorithm
-  if (fabs(b.x) >= fabs(b.y)) {
-    const double r = b.y / b.x, den = b.x + b.y * r;
-    return {(a.x + a.y * r) / den, (a.y - a.x * r) / den};
-  }
-  const double r = b.x / b.y, den = b.x * r + b.y;
-  return {(a.x * r + a.y) / den, (a.y * r - a.x) / den};
-}
-__device__ inline double2 cexp(double2 z) {
-  const double e = exp(z.x);
-  double s, c;
-  sincos(z.y, &s, &c);
-  return {e * c, e * s};
-}
+using wm::cadd;
+using wm::cmul;
+using wm::wave_sum;
 
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
-}
 // Block (256-thread) sum of a complex value; every thread gets the result.
 __device__ inline double2 block_sum2(double2 v, double2* red) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -221,24 +203,13 @@ __device__ __forceinline__ void weight_update_body(const double2* ov_new, double
                                                    double* weights, double* scalars, const double2* h0_prop, double dt,
                                                    int W) {
   __shared__ double red[16];
-  const double sqdt = sqrt(dt);
   const double pcs = scalars[1];
   const double2 h0p = *h0_prop;
   double local = 0.0;
   for (int w = threadIdx.x; w < W; w += blockDim.x) {
     const double2 on = ov_new[w], oo = overlaps[w];
-    const double2 ratio = cdiv(on, oo);
-    const double2 sh = terms[2 * w], ft = terms[2 * w + 1];
-    const double2 arg = {-sqdt * sh.x + ft.x + dt * (pcs + h0p.x), -sqdt * sh.y + ft.y + dt * h0p.y};
-    const double2 imp = cmul(cexp(arg), ratio);
-    const double2 ph_arg = cmul(cexp(double2{-sqdt * sh.x, -sqdt * sh.y}), ratio);
-    const double theta = atan2(ph_arg.y, ph_arg.x);
-    double ph = hypot(imp.x, imp.y) * cos(theta);
-    if (isnan(ph)) ph = 0.0;
-    if (ph < 1.0e-3) ph = 0.0;
-    if (ph > 100.0) ph = 0.0;
-    double wn = ph * weights[w];
-    if (wn > 100.0) wn = 0.0;
+    const double wn = wm::clipped_weight(
+        wm::phaseless_factor(on, oo, terms[2 * w], terms[2 * w + 1], pcs, h0p, dt), weights[w]);
     weights[w] = wn;
     overlaps[w] = on;
     local += wn;

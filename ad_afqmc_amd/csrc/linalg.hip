@@ -10,26 +10,14 @@
 //     job-free walker entry point, where no Gram or triangle workspace exists.
 #include "afq_internal.h"
 #include "group.h"
+#include "wave_math.h"
 
 namespace afq {
 namespace {
 
-__device__ inline double2 cmul(double2 a, double2 b) { return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
+using wm::cmul;
+using wm::wave_lds_sync;
 
-// 1 / (a.x + i a.y) without branches or divisions: conj(a) / |a|^2 on a
-// scaled by the power of two 2^-e (exact) that brings max(|re|, |im|) into
-// [0.5, 1), so |a|^2 can neither overflow nor underflow; 1 / |a|^2 from the
-// hardware reciprocal and two Newton steps (within about an ulp).
-__device__ inline double2 crecip_fast(double2 a) {
-  const int e = __builtin_amdgcn_frexp_exp(fmax(fabs(a.x), fabs(a.y)));
-  const double xs = __builtin_amdgcn_ldexp(a.x, -e), ys = __builtin_amdgcn_ldexp(a.y, -e);
-  const double q = fma(xs, xs, ys * ys);
-  double r = __builtin_amdgcn_rcp(q);
-  r = fma(r, fma(-q, r, 1.0), r);
-  r = fma(r, fma(-q, r, 1.0), r);
-  const double rs = __builtin_amdgcn_ldexp(r, -e);
-  return {xs * rs, -ys * rs};
-}
 __device__ inline double2 crecip(double2 a) {
   // Smith's algorithm for 1/(a.x + i a.y)
   if (fabs(a.x) >= fabs(a.y)) {
@@ -75,43 +63,6 @@ __device__ inline double2 crecip(double2 a) {
 // (and pivot-search rows); n <= 64 matrices of such a launch use dynamic LDS.
 constexpr int kLdsN = 64;  // largest n factored in registers (and LDS)
 
-__device__ __forceinline__ double readlane_d(double x, int l) {
-  const long long v = __double_as_longlong(x);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(v & 0xffffffffLL), l);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// max(v, v of the lane that DPP control CTRL names), rows outside ROWS kept
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_fmax(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp((int)(b & 0xffffffffLL), (int)(b & 0xffffffffLL), CTRL, ROWS, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), CTRL, ROWS, 0xF, false);
-  return fmax(v, __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo)));
-}
-
-// maximum of v over the wave (NaN ignored): within quads, half rows and rows,
-// then rows 0-1 into row 1 and 2-3 into row 3 (row_bcast 15), rows 0-1 into
-// row 3 (row_bcast 31); lane 63 holds the result
-__device__ __forceinline__ double wave_fmax(double v) {
-  v = dpp_fmax<0xB1, 0xF>(v);   // quad_perm [1, 0, 3, 2]
-  v = dpp_fmax<0x4E, 0xF>(v);   // quad_perm [2, 3, 0, 1]
-  v = dpp_fmax<0x141, 0xF>(v);  // row_half_mirror
-  v = dpp_fmax<0x140, 0xF>(v);  // row_mirror
-  v = dpp_fmax<0x142, 0xA>(v);  // row_bcast 15
-  v = dpp_fmax<0x143, 0xC>(v);  // row_bcast 31
-  return readlane_d(v, 63);
-}
-
-// orders a wave's LDS accesses (they are performed in issue order) without a
-// work-group barrier
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ void gj_reg_body(const DetInvSet& set, long b) {
   __shared__ double2 ubuf[2][16][64];   // panel columns minus the unit vectors, U[t][row], by panel parity
   __shared__ double2 prow[4][16][16];   // per wave: [column][t] of the panel's pivot rows before the panel
@@ -140,47 +91,7 @@ __device__ __forceinline__ void gj_reg_body(const DetInvSet& set, long b) {
       // ---- the panel, by this wave alone: Gauss-Jordan steps on its 16 columns
       double2 dp = {1.0, 0.0};
       int pj[16];
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        pj[t] = -1;
-        if (t < np) {
-          const double2 x = a[t];
-          const bool cand = lane < n && !((used >> lane) & 1ull);
-          const double v = cand ? fabs(x.x) + fabs(x.y) : -1.0;
-          const double m = wave_fmax(v);
-          // lowest row of maximal measure (a column of NaNs falls back to the
-          // lowest unused row, so p is always a valid row)
-          const unsigned long long best = __ballot(cand && v == m), open = __ballot(cand);
-          const int p = __builtin_ctzll(best ? best : open);
-          pj[t] = p;
-          const double2 d = {readlane_d(x.x, p), readlane_d(x.y, p)};
-          dp = cmul(dp, d);
-          used |= 1ull << p;
-          // column t becomes the unit vector of row p: the common update
-          // below then leaves 1 / d in row p and -f / d in the others
-          const bool isp = lane == p;
-          a[t] = isp ? double2{1.0, 0.0} : double2{0.0, 0.0};
-          if (isp) {
-#pragma unroll
-            for (int s = 0; s < 16; ++s) rrow[s] = a[s];
-          }
-          const double2 dinv = crecip_fast(d);
-          const double sc = isp ? 0.0 : 1.0;
-          const double2 fd = cmul(x, dinv);
-          const double2 g = isp ? dinv : double2{-fd.x, -fd.y};
-          wave_lds_sync();
-          double2 r[16];
-#pragma unroll
-          for (int s = 0; s < 16; ++s) r[s] = rrow[s];
-#pragma unroll
-          for (int s = 0; s < 16; ++s) {
-            const double2 y = a[s];
-            a[s].x = fma(g.x, r[s].x, fma(-g.y, r[s].y, sc * y.x));
-            a[s].y = fma(g.x, r[s].y, fma(g.y, r[s].x, sc * y.y));
-          }
-          wave_lds_sync();
-        }
-      }
+      wm::gj_panel(a, np, n, lane, used, rrow, pj, dp);
       if (lane == 0) {
         pdet[P] = dp;
 #pragma unroll
@@ -229,15 +140,7 @@ __device__ __forceinline__ void gj_reg_body(const DetInvSet& set, long b) {
   if (tid == 0) {
     double2 dprod = {1.0, 0.0};
     for (int q = 0; q < npan; ++q) dprod = cmul(dprod, pdet[q]);
-    // sign of the pivot permutation: n minus its number of cycles transpositions
-    unsigned long long seen = 0;
-    int cycles = 0;
-    for (int s0 = 0; s0 < n; ++s0) {
-      if ((seen >> s0) & 1ull) continue;
-      ++cycles;
-      for (int q = s0; !((seen >> q) & 1ull); q = piv[q]) seen |= 1ull << q;
-    }
-    const bool neg = ((n - cycles) & 1) != 0;
+    const bool neg = wm::odd_permutation(piv, n);
     set.det[b] = neg ? double2{-dprod.x, -dprod.y} : dprod;
   }
   if (!want_inv) return;
@@ -412,15 +315,8 @@ __global__ __launch_bounds__(256) void gj_det_inv_grouped_kernel(const DetInvSet
     gj_det_inv_body<NMAX>(set, item - prefix[j], lds_gj);
 }
 
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
-}
+using wm::wave_sum;
 
-// CGS2 on one panel per work-group, in global memory (the panel stays in L2).
-// Column j: two passes of r = Q[:, :j]^H a_j, a_j -= Q r, then a_j /= |a_j|.
-// The resulting R has a positive real diagonal.
 __global__ __launch_bounds__(256) void cgs2_kernel(double2* __restrict__ Wp, long ld, long sW, int nr, int nc) {
   __shared__ double2 r[128];
   __shared__ double red[4];
