@@ -231,6 +231,8 @@ struct afq_job {
   // (Wr, 4, Gpad); rows padded to 16, k to 32
   uint16_t* lt_split = nullptr;
   uint16_t* xs_split = nullptr;
+  // fused FP64 propagator: exp(-dt/2 h1) per propagated spin, packed
+  double* ep[2] = {nullptr, nullptr};
   // split-BF16 x3 fused propagator: exp(-dt/2 h1) - I per propagated spin as
   // three bf16 planes (k_split_e1_bf16)
   uint16_t* e1s[2] = {nullptr, nullptr};

@@ -10,6 +10,7 @@
 #include "group.h"
 #include "kernels.h"
 #include "small.h"
+#include "trot_f64.h"
 #include "trot_fused.h"
 #include "pipeline.h"
 
@@ -84,6 +85,8 @@ void release(afq_job* j) {
   fr(j->rot_chol32[0]);
   if (!j->rhf) fr(j->rot_chol32[1]);
   fr(j->vhs32);
+  fr(j->ep[0]);
+  fr(j->ep[1]);
   fr(j->e1s[0]);
   fr(j->e1s[1]);
   fr(j->vsplit);
@@ -710,6 +713,23 @@ int trotprop(afq_job* j, void* up, void* dn, const double2* xs, hipStream_t st) 
     AFQ_TRY(gemm_f64(g, st));
   }
   PanelCols pc(j);
+  if (j->sym_chol && j->ep[0]) {
+    TrotF64 f;
+    f.N = N;
+    f.W = W;
+    f.nspin = j->nspin_prop;
+    f.nterms = j->d.n_exp_terms;
+    for (int s = 0; s < j->nspin_prop; ++s) {
+      f.wb[s] = static_cast<double2*>(s == 0 ? up : dn);
+      f.c[s] = pc.c[s];
+      f.e[s] = j->ep[s];
+    }
+    f.vhs = j->vhsp;
+    f.npk = j->npk;
+    f.t0 = j->tbuf[0];
+    ProfScope ps(j, AFQ_K_TAYLOR, st);
+    return trot_f64(f, st);
+  }
   const long per = (long)N * pc.ctot;
   double2* t0 = j->tbuf[0];
   double2* t1 = j->tbuf[1];
@@ -1158,6 +1178,10 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
   } else {
     A_(j->vhs, W * N * N);
     for (auto& t : j->tbuf) A_(t, W * N * wprop);
+    if (j->npk > 0 && trot_f64_supported((int)N)) {
+      A_(j->ep[0], trot_f64_e_elems((int)N));
+      if (!j->restricted) A_(j->ep[1], trot_f64_e_elems((int)N));
+    }
   }
   A_(j->ov_new, W);
   A_(j->coul, 2 * W * G);
@@ -1437,6 +1461,7 @@ int afq_build_propagation_intermediates(afq_job_t j, void* stream) {
     AFQ_TRY(expm_device(As, N, j->exp_h1[s], j->tmp_nn + 5 * NN, j->dscratch, st));
     if (j->lp) AFQ_TRY(k_minus_identity_f32(j->exp_h1[s], j->exp_h1m32[s], N, st));
     if (j->e1s[s]) AFQ_TRY(k_split_e1_bf16(j->exp_h1[s], N, j->e1s[s], st));
+    if (j->ep[s]) AFQ_TRY(k_pack_e_f64(j->exp_h1[s], N, j->ep[s], st));
   }
   AFQ_HIP(hipMemcpyAsync(&j->h0_prop_host, j->h0_prop, sizeof(double2), hipMemcpyDeviceToHost, st));
   AFQ_HIP(hipStreamSynchronize(st));
@@ -1510,6 +1535,7 @@ int afq_set_intermediate(afq_job_t j, int which, int spin, const void* src, void
       j->have_exp[spin] = true;
       if (j->lp) AFQ_TRY(k_minus_identity_f32(j->exp_h1[spin], j->exp_h1m32[spin], (int)N, S(stream)));
       if (j->e1s[spin]) AFQ_TRY(k_split_e1_bf16(j->exp_h1[spin], (int)N, j->e1s[spin], S(stream)));
+      if (j->ep[spin]) AFQ_TRY(k_pack_e_f64(j->exp_h1[spin], (int)N, j->ep[spin], S(stream)));
       break;
     default: break;
   }
