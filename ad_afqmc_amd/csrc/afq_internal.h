@@ -263,8 +263,10 @@ struct afq_job {
   long npk = 0;
   bool sym_chol = false;
   double* cholp = nullptr;                // (G, npk) FP64 packed L
-  double2* vhsp = nullptr;                // (W, npk) FP64 packed VHS
+  double2* vhsp = nullptr;                // (W, npk) FP64 packed VHS, or by blocks (vhs_f64) with ep
   float2* vhsp32 = nullptr;               // (W, npk) reduced-precision packed VHS
+  double* fb_ws = nullptr;                // partial sums of the FP64 force bias
+  long fb_ws_elems = 0;
   double* gemm_ws = nullptr;              // split-K workspace
   long gemm_ws_elems = 0;
 

@@ -12,6 +12,7 @@
 #include "small.h"
 #include "trot_f64.h"
 #include "trot_fused.h"
+#include "walker_gemm.h"
 #include "pipeline.h"
 
 namespace afq {
@@ -76,6 +77,7 @@ void release(afq_job* j) {
   fr(j->cum);
   fr(j->tmp_nn);
   fr(j->gemm_ws);
+  fr(j->fb_ws);
   fr(j->chol32);
   fr(j->cholp);
   fr(j->vhsp);
@@ -265,6 +267,23 @@ int force_bias_gemm(afq_job* j, double2* out, hipStream_t st) {
     b.ws_elems = j->gemm_ws_elems;
     return gemm_bf3(b, st);
   }
+  if (!j->lp) {
+    ForceBias64 f;
+    f.W = j->W;
+    f.G = j->G;
+    f.nspin = j->nspin_meas;
+    for (int s = 0; s < j->nspin_meas; ++s) {
+      f.K[s] = (long)j->nocc[s] * j->N;
+      f.green[s] = j->green[s];
+      f.rc[s] = j->rot_chol[s];
+    }
+    f.fac = j->one_spin ? 2.0 : 1.0;
+    f.out = out;
+    f.ws = j->fb_ws;
+    f.ws_elems = j->fb_ws_elems;
+    ProfScope ps(j, AFQ_K_FORCE_BIAS, st);
+    return force_bias_f64(f, st);
+  }
   for (int s = 0; s < j->nspin_meas; ++s) {
     const int O = j->nocc[s];
     Gemm g;
@@ -311,11 +330,9 @@ int force_bias_gemm(afq_job* j, double2* out, hipStream_t st) {
       b.ws = j->gemm_ws;
       b.ws_elems = j->gemm_ws_elems;
       AFQ_TRY(gemm_bf3(b, st));
-    } else if (j->lp) {
+    } else {
       g.B = j->rot_chol32[s];
       AFQ_TRY(gemm_lp(LpKind::FORCE_BIAS, false, g, st));
-    } else {
-      AFQ_TRY(gemm_f64(g, st));
     }
   }
   return AFQ_OK;
@@ -694,6 +711,27 @@ int trotprop(afq_job* j, void* up, void* dn, const double2* xs, hipStream_t st) 
   if (j->lp) return trotprop_lp(j, up, dn, xs, st);
   const int N = j->N, W = j->W;
   const long NN = (long)N * N;
+  if (j->sym_chol && j->ep[0]) {
+    {
+      ProfScope ps(j, AFQ_K_VHS, st);
+      AFQ_TRY(vhs_f64(xs, j->cholp, N, j->G, W, std::sqrt(j->d.dt), j->vhsp, st));
+    }
+    PanelCols pc(j);
+    TrotF64 f;
+    f.N = N;
+    f.W = W;
+    f.nspin = j->nspin_prop;
+    f.nterms = j->d.n_exp_terms;
+    for (int s = 0; s < j->nspin_prop; ++s) {
+      f.wb[s] = static_cast<double2*>(s == 0 ? up : dn);
+      f.c[s] = pc.c[s];
+      f.e[s] = j->ep[s];
+    }
+    f.vhs = j->vhsp;
+    f.t0 = j->tbuf[0];
+    ProfScope ps(j, AFQ_K_TAYLOR, st);
+    return trot_f64(f, st);
+  }
   {
     const bool sym = j->sym_chol;
     const long ncols = sym ? j->npk : NN;
@@ -713,23 +751,6 @@ int trotprop(afq_job* j, void* up, void* dn, const double2* xs, hipStream_t st) 
     AFQ_TRY(gemm_f64(g, st));
   }
   PanelCols pc(j);
-  if (j->sym_chol && j->ep[0]) {
-    TrotF64 f;
-    f.N = N;
-    f.W = W;
-    f.nspin = j->nspin_prop;
-    f.nterms = j->d.n_exp_terms;
-    for (int s = 0; s < j->nspin_prop; ++s) {
-      f.wb[s] = static_cast<double2*>(s == 0 ? up : dn);
-      f.c[s] = pc.c[s];
-      f.e[s] = j->ep[s];
-    }
-    f.vhs = j->vhsp;
-    f.npk = j->npk;
-    f.t0 = j->tbuf[0];
-    ProfScope ps(j, AFQ_K_TAYLOR, st);
-    return trot_f64(f, st);
-  }
   const long per = (long)N * pc.ctot;
   double2* t0 = j->tbuf[0];
   double2* t1 = j->tbuf[1];
@@ -1134,7 +1155,7 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
       A_(j->vhsp32, W * j->npk);
     } else {
       A_(j->cholp, G * j->npk);
-      A_(j->vhsp, W * j->npk);
+      A_(j->vhsp, W * (trot_f64_supported((int)N) ? vhs_f64_elems((int)N) : j->npk));
     }
   }
   if (j->lp) {
@@ -1196,6 +1217,13 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
   A_(j->tmp_nn, 8 * N * N);
   // split-K partials: up to 16 slices of the (W, G) complex force bias, or of an N x N setup product
   j->gemm_ws_elems = 16 * std::max(2 * W * G, N * N);
+  if (!j->lp) {
+    j->fb_ws_elems = 0;
+    for (long w = 1; w <= W; w = w < W ? std::min(W, 2 * w) : W + 1)
+      j->fb_ws_elems = std::max(j->fb_ws_elems, force_bias_f64_ws((int)w, (int)G, j->nocc[0] * N,
+                                                                  j->nspin_meas > 1 ? j->nocc[1] * N : 0));
+    A_(j->fb_ws, j->fb_ws_elems);
+  }
   A_(j->gemm_ws, j->gemm_ws_elems);
   A_(j->dscratch, 8);
   if (small_steps(j)) {

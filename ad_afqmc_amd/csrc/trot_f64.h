@@ -9,8 +9,7 @@ struct TrotF64 {
   int c[2] = {0, 0};                       // columns of each walker buffer
   double2* wb[2] = {nullptr, nullptr};     // (W, N, c), in place
   const double* e[2] = {nullptr, nullptr}; // packed exp(-dt/2 h1)
-  const double2* vhs = nullptr;            // (W, npk) packed symmetric VHS
-  long npk = 0;
+  const double2* vhs = nullptr;            // the blocks of vhs_f64
   double2* t0 = nullptr;                   // scratch, (W, N, c[0] + c[1])
 };
 bool trot_f64_supported(int N);

@@ -10,9 +10,9 @@
 // With A = VHS complex, D[:, (j, re/im)] += Re A . B + Im A . B', B' the columns
 // of B swapped in pairs with a sign, so a 16 x 16 block takes two MFMAs per
 // 4-deep step and no column is padded but the last.  A's fragments go straight
-// from the packed lower block triangle to registers (a block above the diagonal
-// is read from its mirror), eight k ahead of their use; k = 4 q + t within a
-// 16-deep block for lane group q and MFMA t, on both operands.
+// from memory to registers, 1 KB of consecutive bytes each, eight k ahead of
+// their use; k = 4 q + t within a 16-deep block for lane group q and MFMA t, on
+// both operands.
 //
 // Row blocks: every wave takes R / 8 of them, four more go to the first waves of
 // the four SIMDs, and the last one to three are split by columns over the waves,
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(NT, 2) void trot_f64_kernel(TrotArgs a) {
   const int d0 = 16 * NB * slab, dw = min(16 * NB, 2 * cs - d0);  // real columns of the slab
   double* wb = reinterpret_cast<double*>(f.wb[s] + w * (long)N * cs) + d0;
   double* t0 = reinterpret_cast<double*>(f.t0 + w * (long)N * ct + (s ? f.c[0] : 0)) + d0;
-  const double2* V = f.vhs + w * f.npk;
+  const double2* V = f.vhs + w * 256L * R * R + lane;
   const double* E = f.e[s];
 
   // row blocks of this wave, and its column-split blocks of the last rows
@@ -121,16 +121,13 @@ __global__ __launch_bounds__(NT, 2) void trot_f64_kernel(TrotArgs a) {
       for (int m = 0; m < MB + XB; ++m) {
         const int ib = rb[m], k = on[m] ? kb : 0, hh = on[m] ? h : 0;
         if (VH) {
-          const bool low = ib >= k;
-          const int b = low ? ib * (ib + 1) / 2 + k : k * (k + 1) / 2 + ib;
-          const double2* src = V + 256L * b;
-          const int o = low ? c16 * 16 + 4 * q + 2 * hh : (4 * q + 2 * hh) * 16 + c16, st = low ? 1 : 16;
-          F.x[m][0] = src[o];
-          F.x[m][1] = src[o + st];
+          const double2* src = V + 256L * (ib * R + k) + 128 * hh;
+          F.x[m][0] = src[0];
+          F.x[m][1] = src[64];
         } else {
-          const double* src = E + 256L * (ib * R + k) + (4 * q + 2 * hh) * 16 + c16;
+          const double* src = E + 256L * (ib * R + k) + 128 * hh + lane;
           F.x[m][0].x = src[0];
-          F.x[m][1].x = src[16];
+          F.x[m][1].x = src[64];
         }
       }
     };
@@ -230,11 +227,12 @@ __global__ __launch_bounds__(NT, 2) void trot_f64_kernel(TrotArgs a) {
   });
 }
 
-// E (N x N, row-major) -> [row block][k block][k][row], zero past N
+// E (N x N, row-major) -> [row block][k block][k % 4][k / 4][row], zero past N
 __global__ void pack_e_kernel(const double* __restrict__ e, int N, int R, double* __restrict__ out) {
   const long t = blockIdx.x * 256L + threadIdx.x;
   if (t >= 256L * R * R) return;
-  const int b = (int)(t >> 8), i = 16 * (b / R) + (int)(t & 15), k = 16 * (b % R) + (int)((t >> 4) & 15);
+  const int b = (int)(t >> 8), i = 16 * (b / R) + (int)(t & 15);
+  const int k = 16 * (b % R) + 4 * (int)((t >> 4) & 3) + (int)((t >> 6) & 3);
   out[t] = i < N && k < N ? e[(long)i * N + k] : 0.0;
 }
 
