@@ -904,7 +904,7 @@ struct Seg {
     }
     if (sp.nsp == 2) AFQ_TRY(k_axpby4(hbar_tot, b.hmodbar, b.hmodbar + NN, 1.0, nullptr, nullptr, 0.0, NN, st));
     // m adjoint: + h0_prop' m (h0_prop = -h0 + sum m^2/2) + sum L_g . hbar (v1 = -sum m_g L_g)
-    AFQ_TRY(GB(G, 1, NN).a(j->chol, NN, 0, false).b(hbar_tot, 1, 0, false).c(b.tg, 1, 0).run(st));
+    AFQ_TRY(GB(G, 1, NN).a(j->chol, NN, 0, false).b(hbar_tot, 1, 0, false).c(b.tg, 1, 0).ws(j).run(st));
     LAUNCH(adj_mbar_final_kernel, G, b.mbar, j->mreal, b.scal + 1, b.tg, (int)G);
     // L adjoint
     AFQ_TRY(cpy(chol_bar, b.Lbar, sizeof(double) * G * NN));

@@ -950,9 +950,14 @@ int compute_v0(afq_job* j, double* v0, hipStream_t st) {
   const int N = j->N, G = j->G;
   const long NN = (long)N * N;
   // accumulated over gamma chunks of a permuted copy: v0 = perm (N x nN) . L_chunk (nN x N)
-  long gch = std::max(1L, std::min((long)G, (64L << 20) / (long)(sizeof(double) * NN)));
-  double* perm = nullptr;
-  AFQ_TRY(dalloc_n(&perm, (size_t)(gch * NN)));
+  const long gch = std::max(1L, std::min((long)G, (64L << 20) / (long)(sizeof(double) * NN)));
+  // the copy goes into the VHS buffer, which nothing uses between steps, where that holds it
+  double* own = nullptr;
+  double* perm = reinterpret_cast<double*>(j->vhs);
+  if (!perm || 2L * j->Wcap < gch) {
+    AFQ_TRY(dalloc_n(&own, (size_t)(gch * NN)));
+    perm = own;
+  }
   int rc = AFQ_OK;
   for (int g0 = 0; g0 < G && rc == AFQ_OK; g0 += (int)gch) {
     const int n = (int)std::min(gch, (long)(G - g0));
@@ -974,8 +979,10 @@ int compute_v0(afq_job* j, double* v0, hipStream_t st) {
     g.beta = double2{g0 == 0 ? 0.0 : 1.0, 0.0};
     rc = gemm_f64(g, st);
   }
-  (void)hipStreamSynchronize(st);
-  (void)hipFree(perm);
+  if (own) {
+    (void)hipStreamSynchronize(st);
+    (void)hipFree(own);
+  }
   return rc;
 }
 
@@ -1457,6 +1464,8 @@ int afq_build_propagation_intermediates(afq_job_t j, void* stream) {
     g.ldb = 1;
     g.C = j->mreal;
     g.ldc = 1;
+    g.ws = j->gemm_ws;
+    g.ws_elems = j->gemm_ws_elems;
     AFQ_TRY(gemm_f64(g, st));
   }
   double* mfr = j->mreal + G;

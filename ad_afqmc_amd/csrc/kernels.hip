@@ -74,6 +74,7 @@ __global__ void norm1_kernel(const double* A, int n, double* out) {
   double best = 0.0;
   for (int j = threadIdx.x; j < n; j += 256) {
     double s = 0.0;
+#pragma unroll 16
     for (int i = 0; i < n; ++i) s += fabs(A[(long)i * n + j]);
     best = fmax(best, s);
   }
@@ -418,9 +419,16 @@ __global__ void sym_check_kernel(const double* __restrict__ L, long total, int N
     dmax = fmax(dmax, __shfl_xor(dmax, off));
     amax = fmax(amax, __shfl_xor(amax, off));
   }
+  // one pair of atomics a block: they serialise on their two words
+  __shared__ double red[2][4];
   if ((threadIdx.x & 63) == 0) {
-    atomicMax(&out[0], (unsigned long long)__double_as_longlong(dmax));
-    atomicMax(&out[1], (unsigned long long)__double_as_longlong(amax));
+    red[0][threadIdx.x >> 6] = dmax;
+    red[1][threadIdx.x >> 6] = amax;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const double* r = red[threadIdx.x];
+    atomicMax(&out[threadIdx.x], (unsigned long long)__double_as_longlong(fmax(fmax(r[0], r[1]), fmax(r[2], r[3]))));
   }
 }
 
@@ -640,7 +648,7 @@ int k_sym_check(const double* L, int G, int N, unsigned long long* out2, hipStre
   const long total = (long)G * N * N;
   if (total <= 0) return AFQ_OK;
   AFQ_HIP(hipMemsetAsync(out2, 0, 2 * sizeof(unsigned long long), s));
-  const unsigned blocks = (unsigned)std::min<long>(4096, (total + 255) / 256);
+  const unsigned blocks = (unsigned)std::min<long>(2048, (total + 255) / 256);
   hipLaunchKernelGGL(sym_check_kernel, dim3(blocks), dim3(256), 0, s, L, total, N, out2);
   return launch_status("sym_check_kernel");
 }
