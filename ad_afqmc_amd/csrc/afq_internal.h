@@ -265,6 +265,8 @@ struct afq_job {
   double* cholp = nullptr;                // (G, npk) FP64 packed L
   double2* vhsp = nullptr;                // (W, npk) FP64 packed VHS, or by blocks (vhs_f64) with ep
   float2* vhsp32 = nullptr;               // (W, npk) reduced-precision packed VHS
+  char* slab = nullptr;                   // the allocation that holds the job's buffers
+  size_t slab_bytes = 0;
   double* fb_ws = nullptr;                // partial sums of the FP64 force bias
   long fb_ws_elems = 0;
   double* gemm_ws = nullptr;              // split-K workspace
