@@ -202,8 +202,8 @@ __global__ void adj_seed_kernel(const double* bo, int nb, double* seg, double* e
   *energy_out = num / den;
 }
 
-// F~ = c kappa_w f (in place, layout [g][i][w][j]) and its copy in layout [w][i][g][j].
-__global__ void adj_fscale_kernel(double2* F, const double* kappa, double c, int G, int O, int Wc, double2* Fp) {
+// Fp = c kappa_w f, from layout [g][i][w][j] to [w][i][g][j].  Bound: HBM, one read and one write.
+__global__ void adj_fscale_kernel(const double2* F, const double* kappa, double c, int G, int O, int Wc, double2* Fp) {
   const long n = (long)G * O * Wc * O;
   const long idx = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (idx >= n) return;
@@ -214,9 +214,8 @@ __global__ void adj_fscale_kernel(double2* F, const double* kappa, double c, int
   const int i = (int)(t % O);
   const int g = (int)(t / O);
   const double s = c * kappa[wl];
-  const double2 v = {s * F[idx].x, s * F[idx].y};
-  F[idx] = v;
-  Fp[(((long)wl * O + i) * G + g) * O + j] = v;
+  const double2 v = F[idx];
+  Fp[(((long)wl * O + i) * G + g) * O + j] = double2{s * v.x, s * v.y};
 }
 
 // Cc[w][g] = c kappa_w Ct[w][g] (the Coulomb adjoint from the traces Ct)
@@ -496,10 +495,14 @@ void carve(Arena& ar, Buffers& b, const afq_job* j, const Spins& sp, int nb, int
   b.scal = ar.take<double>(4);
   b.Lbar = ar.take<double>(G * NN);
   b.rh1barC = ar.take<double2>(sp.pt);
-  // exchange-adjoint chunks: F and its permuted copy at most ~2 GB each
+  // Exchange-adjoint chunks: F and its permuted copy at most 256 MB each.  At 2 GB
+  // they were most of the arena, and taking and giving back so much memory on
+  // each call held a gradient up by up to 25 ms (N=100, O=20, G=500, 256 walkers:
+  // 14.6 to 40 ms a call at 2 GB, 14.7 at 256 MB, 15.1 at 128 MB).
   const long omax = std::max(sp.O[0], sp.O[1]);
   const long per_w = G * omax * omax * (long)sizeof(double2);
-  b.Wc = (int)std::max(1L, std::min(W, (2048L << 20) / std::max(1L, per_w)));
+  b.Wc = (int)std::max(1L, std::min(W, (256L << 20) / std::max(1L, per_w)));
+  b.Wc = (int)((W + (W + b.Wc - 1) / b.Wc - 1) / ((W + b.Wc - 1) / b.Wc));  // of about equal size
   b.F = ar.take<double2>(G * omax * b.Wc * omax);
   b.Fp = ar.take<double2>(G * omax * b.Wc * omax);
   b.Cc = ar.take<double2>(W * G);
