@@ -50,7 +50,13 @@ __device__ inline double2 crecip(double2 a) {
 // m): A^-1[pinv[r]][piv[c]] = R[r][c], pinv the inverse permutation; det A =
 // sign(piv) prod of the pivots (the determinant alone runs the same sweep).
 //
-// n > 64 (gj_det_inv_body, n <= 256): the matrix is factored in global memory,
+// 64 < n <= 128 (gj_reg2_body): the same with eight waves and two rows a lane
+// (the first of maximal measure is the lowest again).  Bound by the panels,
+// which one wave factors alone; 40 walkers 256 us at n=100 and 213 at n=82,
+// against 950 and 800 in place in global memory, a barrier and a round trip to
+// L2 for each column.
+//
+// n > 128 (gj_det_inv_body, n <= 256): the matrix is factored in global memory,
 // in the inverse's buffer or the set's scratch (it stays in L2), with explicit
 // row interchanges (the first row of maximal measure at or below k).  Thread t
 // owns the columns t % 64 + 64 c for the rows t/64, t/64 + 4, ..., so the
@@ -61,7 +67,10 @@ __device__ inline double2 crecip(double2 a) {
 // trailing rows and columns are eliminated (the pivots, hence the determinant,
 // are the same).  NMAX = kDetInvMaxN; each thread covers NMAX / 64 columns
 // (and pivot-search rows); n <= 64 matrices of such a launch use dynamic LDS.
-constexpr int kLdsN = 64;  // largest n factored in registers (and LDS)
+constexpr int kLdsN = 64;   // largest n of one register row a lane (and of the LDS Cholesky)
+constexpr int kReg2N = 128;  // largest n of two register rows a lane
+constexpr size_t kReg2Lds = sizeof(double2) * (2 * 16 * kReg2N + 8 * 16 * 16);
+constexpr int det_inv_threads(int nmax) { return nmax == kReg2N ? 512 : 256; }
 
 __device__ __forceinline__ void gj_reg_body(const DetInvSet& set, long b) {
   __shared__ double2 ubuf[2][16][64];   // panel columns minus the unit vectors, U[t][row], by panel parity
@@ -153,6 +162,159 @@ __device__ __forceinline__ void gj_reg_body(const DetInvSet& set, long b) {
     for (int t = 0; t < 16; ++t) {
       const int c = c0 + t;
       if (c < n) dst[row + piv[c]] = a[t];
+    }
+  }
+}
+
+// Gauss-Jordan steps of one wave on a panel of 16 columns, as wm::gj_panel, lane
+// i holding rows i and i + 64.
+__device__ __forceinline__ void gj_panel2(double2 (&a)[2][16], int np, int n, int lane, unsigned long long (&used)[2],
+                                          double2* rrow, int (&pj)[16], double2& dp) {
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    pj[t] = -1;
+    if (t < np) {
+      const double2 x0 = a[0][t], x1 = a[1][t];
+      const bool c0 = lane < n && !((used[0] >> lane) & 1ull), c1 = lane + 64 < n && !((used[1] >> lane) & 1ull);
+      const double v0 = c0 ? fabs(x0.x) + fabs(x0.y) : -1.0, v1 = c1 ? fabs(x1.x) + fabs(x1.y) : -1.0;
+      const double m = wm::wave_fmax(fmax(v0, v1));
+      const unsigned long long b0 = __ballot(c0 && v0 == m), b1 = __ballot(c1 && v1 == m);
+      const unsigned long long o0 = __ballot(c0), o1 = __ballot(c1);
+      const bool any = (b0 | b1) != 0;  // a column of NaNs falls back to the lowest unused row
+      const unsigned long long w0 = any ? b0 : o0, w1 = any ? b1 : o1;
+      const bool hi = w0 == 0;
+      const int l = __builtin_ctzll(hi ? w1 : w0);
+      pj[t] = hi ? 64 + l : l;
+      const double2 xs = {hi ? x1.x : x0.x, hi ? x1.y : x0.y};
+      const double2 d = {wm::readlane_d(xs.x, l), wm::readlane_d(xs.y, l)};
+      dp = cmul(dp, d);
+      used[0] |= hi ? 0ull : 1ull << l;
+      used[1] |= hi ? 1ull << l : 0ull;
+      const bool is0 = !hi && lane == l, is1 = hi && lane == l;
+      a[0][t] = double2{is0 ? 1.0 : 0.0, 0.0};
+      a[1][t] = double2{is1 ? 1.0 : 0.0, 0.0};
+      if (lane == l) {
+#pragma unroll
+        for (int s = 0; s < 16; ++s) rrow[s] = double2{hi ? a[1][s].x : a[0][s].x, hi ? a[1][s].y : a[0][s].y};
+      }
+      const double2 dinv = wm::crecip_fast(d);
+      const double2 f0 = cmul(x0, dinv), f1 = cmul(x1, dinv);
+      const double2 g0 = is0 ? dinv : double2{-f0.x, -f0.y}, g1 = is1 ? dinv : double2{-f1.x, -f1.y};
+      const double s0 = is0 ? 0.0 : 1.0, s1 = is1 ? 0.0 : 1.0;
+      wave_lds_sync();
+#pragma unroll
+      for (int s = 0; s < 16; ++s) {
+        const double2 r = rrow[s], y = a[0][s], z = a[1][s];
+        a[0][s].x = fma(g0.x, r.x, fma(-g0.y, r.y, s0 * y.x));
+        a[0][s].y = fma(g0.x, r.y, fma(g0.y, r.x, s0 * y.y));
+        a[1][s].x = fma(g1.x, r.x, fma(-g1.y, r.y, s1 * z.x));
+        a[1][s].y = fma(g1.x, r.y, fma(g1.y, r.x, s1 * z.y));
+      }
+      wave_lds_sync();
+    }
+  }
+}
+
+// gj_reg_body for 64 < n <= 128: eight waves of 16 columns, each lane with two
+// rows.  lds: kReg2Lds bytes.
+__device__ __forceinline__ void gj_reg2_body(const DetInvSet& set, long b, double2* __restrict__ lds) {
+  double2(*ubuf)[16][128] = reinterpret_cast<double2(*)[16][128]>(lds);             // [2], by panel parity
+  double2(*prow)[16][16] = reinterpret_cast<double2(*)[16][16]>(lds + 2 * 16 * 128);  // [8], per wave
+  __shared__ double2 rrow[16], pdet[8];
+  __shared__ int piv[128], pinv[128];
+  const int n = set.n;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c0 = 16 * wave;
+  const double2* src = set.S + b * set.strideS;
+  for (int e = lane; e < 16 * 16; e += 64) (&prow[wave][0][0])[e] = double2{0.0, 0.0};
+  double2 a[2][16];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      const int r = lane + 64 * h, c = c0 + t;
+      a[h][t] = (r < n && c < n) ? src[r * n + c] : double2{0.0, 0.0};
+    }
+  unsigned long long used[2] = {0, 0};  // rows already used as pivots (wave-uniform)
+  const int npan = (n + 15) >> 4;
+  for (int P = 0; P < npan; ++P) {
+    const int np = min(16, n - 16 * P);
+    double2(&U)[16][128] = ubuf[P & 1];
+    if (wave == P) {
+      double2 dp = {1.0, 0.0};
+      int pj[16];
+      gj_panel2(a, np, n, lane, used, rrow, pj, dp);
+      if (lane == 0) {
+        pdet[P] = dp;
+#pragma unroll
+        for (int t = 0; t < 16; ++t)
+          if (t < np) piv[16 * P + t] = pj[t];
+      }
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        U[t][lane] = (lane == pj[t]) ? double2{a[0][t].x - 1.0, a[0][t].y} : a[0][t];
+        U[t][lane + 64] = (lane + 64 == pj[t]) ? double2{a[1][t].x - 1.0, a[1][t].y} : a[1][t];
+      }
+    }
+    __syncthreads();
+    if (wave != P) {
+      int j0 = -1, j1 = -1;  // the panel's steps whose pivots are this lane's rows
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        const int p = t < np ? __builtin_amdgcn_readfirstlane(piv[16 * P + t]) : -1;
+        if (p >= 64)
+          used[1] |= 1ull << (p - 64);
+        else if (p >= 0)
+          used[0] |= 1ull << p;
+        j0 = (p == lane) ? t : j0;
+        j1 = (p == lane + 64) ? t : j1;
+      }
+      if (c0 < n) {
+        if (j0 >= 0) {
+#pragma unroll
+          for (int s = 0; s < 16; ++s) prow[wave][s][j0] = a[0][s];
+        }
+        if (j1 >= 0) {
+#pragma unroll
+          for (int s = 0; s < 16; ++s) prow[wave][s][j1] = a[1][s];
+        }
+        wave_lds_sync();
+#pragma unroll 4
+        for (int t = 0; t < 16; ++t) {
+          const double2 u0 = U[t][lane], u1 = U[t][lane + 64];
+#pragma unroll
+          for (int s = 0; s < 16; ++s) {
+            const double2 r = prow[wave][s][t];
+            a[0][s].x = fma(u0.x, r.x, fma(-u0.y, r.y, a[0][s].x));
+            a[0][s].y = fma(u0.x, r.y, fma(u0.y, r.x, a[0][s].y));
+            a[1][s].x = fma(u1.x, r.x, fma(-u1.y, r.y, a[1][s].x));
+            a[1][s].y = fma(u1.x, r.y, fma(u1.y, r.x, a[1][s].y));
+          }
+        }
+        wave_lds_sync();
+      }
+    }
+  }
+  __syncthreads();  // piv and pdet complete
+  if (tid < n) pinv[piv[tid]] = tid;
+  if (tid == 0) {
+    double2 dprod = {1.0, 0.0};
+    for (int q = 0; q < npan; ++q) dprod = cmul(dprod, pdet[q]);
+    const bool neg = wm::odd_permutation(piv, n);
+    set.det[b] = neg ? double2{-dprod.x, -dprod.y} : dprod;
+  }
+  if (!set.inv) return;
+  __syncthreads();
+  double2* dst = set.inv + b * set.strideInv;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = lane + 64 * h;
+    if (r < n) {
+      const long row = (long)pinv[r] * n;
+#pragma unroll
+      for (int t = 0; t < 16; ++t)
+        if (c0 + t < n) dst[row + piv[c0 + t]] = a[h][t];
     }
   }
 }
@@ -293,24 +455,28 @@ __device__ __forceinline__ void gj_det_inv_body(const DetInvSet& set, long b, do
 }
 
 template <int NMAX>
-__global__ __launch_bounds__(256) void gj_det_inv_kernel(DetInvSet s0, DetInvSet s1) {
+__global__ __launch_bounds__(det_inv_threads(NMAX)) void gj_det_inv_kernel(DetInvSet s0, DetInvSet s1) {
   extern __shared__ double2 lds_gj[];
   if constexpr (NMAX == kLdsN)
     gj_reg_body(blockIdx.y == 0 ? s0 : s1, blockIdx.x);
+  else if constexpr (NMAX == kReg2N)
+    gj_reg2_body(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
   else
     gj_det_inv_body<NMAX>(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
 }
 
 // Grouped: work-group i factors matrix i - prefix[j] of job j's set.
 template <int NMAX>
-__global__ __launch_bounds__(256) void gj_det_inv_grouped_kernel(const DetInvSet* __restrict__ sets,
-                                                                 const int* __restrict__ prefix, int njobs) {
+__global__ __launch_bounds__(det_inv_threads(NMAX)) void gj_det_inv_grouped_kernel(
+    const DetInvSet* __restrict__ sets, const int* __restrict__ prefix, int njobs) {
   extern __shared__ double2 lds_gj[];
   const int item = blockIdx.x;
   const int j = group_find(prefix, njobs, item);
   const DetInvSet set = sets[j];
   if constexpr (NMAX == kLdsN)
     gj_reg_body(set, item - prefix[j]);
+  else if constexpr (NMAX == kReg2N)
+    gj_reg2_body(set, item - prefix[j], lds_gj);
   else
     gj_det_inv_body<NMAX>(set, item - prefix[j], lds_gj);
 }
@@ -517,7 +683,7 @@ template <int NMAX>
 static int launch_det_inv(const DetInvSet* sets, int nsets, int count, size_t lds, hipStream_t stream) {
   static bool raised = false;
   AFQ_TRY(raise_lds(reinterpret_cast<const void*>(gj_det_inv_kernel<NMAX>), &raised, "det/inverse"));
-  hipLaunchKernelGGL(gj_det_inv_kernel<NMAX>, dim3(count, nsets), dim3(256), lds, stream, sets[0],
+  hipLaunchKernelGGL(gj_det_inv_kernel<NMAX>, dim3(count, nsets), dim3(det_inv_threads(NMAX)), lds, stream, sets[0],
                      sets[nsets > 1 ? 1 : 0]);
   return launch_status("gj_det_inv_kernel");
 }
@@ -530,16 +696,17 @@ int batched_det_inv_sets(const DetInvSet* sets, int nsets, int count, hipStream_
     nmax = std::max(nmax, sets[i].n);
   }
   if (count <= 0) return AFQ_OK;
-  // n <= 64: the matrices stay in registers, no dynamic LDS
-  return nmax <= kLdsN ? launch_det_inv<kLdsN>(sets, nsets, count, 0, stream)
-                       : launch_det_inv<kDetInvMaxN>(sets, nsets, count, matrix_lds_bytes(nmax), stream);
+  // n <= 128: the matrices stay in registers
+  return nmax <= kLdsN    ? launch_det_inv<kLdsN>(sets, nsets, count, 0, stream)
+         : nmax <= kReg2N ? launch_det_inv<kReg2N>(sets, nsets, count, kReg2Lds, stream)
+                          : launch_det_inv<kDetInvMaxN>(sets, nsets, count, matrix_lds_bytes(nmax), stream);
 }
 
 template <int NMAX>
 static int launch_det_inv_grouped(const GroupTab<DetInvSet>& t, size_t lds, hipStream_t stream) {
   static bool raised = false;
   AFQ_TRY(raise_lds(reinterpret_cast<const void*>(gj_det_inv_grouped_kernel<NMAX>), &raised, "det/inverse"));
-  hipLaunchKernelGGL(gj_det_inv_grouped_kernel<NMAX>, dim3((unsigned)t.total), dim3(256), lds, stream, t.params,
+  hipLaunchKernelGGL(gj_det_inv_grouped_kernel<NMAX>, dim3((unsigned)t.total), dim3(det_inv_threads(NMAX)), lds, stream, t.params,
                      t.prefix, t.njobs);
   return launch_status("gj_det_inv_grouped_kernel");
 }
@@ -548,8 +715,9 @@ int det_inv_grouped(const GroupTab<DetInvSet>& t, int nmax, hipStream_t stream) 
   if (t.njobs < 1 || t.total < 1) return AFQ_OK;
   if (nmax < 1 || nmax > kDetInvMaxN)
     return fail(AFQ_E_UNSUPPORTED, "det/inverse kernel supports 1 <= n <= " + std::to_string(kDetInvMaxN));
-  return nmax <= kLdsN ? launch_det_inv_grouped<kLdsN>(t, 0, stream)
-                       : launch_det_inv_grouped<kDetInvMaxN>(t, matrix_lds_bytes(nmax), stream);
+  return nmax <= kLdsN    ? launch_det_inv_grouped<kLdsN>(t, 0, stream)
+         : nmax <= kReg2N ? launch_det_inv_grouped<kReg2N>(t, kReg2Lds, stream)
+                          : launch_det_inv_grouped<kDetInvMaxN>(t, matrix_lds_bytes(nmax), stream);
 }
 
 int batched_det_inv(const double2* S, long strideS, int n, int count, double2* det, double2* inv, long strideInv,

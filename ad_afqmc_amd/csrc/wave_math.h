@@ -135,15 +135,16 @@ __device__ __forceinline__ void gj_panel(double2 (&a)[NP], int np, int n, int la
   }
 }
 
-// sign of the permutation piv of n <= 64 as true for odd: n minus its number of
+// sign of the permutation piv of n <= 128 as true for odd: n minus its number of
 // cycles transpositions
 __device__ inline bool odd_permutation(const int* piv, int n) {
-  unsigned long long seen = 0;
+  unsigned long long s0 = 0, s1 = 0;
+  auto seen = [&](int q) { return (((q < 64 ? s0 : s1) >> (q & 63)) & 1ull) != 0; };
   int cycles = 0;
-  for (int s0 = 0; s0 < n; ++s0) {
-    if ((seen >> s0) & 1ull) continue;
+  for (int s = 0; s < n; ++s) {
+    if (seen(s)) continue;
     ++cycles;
-    for (int q = s0; !((seen >> q) & 1ull); q = piv[q]) seen |= 1ull << q;
+    for (int q = s; !seen(q); q = piv[q]) (q < 64 ? s0 : s1) |= 1ull << (q & 63);
   }
   return ((n - cycles) & 1) != 0;
 }
