@@ -28,33 +28,35 @@ __device__ inline double2 crecip(double2 a) {
   return {r / den, -1.0 / den};
 }
 
-// Gauss-Jordan determinant and inverse, one 256-thread work-group per matrix,
+// Gauss-Jordan determinant and inverse, one work-group per matrix,
 // partial pivoting on the largest |re|+|im| of the pivot column (LAPACK
 // izamax measure).  blockIdx.y selects one of up to two matrix sets (the two
 // spins' overlap matrices factor in one launch, so a CU holds two work-groups
 // at W = 256).
 //
-// n <= 64 (gj_reg_body): the matrix stays in registers.  Lane i of every wave
-// holds row i, wave w the columns 16 w .. 16 w + 15 (one panel).  Rows are
-// never swapped: the pivot of column k is the first (lowest) not yet used row
-// of maximal measure (a DPP maximum and a ballot).  Panel P is factored by
-// wave P alone, column by column, on its own 16 columns (the pivot row through
-// LDS within the wave; column k replaced by the unit vector of its pivot row,
-// so one branch-free update leaves a_p / d in the pivot row and a - (f / d) a_p
-// elsewhere).  The panel's steps compose to M = I + sum_t U_t e_{p_t}^T, and
-// because of the unit vectors the panel's columns end up holding M e_{p_t}:
-// after one barrier every other wave applies M to its columns as one rank-16
-// update, a += U a[p_t] (rows p_t as they were before the panel).  Four
-// barriers per matrix instead of one per column.  The result R relates to the
-// inverse through the pivot sequence piv (row piv[m] was the pivot of column
-// m): A^-1[pinv[r]][piv[c]] = R[r][c], pinv the inverse permutation; det A =
-// sign(piv) prod of the pivots (the determinant alone runs the same sweep).
+// n <= 128 (gj_reg_body): the matrix stays in registers.  Lane i of every wave
+// holds row i, and row i + 64 where n > 64, wave w the columns 8 w .. 8 w + 7
+// (one panel).  Rows are never swapped: the pivot of column k is the first
+// (lowest) not yet used row of maximal measure (a DPP maximum and a ballot).
+// Panel P is factored by wave P alone, column by column, on its own columns
+// (the pivot row through scalar registers; column k replaced by the unit vector
+// of its pivot row, so one branch-free update leaves a_p / d in the pivot row and
+// a - (f / d) a_p elsewhere).  The panel's steps compose to
+// M = I + sum_t U_t e_{p_t}^T, and because of the unit vectors the panel's
+// columns end up holding M e_{p_t}: after one barrier every other wave applies M
+// to its columns as one rank-8 update, a += U a[p_t] (rows p_t as they were
+// before the panel).  One barrier a panel instead of one a column.  The result R
+// relates to the inverse through the pivot sequence piv (row piv[m] was the
+// pivot of column m): A^-1[pinv[r]][piv[c]] = R[r][c], pinv the inverse
+// permutation; det A = sign(piv) prod of the pivots (the determinant alone runs
+// the same sweep).
 //
-// 64 < n <= 128 (gj_reg2_body): the same with eight waves and two rows a lane
-// (the first of maximal measure is the lowest again).  Bound by the panels,
-// which one wave factors alone; 40 walkers 256 us at n=100 and 213 at n=82,
-// against 950 and 800 in place in global memory, a barrier and a round trip to
-// L2 for each column.
+// Bound by the chain of panel steps and updates (some 0.4 us a column and 2 us a
+// panel).  Panels of 8 columns on 8 waves, against 16 on 4: n=20, 256 matrices
+// 30 -> 20 us; n=40, 512 57 -> 43; n=60 and 58, 2 x 256 84 -> 73; n=100, 40
+// matrices 210 -> 156 (950 in place in global memory, with a barrier and a round
+// trip to L2 for each column); n=82, 48 177 -> 127 (800).  The same steps as a
+// loop, one column after another through the registers, were 3-15% slower.
 //
 // n > 128 (gj_det_inv_body, n <= 256): the matrix is factored in global memory,
 // in the inverse's buffer or the set's scratch (it stays in L2), with explicit
@@ -69,252 +71,141 @@ __device__ inline double2 crecip(double2 a) {
 // (and pivot-search rows); n <= 64 matrices of such a launch use dynamic LDS.
 constexpr int kLdsN = 64;   // largest n of one register row a lane (and of the LDS Cholesky)
 constexpr int kReg2N = 128;  // largest n of two register rows a lane
-constexpr size_t kReg2Lds = sizeof(double2) * (2 * 16 * kReg2N + 8 * 16 * 16);
-constexpr int det_inv_threads(int nmax) { return nmax == kReg2N ? 512 : 256; }
+constexpr int kPanel = 8;    // columns of a wave
+constexpr size_t reg_lds(int h, int nmax) {
+  const size_t work = sizeof(double2) * h * 64 * (2 * kPanel + kPanel);
+  return h == 1 ? std::max(work, sizeof(double2) * nmax * (nmax | 1)) : work;
+}
+constexpr int det_inv_threads(int nmax) { return nmax == kLdsN ? 512 : nmax == kReg2N ? 1024 : 256; }
 
-__device__ __forceinline__ void gj_reg_body(const DetInvSet& set, long b) {
-  __shared__ double2 ubuf[2][16][64];   // panel columns minus the unit vectors, U[t][row], by panel parity
-  __shared__ double2 prow[4][16][16];   // per wave: [column][t] of the panel's pivot rows before the panel
-  __shared__ double2 rrow[16];          // the panel wave's current pivot row
-  __shared__ double2 pdet[4];           // product of each panel's pivots
-  __shared__ int piv[64], pinv[64];
+// H rows a lane (n <= 64 H).  lds: reg_lds(H, n) bytes.
+template <int H>
+__device__ __forceinline__ void gj_reg_body(const DetInvSet& set, long b, double2* __restrict__ lds) {
+  constexpr int ROWS = 64 * H, NW = ROWS / kPanel, NT = 64 * NW;
+  double2(*ubuf)[kPanel][ROWS] = reinterpret_cast<double2(*)[kPanel][ROWS]>(lds);  // [2]: U[t][row], by panel parity
+  // [NW]: per wave, [column][t] of the panel's pivot rows before the panel
+  double2(*prow)[kPanel][kPanel] = reinterpret_cast<double2(*)[kPanel][kPanel]>(lds + 2 * kPanel * ROWS);
+  __shared__ double2 pdet[NW];  // product of each panel's pivots
+  __shared__ int piv[ROWS], pinv[ROWS];
   const int n = set.n;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c0 = 16 * wave;  // this wave's columns c0 .. c0 + 15
-  const bool want_inv = set.inv != nullptr;
+  const int c0 = kPanel * wave;  // this wave's first column
   const double2* src = set.S + b * set.strideS;
-  for (int e = tid; e < 4 * 16 * 16; e += 256) (&prow[0][0][0])[e] = double2{0.0, 0.0};
-  double2 a[16];
-#pragma unroll
-  for (int t = 0; t < 16; ++t) {
-    const int c = c0 + t;
-    a[t] = (lane < n && c < n) ? src[lane * n + c] : double2{0.0, 0.0};
+  double2 a[H][kPanel];
+  // one row a lane: through LDS, in rows of an odd number of entries, so that
+  // global memory is read in runs (lanes a row apart: 9 of 84 us at n = 60)
+  const int ld = n | 1;
+  if constexpr (H == 1) {
+    for (int e = tid; e < n * n; e += NT) {
+      const int r = e / n;
+      lds[r * ld + e - r * n] = src[e];
+    }
+    __syncthreads();
+    src = lds;
   }
-  unsigned long long used = 0;  // rows already used as pivots (wave-uniform)
-  const int npan = (n + 15) >> 4;
+  const int lsrc = H == 1 ? ld : n;
+#pragma unroll
+  for (int h = 0; h < H; ++h)
+#pragma unroll
+    for (int t = 0; t < kPanel; ++t) {
+      const int r = lane + 64 * h, c = c0 + t;
+      a[h][t] = (r < n && c < n) ? src[r * lsrc + c] : double2{0.0, 0.0};
+    }
+  if constexpr (H == 1) __syncthreads();
+  unsigned long long used[H] = {};  // rows already used as pivots (wave-uniform)
+  const int npan = (n + kPanel - 1) / kPanel;
   for (int P = 0; P < npan; ++P) {
-    const int np = min(16, n - 16 * P);
-    double2(&U)[16][64] = ubuf[P & 1];
+    const int np = min(kPanel, n - kPanel * P);
+    double2(&U)[kPanel][ROWS] = ubuf[P & 1];
     if (wave == P) {
-      // ---- the panel, by this wave alone: Gauss-Jordan steps on its 16 columns
+      // ---- the panel, by this wave alone: Gauss-Jordan steps on its columns
       double2 dp = {1.0, 0.0};
-      int pj[16];
-      wm::gj_panel(a, np, n, lane, used, rrow, pj, dp);
+      int pj[kPanel];
+      wm::gj_panel(a, np, n, lane, used, pj, dp);
       if (lane == 0) {
         pdet[P] = dp;
 #pragma unroll
-        for (int t = 0; t < 16; ++t)
-          if (t < np) piv[16 * P + t] = pj[t];
+        for (int t = 0; t < kPanel; ++t)
+          if (t < np) piv[kPanel * P + t] = pj[t];
       }
       // the panel's transform M = I + sum_t U_t e_{p_t}^T: column t of the
-      // panel now holds M e_{p_t} (zero past the panel's width)
+      // panel now holds M e_{p_t}
 #pragma unroll
-      for (int t = 0; t < 16; ++t) U[t][lane] = (lane == pj[t]) ? double2{a[t].x - 1.0, a[t].y} : a[t];
+      for (int t = 0; t < kPanel; ++t)
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+          U[t][lane + 64 * h] = (lane + 64 * h == pj[t]) ? double2{a[h][t].x - 1.0, a[h][t].y} : a[h][t];
     }
     __syncthreads();
-    if (wave != P) {
-      int pj[16];
+    if (wave != P && c0 < n) {
+      int jj[H];  // the panel's steps whose pivots are this lane's rows
 #pragma unroll
-      for (int t = 0; t < 16; ++t) pj[t] = t < np ? __builtin_amdgcn_readfirstlane(piv[16 * P + t]) : -1;
+      for (int h = 0; h < H; ++h) jj[h] = -1;
 #pragma unroll
-      for (int t = 0; t < 16; ++t)
-        if (pj[t] >= 0) used |= 1ull << pj[t];
-      if (c0 < n) {
-        // ---- apply the panel to this wave's columns: a += U a[p_t] (rows
-        // p_t before the panel, through LDS: the lane holding row p_t writes it)
-        int jj = -1;
+      for (int t = 0; t < kPanel; ++t) {
+        const int p = t < np ? __builtin_amdgcn_readfirstlane(piv[kPanel * P + t]) : -1;
 #pragma unroll
-        for (int t = 0; t < 16; ++t) jj = (pj[t] == lane) ? t : jj;
-        if (jj >= 0) {
-#pragma unroll
-          for (int s = 0; s < 16; ++s) prow[wave][s][jj] = a[s];
+        for (int h = 0; h < H; ++h) {
+          used[h] |= p >= 0 && (p >> 6) == h ? 1ull << (p & 63) : 0ull;
+          jj[h] = (p == lane + 64 * h) ? t : jj[h];
         }
-        wave_lds_sync();
+      }
+      // ---- apply the panel to this wave's columns: a += U a[p_t] (rows
+      // p_t before the panel, through LDS: the lane holding row p_t writes it)
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
-          const double2 u = U[t][lane];
+      for (int h = 0; h < H; ++h)
+        if (jj[h] >= 0) {
 #pragma unroll
-          for (int s = 0; s < 16; ++s) {
-            const double2 r = prow[wave][s][t];
-            a[s].x = fma(u.x, r.x, fma(-u.y, r.y, a[s].x));
-            a[s].y = fma(u.x, r.y, fma(u.y, r.x, a[s].y));
-          }
+          for (int s = 0; s < kPanel; ++s) prow[wave][s][jj[h]] = a[h][s];
         }
-        wave_lds_sync();
-      }
-    }
-  }
-  __syncthreads();  // piv and pdet complete
-  if (tid == 0) {
-    double2 dprod = {1.0, 0.0};
-    for (int q = 0; q < npan; ++q) dprod = cmul(dprod, pdet[q]);
-    const bool neg = wm::odd_permutation(piv, n);
-    set.det[b] = neg ? double2{-dprod.x, -dprod.y} : dprod;
-  }
-  if (!want_inv) return;
-  if (tid < n) pinv[piv[tid]] = tid;
-  __syncthreads();
-  double2* dst = set.inv + b * set.strideInv;
-  if (lane < n) {
-    const long row = (long)pinv[lane] * n;
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const int c = c0 + t;
-      if (c < n) dst[row + piv[c]] = a[t];
-    }
-  }
-}
-
-// Gauss-Jordan steps of one wave on a panel of 16 columns, as wm::gj_panel, lane
-// i holding rows i and i + 64.
-__device__ __forceinline__ void gj_panel2(double2 (&a)[2][16], int np, int n, int lane, unsigned long long (&used)[2],
-                                          double2* rrow, int (&pj)[16], double2& dp) {
-#pragma unroll
-  for (int t = 0; t < 16; ++t) {
-    pj[t] = -1;
-    if (t < np) {
-      const double2 x0 = a[0][t], x1 = a[1][t];
-      const bool c0 = lane < n && !((used[0] >> lane) & 1ull), c1 = lane + 64 < n && !((used[1] >> lane) & 1ull);
-      const double v0 = c0 ? fabs(x0.x) + fabs(x0.y) : -1.0, v1 = c1 ? fabs(x1.x) + fabs(x1.y) : -1.0;
-      const double m = wm::wave_fmax(fmax(v0, v1));
-      const unsigned long long b0 = __ballot(c0 && v0 == m), b1 = __ballot(c1 && v1 == m);
-      const unsigned long long o0 = __ballot(c0), o1 = __ballot(c1);
-      const bool any = (b0 | b1) != 0;  // a column of NaNs falls back to the lowest unused row
-      const unsigned long long w0 = any ? b0 : o0, w1 = any ? b1 : o1;
-      const bool hi = w0 == 0;
-      const int l = __builtin_ctzll(hi ? w1 : w0);
-      pj[t] = hi ? 64 + l : l;
-      const double2 xs = {hi ? x1.x : x0.x, hi ? x1.y : x0.y};
-      const double2 d = {wm::readlane_d(xs.x, l), wm::readlane_d(xs.y, l)};
-      dp = cmul(dp, d);
-      used[0] |= hi ? 0ull : 1ull << l;
-      used[1] |= hi ? 1ull << l : 0ull;
-      const bool is0 = !hi && lane == l, is1 = hi && lane == l;
-      a[0][t] = double2{is0 ? 1.0 : 0.0, 0.0};
-      a[1][t] = double2{is1 ? 1.0 : 0.0, 0.0};
-      if (lane == l) {
-#pragma unroll
-        for (int s = 0; s < 16; ++s) rrow[s] = double2{hi ? a[1][s].x : a[0][s].x, hi ? a[1][s].y : a[0][s].y};
-      }
-      const double2 dinv = wm::crecip_fast(d);
-      const double2 f0 = cmul(x0, dinv), f1 = cmul(x1, dinv);
-      const double2 g0 = is0 ? dinv : double2{-f0.x, -f0.y}, g1 = is1 ? dinv : double2{-f1.x, -f1.y};
-      const double s0 = is0 ? 0.0 : 1.0, s1 = is1 ? 0.0 : 1.0;
       wave_lds_sync();
 #pragma unroll
-      for (int s = 0; s < 16; ++s) {
-        const double2 r = rrow[s], y = a[0][s], z = a[1][s];
-        a[0][s].x = fma(g0.x, r.x, fma(-g0.y, r.y, s0 * y.x));
-        a[0][s].y = fma(g0.x, r.y, fma(g0.y, r.x, s0 * y.y));
-        a[1][s].x = fma(g1.x, r.x, fma(-g1.y, r.y, s1 * z.x));
-        a[1][s].y = fma(g1.x, r.y, fma(g1.y, r.x, s1 * z.y));
+      for (int t = 0; t < kPanel; ++t) {
+        if (t >= np) break;  // uniform
+        double2 u[H];
+#pragma unroll
+        for (int h = 0; h < H; ++h) u[h] = U[t][lane + 64 * h];
+#pragma unroll
+        for (int s = 0; s < kPanel; ++s) {
+          const double2 r = prow[wave][s][t];
+#pragma unroll
+          for (int h = 0; h < H; ++h) {
+            a[h][s].x = fma(u[h].x, r.x, fma(-u[h].y, r.y, a[h][s].x));
+            a[h][s].y = fma(u[h].x, r.y, fma(u[h].y, r.x, a[h][s].y));
+          }
+        }
       }
       wave_lds_sync();
     }
   }
-}
-
-// gj_reg_body for 64 < n <= 128: eight waves of 16 columns, each lane with two
-// rows.  lds: kReg2Lds bytes.
-__device__ __forceinline__ void gj_reg2_body(const DetInvSet& set, long b, double2* __restrict__ lds) {
-  double2(*ubuf)[16][128] = reinterpret_cast<double2(*)[16][128]>(lds);             // [2], by panel parity
-  double2(*prow)[16][16] = reinterpret_cast<double2(*)[16][16]>(lds + 2 * 16 * 128);  // [8], per wave
-  __shared__ double2 rrow[16], pdet[8];
-  __shared__ int piv[128], pinv[128];
-  const int n = set.n;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c0 = 16 * wave;
-  const double2* src = set.S + b * set.strideS;
-  for (int e = lane; e < 16 * 16; e += 64) (&prow[wave][0][0])[e] = double2{0.0, 0.0};
-  double2 a[2][16];
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const int r = lane + 64 * h, c = c0 + t;
-      a[h][t] = (r < n && c < n) ? src[r * n + c] : double2{0.0, 0.0};
-    }
-  unsigned long long used[2] = {0, 0};  // rows already used as pivots (wave-uniform)
-  const int npan = (n + 15) >> 4;
-  for (int P = 0; P < npan; ++P) {
-    const int np = min(16, n - 16 * P);
-    double2(&U)[16][128] = ubuf[P & 1];
-    if (wave == P) {
-      double2 dp = {1.0, 0.0};
-      int pj[16];
-      gj_panel2(a, np, n, lane, used, rrow, pj, dp);
-      if (lane == 0) {
-        pdet[P] = dp;
-#pragma unroll
-        for (int t = 0; t < 16; ++t)
-          if (t < np) piv[16 * P + t] = pj[t];
-      }
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        U[t][lane] = (lane == pj[t]) ? double2{a[0][t].x - 1.0, a[0][t].y} : a[0][t];
-        U[t][lane + 64] = (lane + 64 == pj[t]) ? double2{a[1][t].x - 1.0, a[1][t].y} : a[1][t];
-      }
-    }
-    __syncthreads();
-    if (wave != P) {
-      int j0 = -1, j1 = -1;  // the panel's steps whose pivots are this lane's rows
-#pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        const int p = t < np ? __builtin_amdgcn_readfirstlane(piv[16 * P + t]) : -1;
-        if (p >= 64)
-          used[1] |= 1ull << (p - 64);
-        else if (p >= 0)
-          used[0] |= 1ull << p;
-        j0 = (p == lane) ? t : j0;
-        j1 = (p == lane + 64) ? t : j1;
-      }
-      if (c0 < n) {
-        if (j0 >= 0) {
-#pragma unroll
-          for (int s = 0; s < 16; ++s) prow[wave][s][j0] = a[0][s];
-        }
-        if (j1 >= 0) {
-#pragma unroll
-          for (int s = 0; s < 16; ++s) prow[wave][s][j1] = a[1][s];
-        }
-        wave_lds_sync();
-#pragma unroll 4
-        for (int t = 0; t < 16; ++t) {
-          const double2 u0 = U[t][lane], u1 = U[t][lane + 64];
-#pragma unroll
-          for (int s = 0; s < 16; ++s) {
-            const double2 r = prow[wave][s][t];
-            a[0][s].x = fma(u0.x, r.x, fma(-u0.y, r.y, a[0][s].x));
-            a[0][s].y = fma(u0.x, r.y, fma(u0.y, r.x, a[0][s].y));
-            a[1][s].x = fma(u1.x, r.x, fma(-u1.y, r.y, a[1][s].x));
-            a[1][s].y = fma(u1.x, r.y, fma(u1.y, r.x, a[1][s].y));
-          }
-        }
-        wave_lds_sync();
-      }
-    }
-  }
-  __syncthreads();  // piv and pdet complete
-  if (tid < n) pinv[piv[tid]] = tid;
-  if (tid == 0) {
+  __syncthreads();  // piv and pdet complete, U and prow read
+  if (wave == NW - 1) {  // it has the fewest columns to store
+    const bool neg = wm::odd_permutation(piv, n, lane);
     double2 dprod = {1.0, 0.0};
     for (int q = 0; q < npan; ++q) dprod = cmul(dprod, pdet[q]);
-    const bool neg = wm::odd_permutation(piv, n);
-    set.det[b] = neg ? double2{-dprod.x, -dprod.y} : dprod;
+    if (lane == 0) set.det[b] = neg ? double2{-dprod.x, -dprod.y} : dprod;
   }
   if (!set.inv) return;
+  if (tid < n) pinv[piv[tid]] = tid;
   __syncthreads();
   double2* dst = set.inv + b * set.strideInv;
+  double2* out = H == 1 ? lds : dst;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int h = 0; h < H; ++h) {
     const int r = lane + 64 * h;
     if (r < n) {
-      const long row = (long)pinv[r] * n;
+      const long row = (long)pinv[r] * lsrc;
 #pragma unroll
-      for (int t = 0; t < 16; ++t)
-        if (c0 + t < n) dst[row + piv[c0 + t]] = a[h][t];
+      for (int t = 0; t < kPanel; ++t)
+        if (c0 + t < n) out[row + piv[c0 + t]] = a[h][t];
+    }
+  }
+  if constexpr (H == 1) {
+    __syncthreads();
+    for (int e = tid; e < n * n; e += NT) {
+      const int r = e / n;
+      dst[e] = lds[r * ld + e - r * n];
     }
   }
 }
@@ -458,9 +349,9 @@ template <int NMAX>
 __global__ __launch_bounds__(det_inv_threads(NMAX)) void gj_det_inv_kernel(DetInvSet s0, DetInvSet s1) {
   extern __shared__ double2 lds_gj[];
   if constexpr (NMAX == kLdsN)
-    gj_reg_body(blockIdx.y == 0 ? s0 : s1, blockIdx.x);
+    gj_reg_body<1>(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
   else if constexpr (NMAX == kReg2N)
-    gj_reg2_body(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
+    gj_reg_body<2>(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
   else
     gj_det_inv_body<NMAX>(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
 }
@@ -474,9 +365,9 @@ __global__ __launch_bounds__(det_inv_threads(NMAX)) void gj_det_inv_grouped_kern
   const int j = group_find(prefix, njobs, item);
   const DetInvSet set = sets[j];
   if constexpr (NMAX == kLdsN)
-    gj_reg_body(set, item - prefix[j]);
+    gj_reg_body<1>(set, item - prefix[j], lds_gj);
   else if constexpr (NMAX == kReg2N)
-    gj_reg2_body(set, item - prefix[j], lds_gj);
+    gj_reg_body<2>(set, item - prefix[j], lds_gj);
   else
     gj_det_inv_body<NMAX>(set, item - prefix[j], lds_gj);
 }
@@ -697,8 +588,8 @@ int batched_det_inv_sets(const DetInvSet* sets, int nsets, int count, hipStream_
   }
   if (count <= 0) return AFQ_OK;
   // n <= 128: the matrices stay in registers
-  return nmax <= kLdsN    ? launch_det_inv<kLdsN>(sets, nsets, count, 0, stream)
-         : nmax <= kReg2N ? launch_det_inv<kReg2N>(sets, nsets, count, kReg2Lds, stream)
+  return nmax <= kLdsN    ? launch_det_inv<kLdsN>(sets, nsets, count, reg_lds(1, nmax), stream)
+         : nmax <= kReg2N ? launch_det_inv<kReg2N>(sets, nsets, count, reg_lds(2, nmax), stream)
                           : launch_det_inv<kDetInvMaxN>(sets, nsets, count, matrix_lds_bytes(nmax), stream);
 }
 
@@ -715,8 +606,8 @@ int det_inv_grouped(const GroupTab<DetInvSet>& t, int nmax, hipStream_t stream) 
   if (t.njobs < 1 || t.total < 1) return AFQ_OK;
   if (nmax < 1 || nmax > kDetInvMaxN)
     return fail(AFQ_E_UNSUPPORTED, "det/inverse kernel supports 1 <= n <= " + std::to_string(kDetInvMaxN));
-  return nmax <= kLdsN    ? launch_det_inv_grouped<kLdsN>(t, 0, stream)
-         : nmax <= kReg2N ? launch_det_inv_grouped<kReg2N>(t, kReg2Lds, stream)
+  return nmax <= kLdsN    ? launch_det_inv_grouped<kLdsN>(t, reg_lds(1, nmax), stream)
+         : nmax <= kReg2N ? launch_det_inv_grouped<kReg2N>(t, reg_lds(2, nmax), stream)
                           : launch_det_inv_grouped<kDetInvMaxN>(t, matrix_lds_bytes(nmax), stream);
 }
 

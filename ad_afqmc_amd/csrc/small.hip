@@ -118,21 +118,21 @@ __device__ inline void overlap_matrices(const SmallJob& b, const double* T, cons
 
 // Determinant and inverse (over S) of one wave's n x n matrix, n <= NP.
 template <int NP>
-__device__ inline void invert_wave(int n, double2* S, double2* det, double2* row) {
+__device__ inline void invert_wave(int n, double2* S, double2* det) {
   const int lane = threadIdx.x & 63;
-  double2 a[NP];
+  double2 a[1][NP];
 #pragma unroll
-  for (int t = 0; t < NP; ++t) a[t] = (lane < n && t < n) ? S[lane * n + t] : double2{0.0, 0.0};
-  unsigned long long used = 0;
+  for (int t = 0; t < NP; ++t) a[0][t] = (lane < n && t < n) ? S[lane * n + t] : double2{0.0, 0.0};
+  unsigned long long used[1] = {0};
   int pj[NP];
   double2 dp = {1.0, 0.0};
-  wm::gj_panel<NP>(a, n, n, lane, used, row, pj, dp);
+  wm::gj_panel(a, n, n, lane, used, pj, dp);
   int to = 0;  // the column whose pivot is this lane's row
 #pragma unroll
   for (int t = 0; t < NP; ++t) to = (t < n && pj[t] == lane) ? t : to;
 #pragma unroll
   for (int t = 0; t < NP; ++t)
-    if (lane < n && t < n) S[to * n + pj[t]] = a[t];
+    if (lane < n && t < n) S[to * n + pj[t]] = a[0][t];
   // parity of the pivot permutation from its inversions, one row a lane
   int odd = 0;
 #pragma unroll
@@ -145,19 +145,19 @@ typedef __attribute__((address_space(3))) double2* LdsPtr;
 
 // Out of line: one copy of the unrolled sweeps, which the instruction cache
 // holds.
-__device__ __attribute__((noinline)) void invert_call(int n, LdsPtr S, LdsPtr det, LdsPtr row) {
+__device__ __attribute__((noinline)) void invert_call(int n, LdsPtr S, LdsPtr det) {
   if (n <= 8)
-    invert_wave<8>(n, (double2*)S, (double2*)det, (double2*)row);
+    invert_wave<8>(n, (double2*)S, (double2*)det);
   else if (n <= 12)
-    invert_wave<12>(n, (double2*)S, (double2*)det, (double2*)row);
+    invert_wave<12>(n, (double2*)S, (double2*)det);
   else
-    invert_wave<16>(n, (double2*)S, (double2*)det, (double2*)row);
+    invert_wave<16>(n, (double2*)S, (double2*)det);
 }
 
 // The same for S_s of every spin, wave s for spin s.
-__device__ inline void invert(const SmallJob& b, double2 (*S)[256], double2* det, double2 (*row)[16]) {
+__device__ inline void invert(const SmallJob& b, double2 (*S)[256], double2* det) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (wave < b.nspin) invert_call(b.occ[wave], (LdsPtr)S[wave], (LdsPtr)(det + wave), (LdsPtr)row[wave]);
+  if (wave < b.nspin) invert_call(b.occ[wave], (LdsPtr)S[wave], (LdsPtr)(det + wave));
 }
 
 // G_s = (W_s S_s^-1)^T (occ_s x N) of every spin, one after another
@@ -215,7 +215,7 @@ template <int NT, int TR, int TPT, bool RES>
 __global__ __launch_bounds__(NT) void small_step_kernel(SmallStep p) {
   extern __shared__ double2 sm[];
   __shared__ double2 S[2][256];
-  __shared__ double2 det[2], red[NT / 64], row[2][16];
+  __shared__ double2 det[2], red[NT / 64];
   const SmallJob& b = p.b;
   const int tid = threadIdx.x;
   const int N = b.N, c = b.c, G = b.G;
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(NT) void small_step_kernel(SmallStep p) {
   __syncthreads();
   overlap_matrices<NT>(b, T, P, S);
   __syncthreads();
-  invert(b, S, det, row);
+  invert(b, S, det);
   __syncthreads();
 
   const Tiles<NT, TR, TPT> tl(N, c);
@@ -434,7 +434,7 @@ __global__ __launch_bounds__(NT) void small_step_kernel(SmallStep p) {
     Q = nxt;
     overlap_matrices<NT>(b, T, P, S);
     __syncthreads();
-    invert(b, S, det, row);
+    invert(b, S, det);
     __syncthreads();
     const double2 on = cmul(det[0], det[b.nspin - 1]);
     if (tid == NT - 1) {
@@ -554,7 +554,7 @@ __global__ __launch_bounds__(kMeasureThreads) void small_measure_kernel(SmallMea
   extern __shared__ double2 sm[];
   constexpr int NT = kMeasureThreads;
   __shared__ double2 S[2][256];
-  __shared__ double2 det[2], red[NT / 64], row[2][16];
+  __shared__ double2 det[2], red[NT / 64];
   const SmallJob& b = p.b;
   const int tid = threadIdx.x;
   const int N = b.N;
@@ -572,7 +572,7 @@ __global__ __launch_bounds__(kMeasureThreads) void small_measure_kernel(SmallMea
   }
   overlap_matrices<NT>(b, T, X, S);
   __syncthreads();
-  invert(b, S, det, row);
+  invert(b, S, det);
   __syncthreads();
   if (tid == 0) {
     for (int s = 0; s < b.nspin; ++s) b.det[s][w] = det[s];

@@ -83,70 +83,89 @@ __device__ inline void wave_lds_sync() {
 }
 
 // Gauss-Jordan steps of one wave on the np <= NP columns a[] of a panel, lane i
-// holding row i of n.  Rows are never swapped: the pivot of column t is the
-// first (lowest) not yet used row of maximal |re| + |im| (pj[t], -1 past np;
-// `used` marks the rows taken), and column t is replaced by the unit vector of
-// its pivot row, so one branch-free update leaves a_p / d in the pivot row and
-// a - (f / d) a_p elsewhere.  dp collects the product of the pivots; rrow is
-// an NP-element LDS row of the wave.
-template <int NP>
-__device__ __forceinline__ void gj_panel(double2 (&a)[NP], int np, int n, int lane, unsigned long long& used,
-                                         double2* rrow, int (&pj)[NP], double2& dp) {
+// holding the rows i + 64 h of n.  Rows are never swapped: the pivot of column t
+// is the first (lowest) not yet used row of maximal |re| + |im| (pj[t], -1 past
+// np; `used` marks the rows taken), and column t is replaced by the unit vector
+// of its pivot row, so one branch-free update leaves a_p / d in the pivot row
+// and a - (f / d) a_p elsewhere.  dp collects the product of the pivots.  The
+// pivot row reaches the lanes through scalar registers: it is one of H, and a
+// round trip through LDS costs more (H = 2, n = 100: 256 us, 210 without).
+template <int H, int NP>
+__device__ __forceinline__ void gj_panel(double2 (&a)[H][NP], int np, int n, int lane, unsigned long long (&used)[H],
+                                         int (&pj)[NP], double2& dp) {
+  static_assert(H == 1 || H == 2, "one or two rows a lane");
 #pragma unroll
   for (int t = 0; t < NP; ++t) {
     pj[t] = -1;
     if (t < np) {
-      const double2 x = a[t];
-      const bool cand = lane < n && !((used >> lane) & 1ull);
-      const double v = cand ? fabs(x.x) + fabs(x.y) : -1.0;
-      const double m = wave_fmax(v);
+      double2 x[H];
+      bool cand[H];
+      double v[H];
+#pragma unroll
+      for (int h = 0; h < H; ++h) {
+        x[h] = a[h][t];
+        cand[h] = lane + 64 * h < n && !((used[h] >> lane) & 1ull);
+        v[h] = cand[h] ? fabs(x[h].x) + fabs(x[h].y) : -1.0;
+      }
+      const double m = wave_fmax(H == 1 ? v[0] : fmax(v[0], v[H - 1]));
       // lowest row of maximal measure (a column of NaNs falls back to the
       // lowest unused row, so p is always a valid row)
-      const unsigned long long best = __ballot(cand && v == m), open = __ballot(cand);
-      const int p = __builtin_ctzll(best ? best : open);
-      pj[t] = p;
-      const double2 d = {readlane_d(x.x, p), readlane_d(x.y, p)};
+      unsigned long long best[H], any = 0;
+#pragma unroll
+      for (int h = 0; h < H; ++h) {
+        best[h] = __ballot(cand[h] && v[h] == m);
+        any |= best[h];
+      }
+#pragma unroll
+      for (int h = 0; h < H; ++h)
+        if (!any) best[h] = __ballot(cand[h]);
+      const bool hi = H > 1 && best[0] == 0;
+      const int p = __builtin_ctzll(hi ? best[H - 1] : best[0]);
+      pj[t] = hi ? 64 + p : p;
+      const double2 xp = {hi ? x[H - 1].x : x[0].x, hi ? x[H - 1].y : x[0].y};
+      const double2 d = {readlane_d(xp.x, p), readlane_d(xp.y, p)};
       dp = cmul(dp, d);
-      used |= 1ull << p;
       // column t becomes the unit vector of row p: the common update
       // below then leaves 1 / d in row p and -f / d in the others
-      const bool isp = lane == p;
-      a[t] = isp ? double2{1.0, 0.0} : double2{0.0, 0.0};
-      if (isp) {
-#pragma unroll
-        for (int s = 0; s < NP; ++s) rrow[s] = a[s];
-      }
       const double2 dinv = crecip_fast(d);
-      const double sc = isp ? 0.0 : 1.0;
-      const double2 fd = cmul(x, dinv);
-      const double2 g = isp ? dinv : double2{-fd.x, -fd.y};
-      wave_lds_sync();
-      double2 r[NP];
+      double2 g[H];
+      double sc[H];
 #pragma unroll
-      for (int s = 0; s < NP; ++s) r[s] = rrow[s];
+      for (int h = 0; h < H; ++h) {
+        const bool isp = lane == p && hi == (h == 1);
+        used[h] |= hi == (h == 1) ? 1ull << p : 0ull;
+        a[h][t] = isp ? double2{1.0, 0.0} : double2{0.0, 0.0};
+        sc[h] = isp ? 0.0 : 1.0;
+        const double2 fd = cmul(x[h], dinv);
+        g[h] = isp ? dinv : double2{-fd.x, -fd.y};
+      }
 #pragma unroll
       for (int s = 0; s < NP; ++s) {
-        const double2 y = a[s];
-        a[s].x = fma(g.x, r[s].x, fma(-g.y, r[s].y, sc * y.x));
-        a[s].y = fma(g.x, r[s].y, fma(g.y, r[s].x, sc * y.y));
+        const double2 z = {hi ? a[H - 1][s].x : a[0][s].x, hi ? a[H - 1][s].y : a[0][s].y};
+        const double2 r = {readlane_d(z.x, p), readlane_d(z.y, p)};
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+          const double2 y = a[h][s];
+          a[h][s].x = fma(g[h].x, r.x, fma(-g[h].y, r.y, sc[h] * y.x));
+          a[h][s].y = fma(g[h].x, r.y, fma(g[h].y, r.x, sc[h] * y.y));
+        }
       }
-      wave_lds_sync();
     }
   }
 }
 
-// sign of the permutation piv of n <= 128 as true for odd: n minus its number of
-// cycles transpositions
-__device__ inline bool odd_permutation(const int* piv, int n) {
-  unsigned long long s0 = 0, s1 = 0;
-  auto seen = [&](int q) { return (((q < 64 ? s0 : s1) >> (q & 63)) & 1ull) != 0; };
-  int cycles = 0;
-  for (int s = 0; s < n; ++s) {
-    if (seen(s)) continue;
-    ++cycles;
-    for (int q = s; !seen(q); q = piv[q]) (q < 64 ? s0 : s1) |= 1ull << (q & 63);
+// sign of the permutation piv of n <= 128 (in LDS) as true for odd, by one wave:
+// the parity of its inversions
+__device__ inline bool odd_permutation(const int* piv, int n, int lane) {
+  int odd = 0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int i = lane + 64 * h;
+    const int pi = i < n ? piv[i] : -1;
+#pragma unroll 8
+    for (int m = 1; m < n; ++m) odd += m > i && piv[m] < pi;
   }
-  return ((n - cycles) & 1) != 0;
+  return __popcll(__ballot(odd & 1)) & 1;
 }
 
 // Phaseless factor |I| cos(theta) (propagation.py:306-320), not clipped, of a
