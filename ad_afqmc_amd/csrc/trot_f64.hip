@@ -19,12 +19,13 @@
 // so the SIMDs differ by one block at most (N = 200: 17 of 16.25 blocks, where
 // whole row blocks would leave 20).
 //
-// Bound: the FP64 matrix cores, 8 N^2 c flops a term, and the loads of the VHS
-// blocks below the diagonal, whose lanes step by rows (fetching two to four
-// steps ahead instead of one made N = 100 slower, 143 -> 177 us).  Measured
+// Bound: the FP64 matrix cores, 8 N^2 c flops a term, and at N = 100 the reads of
+// the VHS, once a term and slab (fetching two to four steps ahead instead of one
+// was slower there, 143 -> 177 us).  Measured
 // against one launch a product with the running sum in memory, per step: N = 200,
 // 40 columns, 512 walkers 1.30 -> 0.82 ms (48 TFLOP/s); N = 300, 60 + 58 columns,
 // 256 walkers 3.25 -> 2.58 ms; N = 100, 20 columns, 256 walkers 181 -> 143 us.
+// With the VHS read in the order of the fragments: 0.79 and 2.43 ms, 87 us.
 #include "trot_f64.h"
 
 #include <cmath>
@@ -277,9 +278,11 @@ int trot_f64(const TrotF64& f, hipStream_t st) {
   a.f = f;
   a.R = blocks_of(f.N);
   const int MB = std::max(1, main_blocks(a.R));
-  // column blocks a slab: the least time of the work-groups' rounds over 256
-  // CUs, two a CU where LDS and registers hold two; more of them read the VHS
-  // less often
+  // Column blocks a slab: the least work of the busiest CU's work-groups, however
+  // many of them share it; at equal work the larger slab, which reads the VHS
+  // less often (N=100, 20 columns, 256 walkers: 3 blocks 87 us, 1 block 93, 2
+  // blocks, which would fill two work-groups a CU, 101; N=150, 50 + 48 columns, 64
+  // walkers: 4 blocks 192, 2 blocks 188).
   int NB = 0;
   double best = 0.0;
   for (int nb = 1; nb <= 5; ++nb) {
@@ -287,10 +290,8 @@ int trot_f64(const TrotF64& f, hipStream_t st) {
     if (!held(MB, nb) || lds > kLdsMax) continue;
     long S = 0;
     for (int s = 0; s < f.nspin; ++s) S += ((f.c[s] + 7) / 8 + nb - 1) / nb;
-    const int per = MB * nb <= 5 && 2 * lds <= 160 * 1024 ? 2 : 1;
-    const double rounds = std::ceil((double)(S * f.W) / (256.0 * per));
-    const double t = rounds * per * simd_blocks(a.R, nb);
-    if (NB == 0 || t <= best * 1.0001) {
+    const double t = std::ceil((double)(S * f.W) / 256.0) * simd_blocks(a.R, nb);
+    if (NB == 0 || t <= best) {
       NB = nb;
       best = t;
     }
