@@ -850,8 +850,17 @@ int dispatch_shape(const Gemm& g, hipStream_t s) {
   }
   // both spins' columns of unrestricted walkers (65..128 columns)
   if (g.M > 64 && g.N <= 128 && g.batch > 1) {
-    if constexpr (BF) return launch<BF, AC, BC, AT, BT, TA, TB, TCo, 4, 4, 1, 2>(g, s);
-    return launch<BF, AC, BC, AT, BT, TA, TB, TCo, 4, 4, 1, 1>(g, s);
+    if constexpr (BF) {
+      return launch<BF, AC, BC, AT, BT, TA, TB, TCo, 4, 4, 1, 2>(g, s);
+    } else {
+      // the tile with less padding, the wider-spread one only where it pays: at
+      // N=141, 67 columns, 150 walkers 48 x 80 tiles fill 0.82 of their blocks and
+      // 64 x 64 ones 0.38 (64 -> 37 us a term)
+      const long a = (long)((g.M + 63) / 64 * 64) * ((g.N + 63) / 64 * 64);
+      const long b = (long)((g.M + 47) / 48 * 48) * ((g.N + 79) / 80 * 80);
+      return 10 * b <= 8 * a ? launch<BF, AC, BC, AT, BT, TA, TB, TCo, 3, 5, 1, 1>(g, s)
+                             : launch<BF, AC, BC, AT, BT, TA, TB, TCo, 4, 4, 1, 1>(g, s);
+    }
   }
   if (g.N <= 48) return launch<BF, AC, BC, AT, BT, TA, TB, TCo, 4, 1, 1, 3>(g, s);
   if (g.N <= 64 && g.M > 64) return launch<BF, AC, BC, AT, BT, TA, TB, TCo, 4, 1, 1, 4>(g, s);
