@@ -495,13 +495,17 @@ void carve(Arena& ar, Buffers& b, const afq_job* j, const Spins& sp, int nb, int
   b.scal = ar.take<double>(4);
   b.Lbar = ar.take<double>(G * NN);
   b.rh1barC = ar.take<double2>(sp.pt);
-  // Exchange-adjoint chunks: F and its permuted copy at most 256 MB each.  At 2 GB
-  // they were most of the arena, and taking and giving back so much memory on
-  // each call held a gradient up by up to 25 ms (N=100, O=20, G=500, 256 walkers:
-  // 14.6 to 40 ms a call at 2 GB, 14.7 at 256 MB, 15.1 at 128 MB).
+  // Exchange-adjoint chunks: F and its permuted copy at most 256 MB each, or what
+  // 1024 rows (walker, orbital) of them take, up to 2 GB.  At 2 GB they were most
+  // of the arena, and taking and giving back so much memory on each call held a
+  // gradient up by up to 25 ms (N=100, O=20, G=500, 256 walkers: 14.6 to 40 ms a
+  // call at 2 GB, 14.7 at 256 MB, 15.1 at 128 MB); with few rows the products are
+  // short of work-groups (N=300, O=60, G=2000, 256 walkers, 2 steps: 411 ms in
+  // chunks of 2 walkers, 320 in chunks of 18).
   const long omax = std::max(sp.O[0], sp.O[1]);
   const long per_w = G * omax * omax * (long)sizeof(double2);
-  b.Wc = (int)std::max(1L, std::min(W, (256L << 20) / std::max(1L, per_w)));
+  const long room = std::min(2048L << 20, std::max(256L << 20, (1024 + omax - 1) / omax * per_w));
+  b.Wc = (int)std::max(1L, std::min(W, room / std::max(1L, per_w)));
   b.Wc = (int)((W + (W + b.Wc - 1) / b.Wc - 1) / ((W + b.Wc - 1) / b.Wc));  // of about equal size
   b.F = ar.take<double2>(G * omax * b.Wc * omax);
   b.Fp = ar.take<double2>(G * omax * b.Wc * omax);
