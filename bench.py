@@ -101,10 +101,11 @@ def vhs_columns(chol, N):
     return npk if dmax <= 1e-12 * amax else N * N
 
 
-def launch_flops(cls, N, Oa, Ob, G, W, unrestricted=False, vhs_cols=None):
+def launch_flops(cls, N, Oa, Ob, G, W, unrestricted=False, vhs_cols=None, exchange_virtual=False):
     """Flops of one launch of a kernel class, as the kernel computes them,
     averaged over the launches of a block: the VHS product covers `vhs_cols`
-    columns (N^2 by default); a Taylor launch covers the walker panel (both
+    columns (N^2 by default); the FP64 exchange (`exchange_virtual`) contracts
+    over the N - O orbitals that the trial leaves empty; a Taylor launch covers the walker panel (both
     spins' columns side by side for unrestricted walkers); the one-body,
     exchange, force-bias, Green's-function and overlap launches alternate
     between the spins of an unrestricted or UHF case."""
@@ -117,7 +118,7 @@ def launch_flops(cls, N, Oa, Ob, G, W, unrestricted=False, vhs_cols=None):
     if cls == "exp_h1":
         return mean(lambda o: 4.0 * N * N * o * W) if unrestricted else 4.0 * N * N * Oa * W
     if cls == "exchange":
-        return mean(lambda o: 4.0 * G * o * o * N * W)
+        return mean(lambda o: 4.0 * G * o * o * (N - o if exchange_virtual else N) * W)
     if cls == "force_bias":
         return mean(lambda o: 4.0 * G * o * N * W)
     if cls == "green":
@@ -513,7 +514,8 @@ def time_config(system, name, precision, steps, warmup, dominant_roofline=False,
         dom_ms, dom_n = job.profile_read(dominant)
         job.profile(dominant, False)
         per_launch = launch_flops(dominant, N, Oa, Ob, G, W, unrestricted=uhf,
-                                  vhs_cols=vhs_columns(system.chol, N) if dominant == "vhs" else None)
+                                  vhs_cols=vhs_columns(system.chol, N) if dominant == "vhs" else None,
+                                  exchange_virtual=precision == "fp64")
         avg_s = dom_ms / max(dom_n, 1) / 1e3
         # bf16x3 does three bf16 MFMA products per FP32-equivalent product: its
         # ceiling is a third of the dense bf16 peak
