@@ -54,7 +54,7 @@ struct WgArgs {
   long T8;
   double* out;
   double scale;
-  int N, R;                   // VHS epilogue
+  int R;                      // VHS epilogue
 };
 
 // AK: A row m holds its K elements contiguously (lda = row stride); else A row
@@ -366,7 +366,6 @@ long vhs_f64_elems(int N) {
 int vhs_f64(const double2* xs, const double* lp, int N, int G, int W, double sqdt, double2* out, hipStream_t st) {
   WgArgs p{};
   p.R = (N + 15) / 16;
-  p.N = N;
   p.M = p.R * (p.R + 1) / 2 * 256;
   p.A[0] = lp;
   p.lda[0] = p.M;
