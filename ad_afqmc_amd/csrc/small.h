@@ -30,8 +30,8 @@ struct SmallStep {
   const double2* mf;
   const double* fields;   // (nsteps, W, G)
   const double2* h0p;
-  const double* scalars;  // e_estimate
-  double* h;              // (nsteps, W): the phaseless factor at the shift e_estimate, not clipped
+  const double* scalars;  // the shift that the steps start with
+  double* h;              // (nsteps, W): the phaseless factor at that shift, not clipped
   double2* overlaps;      // in: of the incoming walkers; out: of the new ones
   // of the last step
   double2 *fb, *xs, *terms, *ov_new;

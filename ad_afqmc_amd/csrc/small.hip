@@ -438,8 +438,7 @@ __global__ __launch_bounds__(NT) void small_step_kernel(SmallStep p) {
     __syncthreads();
     const double2 on = cmul(det[0], det[b.nspin - 1]);
     if (tid == NT - 1) {
-      const double e_est = p.scalars[0];
-      p.h[(long)step * b.W + w] = factor_call(on, oo, sh, ft, e_est, *p.h0p, p.dt);
+      p.h[(long)step * b.W + w] = factor_call(on, oo, sh, ft, p.scalars[1], *p.h0p, p.dt);
       if (last) {
         p.overlaps[w] = on;
         p.terms[2 * w] = sh;
@@ -452,16 +451,20 @@ __global__ __launch_bounds__(NT) void small_step_kernel(SmallStep p) {
   store_panel<NT>(b, w, P);
 }
 
-// The weights through nsteps steps: factor h exp(dt (shift - e_estimate)),
-// clipped (propagation.py:320-334), the shift following from each step's sum.
+// The weights through nsteps steps: factor h exp(dt (shift - shift at the first
+// step)), clipped (propagation.py:320-334), the shift following from each step's
+// sum.  The factors are taken at the first step's shift and not at e_estimate,
+// so that a step's weights do not depend on e_estimate (which may be far from
+// the shift, or not finite) and a single step needs no rescaling.
 __global__ __launch_bounds__(1024) void small_weights_kernel(const double* __restrict__ h, int nsteps, int W, double dt,
                                                              double* __restrict__ weights,
                                                              double* __restrict__ scalars) {
   __shared__ double red[2][16];
   const double e_est = scalars[0];
-  double pcs = scalars[1];
+  const double first = scalars[1];
+  double pcs = first;
   for (int s = 0; s < nsteps; ++s) {
-    const double f = exp(dt * (pcs - e_est));
+    const double f = exp(dt * (pcs - first));
     double sum = 0.0;
     for (int w = threadIdx.x; w < W; w += 1024) {
       const double wn = wm::clipped_weight(f * h[(long)s * W + w], weights[w]);
