@@ -22,6 +22,14 @@ int fail(int code, const std::string& m) {
   g_err = m;
   return code;
 }
+
+int raise_lds(const void* kernel, size_t bytes, std::atomic<bool>& done, const char* what) {
+  if (done.load(std::memory_order_acquire)) return AFQ_OK;
+  const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  if (e != hipSuccess) return fail(AFQ_E_HIP, std::string(what) + " LDS attribute: " + hipGetErrorString(e));
+  done.store(true, std::memory_order_release);
+  return AFQ_OK;
+}
 }  // namespace afq
 
 using namespace afq;

@@ -53,6 +53,11 @@ constexpr int kPairs = 4 * kSteps;    // its k pairs
 
 // Register budget: three waves a SIMD where the accumulators leave room.
 constexpr int waves_per_simd(int mb, int nb, int waves) { return waves == 4 && mb * nb <= 10 ? 3 : 2; }
+// LDS bytes for the passes of d: as many work-groups a CU as the registers allow.
+constexpr size_t tile_room(int mb, int nb, int waves) {
+  const int per_cu = waves_per_simd(mb, nb, waves) * 4 / waves;
+  return (per_cu == 3 ? 46 : per_cu == 2 ? 74 : 148) * 1024;
+}
 
 template <int MB, int NB, int WR, int WC>
 __global__ __launch_bounds__(64 * WR * WC, (waves_per_simd(MB, NB, WR * WC))) void exchange_f64_kernel(ExF64 p) {
@@ -461,14 +466,11 @@ int mm(hipStream_t st, int M, int N, int K, const double* A, long lda, bool at, 
 
 template <int MB, int NB, int WR, int WC>
 int launch(const ExF64& p, long grid, hipStream_t st) {
-  const size_t stage = sizeof(double2) * 2 * kPairs * 16 * NB * WC;
-  const size_t tile = sizeof(double) * p.lds_elems;
-  const size_t bytes = std::max(stage, tile);
-  if (bytes > 48 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(exchange_f64_kernel<MB, NB, WR, WC>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e != hipSuccess) return fail(AFQ_E_HIP, std::string("exchange LDS attribute: ") + hipGetErrorString(e));
-  }
+  constexpr size_t stage = sizeof(double2) * 2 * kPairs * 16 * NB * WC;
+  const size_t bytes = std::max(stage, sizeof(double) * p.lds_elems);
+  static std::atomic<bool> raised{false};
+  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(exchange_f64_kernel<MB, NB, WR, WC>),
+                    std::max(stage, tile_room(MB, NB, WR * WC)), raised, "exchange"));
   hipLaunchKernelGGL((exchange_f64_kernel<MB, NB, WR, WC>), dim3((unsigned)grid), dim3(64 * WR * WC), bytes, st, p);
   return launch_status("exchange_f64_kernel");
 }
@@ -559,10 +561,10 @@ int exchange_f64_set_trial(const double* mo, int N, int O, double* Q, double* P,
   double* inv = gram + OO;
   if (Nv > 0) {
     const size_t bytes = sizeof(double) * N * O;
-    if (bytes <= 152 * 1024) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(householder_kernel<true>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-      if (e != hipSuccess) return fail(AFQ_E_HIP, std::string("householder LDS attribute: ") + hipGetErrorString(e));
+    constexpr size_t most = 152 * 1024;
+    if (bytes <= most) {
+      static std::atomic<bool> raised{false};
+      AFQ_TRY(raise_lds(reinterpret_cast<const void*>(householder_kernel<true>), most, raised, "householder"));
       hipLaunchKernelGGL(householder_kernel<true>, dim3(1), dim3(1024), bytes, st, mo, N, O, V, tau);
     } else {
       hipLaunchKernelGGL(householder_kernel<false>, dim3(1), dim3(1024), 0, st, mo, N, O, V, tau);
@@ -660,10 +662,8 @@ int k_exchange_f64(const double* a, const double* Q, const double* c0, const dou
   p.nchunk = exchange_f64_nchunk(O, G);
   p.coul = coul;
   p.kpart = kpart;
-  // LDS of the d passes: as many work-groups a CU as the registers allow
   const long ld = 16L * t.NB * t.WC + 2;
-  const int waves = t.WR * t.WC, per_cu = waves_per_simd(t.MB, t.NB, waves) * 4 / waves;
-  const long room = (per_cu == 3 ? 46 : per_cu == 2 ? 74 : 148) * 1024L / (long)sizeof(double);
+  const long room = (long)(tile_room(t.MB, t.NB, t.WR * t.WC) / sizeof(double));
   p.gp = (int)std::min((long)t.gw, room / (O * ld));
   p.strip = O;
   if (p.gp == 0) {  // one g in strips: strip rows, and the strip's columns of all rows

@@ -525,15 +525,8 @@ __global__ __launch_bounds__(256) void cholesky_grouped_kernel(const CholSet* __
   cholesky_upper_body<NMAX>(c.S, c.strideS, c.n, c.R, c.strideR, item - prefix[j], lds_ch);
 }
 
-// Raises a kernel's dynamic LDS limit to 96 KB (once per kernel).
-int raise_lds(const void* kernel, bool* done, const char* what) {
-  if (*done) return AFQ_OK;
-  hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-  if (e != hipSuccess) return fail(AFQ_E_HIP, std::string(what) + " LDS attribute: " + hipGetErrorString(e));
-  *done = true;
-  return AFQ_OK;
-}
-
+// Dynamic LDS of the largest of these kernels' launches (64 x 65 entries), and room
+constexpr size_t kLdsMax = 96 * 1024;
 
 // Grouped copies / conjugate copies: work-group i covers elements
 // [(i - prefix[j]) * 1024, +1024) of job j's vector.
@@ -572,8 +565,8 @@ static int check_det_inv_set(const DetInvSet& s) {
 
 template <int NMAX>
 static int launch_det_inv(const DetInvSet* sets, int nsets, int count, size_t lds, hipStream_t stream) {
-  static bool raised = false;
-  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(gj_det_inv_kernel<NMAX>), &raised, "det/inverse"));
+  static std::atomic<bool> raised{false};
+  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(gj_det_inv_kernel<NMAX>), kLdsMax, raised, "det/inverse"));
   hipLaunchKernelGGL(gj_det_inv_kernel<NMAX>, dim3(count, nsets), dim3(det_inv_threads(NMAX)), lds, stream, sets[0],
                      sets[nsets > 1 ? 1 : 0]);
   return launch_status("gj_det_inv_kernel");
@@ -595,8 +588,8 @@ int batched_det_inv_sets(const DetInvSet* sets, int nsets, int count, hipStream_
 
 template <int NMAX>
 static int launch_det_inv_grouped(const GroupTab<DetInvSet>& t, size_t lds, hipStream_t stream) {
-  static bool raised = false;
-  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(gj_det_inv_grouped_kernel<NMAX>), &raised, "det/inverse"));
+  static std::atomic<bool> raised{false};
+  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(gj_det_inv_grouped_kernel<NMAX>), kLdsMax, raised, "det/inverse"));
   hipLaunchKernelGGL(gj_det_inv_grouped_kernel<NMAX>, dim3((unsigned)t.total), dim3(det_inv_threads(NMAX)), lds, stream, t.params,
                      t.prefix, t.njobs);
   return launch_status("gj_det_inv_grouped_kernel");
@@ -619,8 +612,8 @@ int batched_det_inv(const double2* S, long strideS, int n, int count, double2* d
 
 template <int NMAX>
 static int launch_cholesky(const CholSet* sets, int nsets, int count, size_t lds, hipStream_t stream) {
-  static bool raised = false;
-  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(cholesky_upper_kernel<NMAX>), &raised, "Cholesky"));
+  static std::atomic<bool> raised{false};
+  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(cholesky_upper_kernel<NMAX>), kLdsMax, raised, "Cholesky"));
   hipLaunchKernelGGL(cholesky_upper_kernel<NMAX>, dim3(count, nsets), dim3(256), lds, stream, sets[0],
                      sets[nsets > 1 ? 1 : 0]);
   return launch_status("cholesky_upper_kernel");
@@ -648,8 +641,8 @@ int batched_cholesky_upper(const double2* S, long strideS, int n, int count, dou
 
 template <int NMAX>
 static int launch_cholesky_grouped(const GroupTab<CholSet>& t, size_t lds, hipStream_t stream) {
-  static bool raised = false;
-  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(cholesky_grouped_kernel<NMAX>), &raised, "Cholesky"));
+  static std::atomic<bool> raised{false};
+  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(cholesky_grouped_kernel<NMAX>), kLdsMax, raised, "Cholesky"));
   hipLaunchKernelGGL(cholesky_grouped_kernel<NMAX>, dim3((unsigned)t.total), dim3(256), lds, stream, t.params,
                      t.prefix, t.njobs);
   return launch_status("cholesky_grouped_kernel");

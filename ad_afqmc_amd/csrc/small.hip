@@ -721,20 +721,17 @@ __global__ void pack_rc_kernel(const double* __restrict__ rc0, int n0, const dou
   out[t] = double2{at(e), at(e + 1)};
 }
 
-template <typename K>
-int raise(K kernel, size_t bytes) {
-  if (bytes <= 32 * 1024) return AFQ_OK;
-  const hipError_t e =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  if (e != hipSuccess) return fail(AFQ_E_HIP, std::string("small kernel LDS attribute: ") + hipGetErrorString(e));
-  return AFQ_OK;
-}
+// Dynamic LDS at most: of a step that streams L and rot_chol, of one that holds
+// them (two work-groups a CU), and of a measurement.
+constexpr size_t kStepLds = 144 * 1024, kResidentLds = 72 * 1024, kMeasureLds = 96 * 1024;
 
 int osum_of(const SmallJob& b) { return b.occ[0] + (b.nspin > 1 ? b.occ[1] : 0); }
 
 template <int NT, int TR, int TPT, bool RES>
 int launch_step(const SmallStep& p, size_t bytes, hipStream_t st) {
-  AFQ_TRY(raise(small_step_kernel<NT, TR, TPT, RES>, bytes));
+  static std::atomic<bool> raised{false};
+  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(small_step_kernel<NT, TR, TPT, RES>),
+                    RES ? kResidentLds : kStepLds, raised, "small step"));
   hipLaunchKernelGGL((small_step_kernel<NT, TR, TPT, RES>), dim3(p.b.W), dim3(NT), bytes, st, p);
   return launch_status("small_step_kernel");
 }
@@ -745,7 +742,7 @@ size_t small_step_lds(int N, int G, int c, int osum, int nbuf) {
   if (N > kSmallMaxN || G > 2048) return 0;
   const Regions r = regions(N, c, osum, nbuf);
   const size_t bytes = sizeof(double2) * (2 * r.panel + r.v + r.e + r.t + G);
-  return bytes <= 144 * 1024 ? bytes : 0;
+  return bytes <= kStepLds ? bytes : 0;
 }
 
 // A thread then forms at most some 400 products of the exchange, fewer than the
@@ -762,7 +759,7 @@ bool small_energy_whole(int N, int G, int occ0, int occ1) {
 // N = 100, O = 20, 50 walkers).
 size_t small_measure_lds(int N, int c, int osum) {
   const size_t bytes = sizeof(double2) * (size_t)N * (c + osum) + sizeof(double) * (size_t)N * osum;
-  return N * osum <= 1536 && bytes <= 96 * 1024 ? bytes : 0;
+  return N * osum <= 1536 && bytes <= kMeasureLds ? bytes : 0;
 }
 
 long small_l_pairs(int N, bool sym) { return (vhs_entries(N, sym) + 1) / 2; }
@@ -798,10 +795,10 @@ int k_small_step(const SmallStep& p, hipStream_t st) {
   if (bytes == 0) return fail(AFQ_E_UNSUPPORTED, "small step: sizes past the limits");
   const size_t res = bytes + sizeof(double2) * (size_t)b.G * (small_l_pairs(b.N, p.sym) + small_rc_pairs(b.N, osum));
   if (b.N * b.c <= 256) {
-    if (res <= 72 * 1024) return launch_step<256, 1, 1, true>(p, res, st);
+    if (res <= kResidentLds) return launch_step<256, 1, 1, true>(p, res, st);
     return launch_step<256, 1, 1, false>(p, bytes, st);
   }
-  if (res <= 72 * 1024) return launch_step<512, 1, 3, true>(p, res, st);
+  if (res <= kResidentLds) return launch_step<512, 1, 3, true>(p, res, st);
   return launch_step<512, 2, 1, false>(p, bytes, st);
 }
 
@@ -813,7 +810,8 @@ int k_small_weights(const double* h, int nsteps, int W, double dt, double* weigh
 int k_small_measure(const SmallMeasure& p, hipStream_t st) {
   const size_t bytes = small_measure_lds(p.b.N, p.b.c, osum_of(p.b));
   if (bytes == 0) return fail(AFQ_E_UNSUPPORTED, "small measurement: sizes past the limits");
-  AFQ_TRY(raise(small_measure_kernel, bytes));
+  static std::atomic<bool> raised{false};
+  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(small_measure_kernel), kMeasureLds, raised, "small measurement"));
   hipLaunchKernelGGL(small_measure_kernel, dim3(p.b.W), dim3(kMeasureThreads), bytes, st, p);
   return launch_status("small_measure_kernel");
 }

@@ -252,9 +252,8 @@ int simd_blocks(int R, int NB) {
 
 template <int MB, int NB, int XB>
 int launch(const TrotArgs& a, long grid, size_t bytes, hipStream_t st) {
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(trot_f64_kernel<MB, NB, XB>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  if (e != hipSuccess) return fail(AFQ_E_HIP, std::string("propagator LDS attribute: ") + hipGetErrorString(e));
+  static std::atomic<bool> raised{false};
+  AFQ_TRY(raise_lds(reinterpret_cast<const void*>(trot_f64_kernel<MB, NB, XB>), kLdsMax, raised, "propagator"));
   hipLaunchKernelGGL((trot_f64_kernel<MB, NB, XB>), dim3((unsigned)grid), dim3(NT), bytes, st, a);
   return launch_status("trot_f64_kernel");
 }
