@@ -283,9 +283,12 @@ bool x_f64(const afq_job* j, int s) {
 
 // Rebuilds the parts of that exchange that follow from the trial, and from
 // rot_chol once there is one.
-int x_f64_trial(afq_job* j, int s, hipStream_t st) {
-  return exchange_f64_set_trial(j->mo[s], j->N, j->nocc[s], j->xq_q[s], j->xq_p[s], j->xq_tmp, j->gemm_ws,
-                                j->gemm_ws_elems, st);
+int x_f64_trial(afq_job* j, hipStream_t st) {
+  ExTrial sets[2];
+  int n = 0;
+  for (int s = 0; s < (j->rhf ? 1 : 2); ++s)
+    if (x_f64(j, s)) sets[n++] = ExTrial{j->mo[s], j->nocc[s], j->xq_q[s], j->xq_p[s]};
+  return exchange_f64_set_trial(sets, n, j->N, j->xq_tmp, st);
 }
 int x_f64_chol(afq_job* j, int s, hipStream_t st) {
   return exchange_f64_set_chol(j->rot_chol[s], j->xq_q[s], j->xq_p[s], j->N, j->nocc[s], j->G, j->xq_a[s],
@@ -1314,11 +1317,9 @@ int afq_job_set_trial(afq_job_t j, const double* mo_up, const double* mo_dn, con
   if (!j->rhf)
     AFQ_HIP(hipMemcpyAsync(j->mo[1], mo_dn, sizeof(double) * N * j->nocc[1], hipMemcpyDefault, S(stream)));
   AFQ_HIP(hipMemcpyAsync(j->rdm1, rdm1, sizeof(double) * 2 * N * N, hipMemcpyDefault, S(stream)));
+  AFQ_TRY(x_f64_trial(j, S(stream)));
   for (int s = 0; s < (j->rhf ? 1 : 2); ++s)
-    if (x_f64(j, s)) {
-      AFQ_TRY(x_f64_trial(j, s, S(stream)));
-      if (j->rc_set[s]) AFQ_TRY(x_f64_chol(j, s, S(stream)));
-    }
+    if (x_f64(j, s) && j->rc_set[s]) AFQ_TRY(x_f64_chol(j, s, S(stream)));
   j->have_trial = true;
   j->have_meas = j->have_prop = false;
   return AFQ_OK;

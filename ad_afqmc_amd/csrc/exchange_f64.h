@@ -28,9 +28,15 @@ struct ExF64 {
 long exchange_f64_a_elems(int O, int N, int G);
 long exchange_f64_b_elems(int O, int N, int W);
 long exchange_f64_tmp_elems(int O, int N, int G);
-// Q (N, N - O): orthonormal complement of span(mo); P (N, O) = mo (mo^T mo)^-1.
-int exchange_f64_set_trial(const double* mo, int N, int O, double* Q, double* P, double* tmp, double* ws,
-                           long ws_elems, hipStream_t st);
+// Per trial of up to two spins: Q (N, N - O), orthonormal complement of span(mo),
+// and P (N, O) = mo (mo^T mo)^-1.  tmp: the setup workspace of the larger one.
+struct ExTrial {
+  const double* mo;
+  int O;
+  double* Q;
+  double* P;
+};
+int exchange_f64_set_trial(const ExTrial* sets, int nsets, int N, double* tmp, hipStream_t st);
 // From rot_chol (G, O, N): a, c0 (G,), mt (O, N - O), k0 (1,); kg (G,) scratch.
 int exchange_f64_set_chol(const double* rc, const double* Q, const double* P, int N, int O, int G, double* a,
                           double* c0, double* mt, double* k0, double* kg, double* tmp, double* ws, long ws_elems,

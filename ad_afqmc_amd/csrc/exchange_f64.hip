@@ -303,17 +303,36 @@ __global__ __launch_bounds__(256) void exchange_occ_kernel(const double2* __rest
 }
 
 // ------------------------------------------------------------------ setup
-// Householder vectors of T (N x O, row-major): V (O, N), column k's reflector
-// H_k = 1 - tau_k v_k v_k^T with v_k zero above row k.  One work-group; a wave
-// updates whole columns, in LDS where they fit (LOC).
+// QR factors of the trial orbitals T = Q1 R (both spins in a launch, blockIdx.y):
+// Q completes Q1 to an orthogonal matrix, and P = T (T^T T)^-1 = Q1 R^-T.  Taken
+// from R, P is off by the condition of T.  By way of the Gram matrix T^T T, whose
+// condition is its square, the energies of trials with condition 1e3 to 1e5 were
+// off by 1.6 times what f = rot_chol G^T itself gives in FP64; by 0.74 times now.
+struct TrialQR {
+  const double* T;  // (N, O)
+  int O;
+  double* V;        // (O, N) Householder vectors
+  double* tau;      // (O,)
+  double* RT;       // (O, O) R by columns, upper part
+  double* Q1;       // (N, O)
+  double* Q;        // (N, N - O)
+  double* P;        // (N, O)
+};
+struct TrialQR2 {
+  TrialQR s[2];
+};
+
+// Column k's reflector is H_k = 1 - tau_k v_k v_k^T with v_k zero above row k.
+// One work-group; a wave updates whole columns, in LDS where they fit (LOC).
 template <bool LOC>
-__global__ __launch_bounds__(1024) void householder_kernel(const double* __restrict__ T, int N, int O,
-                                                           double* __restrict__ V, double* __restrict__ tau) {
+__global__ __launch_bounds__(1024) void householder_kernel(TrialQR2 sets, int N) {
   extern __shared__ double hv[];
   __shared__ double stau;
+  const TrialQR& q = sets.s[blockIdx.y];
+  const int O = q.O;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  double* X = LOC ? hv : V;
-  for (long e = tid; e < (long)N * O; e += 1024) X[(e % O) * N + e / O] = T[e];
+  double* X = LOC ? hv : q.V;
+  for (long e = tid; e < (long)N * O; e += 1024) X[(e % O) * N + e / O] = q.T[e];
   __syncthreads();
   for (int k = 0; k < O; ++k) {
     double* v = X + (long)k * N;
@@ -326,10 +345,14 @@ __global__ __launch_bounds__(1024) void householder_kernel(const double* __restr
       // v^T v = s - x^2 + vk^2 = 2 nrm (nrm + |x|)
       const double vv = 2.0 * nrm * (nrm + fabs(x));
       const double t = vv > 0.0 ? 2.0 / vv : 0.0;
-      for (int r = lane; r < k; r += 64) v[r] = 0.0;
+      for (int r = lane; r < k; r += 64) {
+        q.RT[k * O + r] = v[r];
+        v[r] = 0.0;
+      }
       if (lane == 0) {
+        q.RT[k * O + k] = x < 0.0 ? nrm : -nrm;
         v[k] = vk;
-        tau[k] = t;
+        q.tau[k] = t;
         stau = t;
       }
     }
@@ -345,33 +368,50 @@ __global__ __launch_bounds__(1024) void householder_kernel(const double* __restr
     __syncthreads();
   }
   if (LOC)
-    for (long e = tid; e < (long)N * O; e += 1024) V[e] = X[e];
+    for (long e = tid; e < (long)N * O; e += 1024) q.V[e] = X[e];
 }
 
-// Column a of Q (N x Nv, row-major): H_0 ... H_{O-1} e_{O + a}, one wave each
-// (a lane owns the rows r = lane mod 64).
-__global__ __launch_bounds__(64) void complement_kernel(const double* __restrict__ V, const double* __restrict__ tau,
-                                                        int N, int O, double* __restrict__ Q) {
-  const int a = blockIdx.x, lane = threadIdx.x, Nv = N - O;
-  double* x = Q + a;
-  for (int r = lane; r < N; r += 64) x[(long)r * Nv] = r == O + a ? 1.0 : 0.0;
+// Column blockIdx.x of H_0 ... H_{O-1}: the first O are Q1, the others Q.  One
+// wave each (a lane owns the rows r = lane mod 64).
+__global__ __launch_bounds__(64) void basis_kernel(TrialQR2 sets, int N) {
+  const TrialQR& q = sets.s[blockIdx.y];
+  const int a = blockIdx.x, lane = threadIdx.x, O = q.O;
+  const int ld = a < O ? O : N - O;
+  double* x = a < O ? q.Q1 + a : q.Q + (a - O);
+  for (int r = lane; r < N; r += 64) x[(long)r * ld] = r == a ? 1.0 : 0.0;
   for (int k = O - 1; k >= 0; --k) {
-    const double* v = V + (long)k * N;
+    const double* v = q.V + (long)k * N;
     const int r0 = k + ((lane - k) & 63);
     double d = 0.0;
-    for (int r = r0; r < N; r += 64) d += v[r] * x[(long)r * Nv];
-    d = tau[k] * wave_sum(d);
-    for (int r = r0; r < N; r += 64) x[(long)r * Nv] -= d * v[r];
+    for (int r = r0; r < N; r += 64) d += v[r] * x[(long)r * ld];
+    d = q.tau[k] * wave_sum(d);
+    for (int r = r0; r < N; r += 64) x[(long)r * ld] -= d * v[r];
   }
 }
 
-__global__ void real_to_complex_kernel(const double* __restrict__ in, double2* __restrict__ out, long n) {
-  const long i = blockIdx.x * 256L + threadIdx.x;
-  if (i < n) out[i] = double2{in[i], 0.0};
-}
-__global__ void real_part_kernel(const double2* __restrict__ in, double* __restrict__ out, long n) {
-  const long i = blockIdx.x * 256L + threadIdx.x;
-  if (i < n) out[i] = in[i].x;
+// Row r of P = Q1 R^-T: R p = (row r of Q1), by back substitution.  One wave a
+// row, lane i holding the entries i and i + 64.
+__global__ __launch_bounds__(64) void dual_kernel(TrialQR2 sets) {
+  static_assert(kExchangeF64MaxO <= 128, "two entries a lane");
+  const TrialQR& q = sets.s[blockIdx.y];
+  const int lane = threadIdx.x, O = q.O;
+  const long row = (long)blockIdx.x * O;
+  double x[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) x[h] = lane + 64 * h < O ? q.Q1[row + lane + 64 * h] : 0.0;
+  for (int j = O - 1; j >= 0; --j) {
+    const double* c = q.RT + (long)j * O;
+    const double pj = __shfl(j < 64 ? x[0] : x[1], j & 63) / c[j];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int i = lane + 64 * h;
+      if (i < j) x[h] -= c[i] * pj;
+      if (i == j) x[h] = pj;
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    if (lane + 64 * h < O) q.P[row + lane + 64 * h] = x[h];
 }
 
 // Tile rows of A from rcv (gn x O x Nv, chunks [0, nck) of gw g's): per chunk,
@@ -542,49 +582,41 @@ static Setup setup_pass(int O, int N, int G) {
   return u;
 }
 
+static long trial_elems(int O, int N) { return 2L * O * N + O + (long)O * O; }
+
 long exchange_f64_tmp_elems(int O, int N, int G) {
   const Setup u = setup_pass(O, N, G);
-  return std::max((long)u.gc * O * (N - O) + 2L * u.gc * O * O + (long)u.ns * O * (N - O),
-                  (long)O * N + O + 6L * O * O + 2);
+  return std::max((long)u.gc * O * (N - O) + 2L * u.gc * O * O + (long)u.ns * O * (N - O), 2 * trial_elems(O, N));
 }
 
-int exchange_f64_set_trial(const double* mo, int N, int O, double* Q, double* P, double* tmp, double* ws,
-                           long ws_elems, hipStream_t st) {
-  const int Nv = N - O;
-  const long OO = (long)O * O;
-  double2* cg = reinterpret_cast<double2*>(tmp);
-  double2* ci = cg + OO;
-  double2* det = ci + OO;
-  double* V = reinterpret_cast<double*>(det + 1);
-  double* tau = V + (long)O * N;
-  double* gram = tau + O;
-  double* inv = gram + OO;
-  if (Nv > 0) {
-    const size_t bytes = sizeof(double) * N * O;
-    constexpr size_t most = 152 * 1024;
-    if (bytes <= most) {
-      static std::atomic<bool> raised{false};
-      AFQ_TRY(raise_lds(reinterpret_cast<const void*>(householder_kernel<true>), most, raised, "householder"));
-      hipLaunchKernelGGL(householder_kernel<true>, dim3(1), dim3(1024), bytes, st, mo, N, O, V, tau);
-    } else {
-      hipLaunchKernelGGL(householder_kernel<false>, dim3(1), dim3(1024), 0, st, mo, N, O, V, tau);
-    }
-    AFQ_TRY(launch_status("householder_kernel"));
-    hipLaunchKernelGGL(complement_kernel, dim3(Nv), dim3(64), 0, st, V, tau, N, O, Q);
-    AFQ_TRY(launch_status("complement_kernel"));
+int exchange_f64_set_trial(const ExTrial* sets, int nsets, int N, double* tmp, hipStream_t st) {
+  if (nsets < 1) return AFQ_OK;
+  TrialQR2 q{};
+  int omax = 0;
+  for (int i = 0; i < nsets; ++i) {
+    const int O = sets[i].O;
+    double* V = tmp;
+    double* tau = V + (long)O * N;
+    double* RT = tau + O;
+    double* Q1 = RT + (long)O * O;
+    q.s[i] = TrialQR{sets[i].mo, O, V, tau, RT, Q1, sets[i].Q, sets[i].P};
+    tmp += trial_elems(O, N);
+    omax = std::max(omax, O);
   }
-  // P = T (T^T T)^-1, then one step P <- P (2 - T^T P)
-  AFQ_TRY(mm(st, O, O, N, mo, O, true, mo, O, gram, O, 1.0, 0.0, ws, ws_elems));
-  hipLaunchKernelGGL(real_to_complex_kernel, dim3(blocks(OO)), dim3(256), 0, st, gram, cg, OO);
-  AFQ_TRY(launch_status("real_to_complex_kernel"));
-  AFQ_TRY(batched_det_inv(cg, OO, O, 1, det, ci, OO, st));
-  hipLaunchKernelGGL(real_part_kernel, dim3(blocks(OO)), dim3(256), 0, st, ci, inv, OO);
-  AFQ_TRY(launch_status("real_part_kernel"));
-  double* P0 = V;  // the reflectors are no longer needed
-  AFQ_TRY(mm(st, N, O, O, mo, O, false, inv, O, P0, O, 1.0, 0.0, ws, ws_elems));
-  AFQ_TRY(mm(st, O, O, N, mo, O, true, P0, O, gram, O, 1.0, 0.0, ws, ws_elems));
-  AFQ_HIP(hipMemcpyAsync(P, P0, sizeof(double) * N * O, hipMemcpyDeviceToDevice, st));
-  return mm(st, N, O, O, P0, O, false, gram, O, P, O, -1.0, 2.0, ws, ws_elems);
+  const size_t bytes = sizeof(double) * N * omax;
+  constexpr size_t most = 152 * 1024;
+  if (bytes <= most) {
+    static std::atomic<bool> raised{false};
+    AFQ_TRY(raise_lds(reinterpret_cast<const void*>(householder_kernel<true>), most, raised, "householder"));
+    hipLaunchKernelGGL(householder_kernel<true>, dim3(1, nsets), dim3(1024), bytes, st, q, N);
+  } else {
+    hipLaunchKernelGGL(householder_kernel<false>, dim3(1, nsets), dim3(1024), 0, st, q, N);
+  }
+  AFQ_TRY(launch_status("householder_kernel"));
+  hipLaunchKernelGGL(basis_kernel, dim3(N, nsets), dim3(64), 0, st, q, N);
+  AFQ_TRY(launch_status("basis_kernel"));
+  hipLaunchKernelGGL(dual_kernel, dim3(N, nsets), dim3(64), 0, st, q);
+  return launch_status("dual_kernel");
 }
 
 int exchange_f64_set_chol(const double* rc, const double* Q, const double* P, int N, int O, int G, double* a,
