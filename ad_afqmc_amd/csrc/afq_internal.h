@@ -247,7 +247,7 @@ struct afq_job {
   uint16_t* vsplit = nullptr;             // (W, 4, 16 ceil(N/16), 32 ceil(N/32)) split VHS planes
   // FP64 exchange over the trial's unoccupied orbitals (exchange_f64.hip), per
   // spin: Q, P from the trial; packed rot_chol Q, tr f0, M^T and K0 from
-  // rot_chol.  Null where another exchange runs (x_f64).
+  // rot_chol.  Null where nothing reads them (x_set).
   double* xq_q[2] = {nullptr, nullptr};   // (N, N - nocc)
   double* xq_p[2] = {nullptr, nullptr};   // (N, nocc)
   double* xq_a[2] = {nullptr, nullptr};
@@ -259,9 +259,8 @@ struct afq_job {
   double2* small_rc = nullptr;
   double* h_step = nullptr;               // (steps, W) phaseless factors of a small job's block
   long h_cap = 0;
-  double* xq_kg = nullptr;                // (G,) setup scratch
+  double* xq_kg = nullptr;                // (2 G,) setup scratch
   double* xq_tmp = nullptr;               // setup scratch
-  bool rc_set[2] = {false, false};        // rot_chol has been built or supplied
   // nocc > 128: stored f blocks of the wide exchange path (k_exchange_wide)
   double2* xwide = nullptr;
   long xwide_elems = 0;

@@ -86,6 +86,7 @@ int check_walkers(const afq_job* j, const void* up, const void* dn) {
 }
 
 bool small_meas(const afq_job* j);
+bool small_whole(const afq_job* j);
 int measure_small(afq_job* j, const void* up, const void* dn, bool qr, bool inverse, double2* energies,
                   double2* overlaps, hipStream_t st);
 
@@ -281,19 +282,27 @@ bool x_f64(const afq_job* j, int s) {
   return j->nocc[s] <= kExchangeF64MaxO && (!j->lp || j->nocc[s] > kExchangeRegMaxO);
 }
 
+// Whether its factors are read: not where a small job's measurement forms the
+// energies without them (small_whole).
+bool x_set(const afq_job* j, int s) { return x_f64(j, s) && !(small_meas(j) && small_whole(j)); }
+
 // Rebuilds the parts of that exchange that follow from the trial, and from
-// rot_chol once there is one.
+// rot_chol (of the spins in `which`, a mask).
 int x_f64_trial(afq_job* j, hipStream_t st) {
   ExTrial sets[2];
   int n = 0;
   for (int s = 0; s < (j->rhf ? 1 : 2); ++s)
-    if (x_f64(j, s)) sets[n++] = ExTrial{j->mo[s], j->nocc[s], j->xq_q[s], j->xq_p[s]};
+    if (x_set(j, s)) sets[n++] = ExTrial{j->mo[s], j->nocc[s], j->xq_q[s], j->xq_p[s]};
   return exchange_f64_set_trial(sets, n, j->N, j->xq_tmp, st);
 }
-int x_f64_chol(afq_job* j, int s, hipStream_t st) {
-  return exchange_f64_set_chol(j->rot_chol[s], j->xq_q[s], j->xq_p[s], j->N, j->nocc[s], j->G, j->xq_a[s],
-                               j->xq_c0[s], j->xq_mt[s], j->xq_k0[s], j->xq_kg, j->xq_tmp, j->gemm_ws,
-                               j->gemm_ws_elems, st);
+int x_f64_chol(afq_job* j, int which, hipStream_t st) {
+  ExChol sets[2];
+  int n = 0;
+  for (int s = 0; s < (j->rhf ? 1 : 2); ++s)
+    if ((which >> s & 1) && x_set(j, s))
+      sets[n++] = ExChol{j->rot_chol[s], j->xq_q[s], j->xq_p[s], j->nocc[s],
+                         j->xq_a[s], j->xq_c0[s], j->xq_mt[s], j->xq_k0[s]};
+  return exchange_f64_set_chol(sets, n, j->N, j->G, j->xq_kg, j->xq_tmp, j->gemm_ws, j->gemm_ws_elems, st);
 }
 
 // FP64 jobs whose walkers fit one work-group each (small.hip): for the
@@ -1077,7 +1086,7 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
     long tmp = 0, nb = 0;
     for (int s = 0; s < (j->rhf ? 1 : 2); ++s) {
       const int O = j->nocc[s];
-      if (!x_f64(j, s)) continue;
+      if (!x_set(j, s)) continue;
       A_(j->xq_q[s], N * (N - O));
       A_(j->xq_p[s], N * O);
       A_(j->xq_a[s], exchange_f64_a_elems(O, (int)N, (int)G));
@@ -1090,7 +1099,7 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
     if (tmp > 0) {
       A_(j->xq_b[0], nb);
       if (small_meas(j) && j->nspin_meas > 1) A_(j->xq_b[1], nb);
-      A_(j->xq_kg, G);
+      A_(j->xq_kg, 2 * G);
       A_(j->xq_tmp, tmp);
     }
   }
@@ -1318,8 +1327,9 @@ int afq_job_set_trial(afq_job_t j, const double* mo_up, const double* mo_dn, con
     AFQ_HIP(hipMemcpyAsync(j->mo[1], mo_dn, sizeof(double) * N * j->nocc[1], hipMemcpyDefault, S(stream)));
   AFQ_HIP(hipMemcpyAsync(j->rdm1, rdm1, sizeof(double) * 2 * N * N, hipMemcpyDefault, S(stream)));
   AFQ_TRY(x_f64_trial(j, S(stream)));
-  for (int s = 0; s < (j->rhf ? 1 : 2); ++s)
-    if (x_f64(j, s) && j->rc_set[s]) AFQ_TRY(x_f64_chol(j, s, S(stream)));
+  // A rot_chol that was built is built again before it counts; one that the caller
+  // supplied stays.
+  AFQ_TRY(x_f64_chol(j, (j->have_rot_chol[0] ? 1 : 0) | (j->have_rot_chol[1] ? 2 : 0), S(stream)));
   j->have_trial = true;
   j->have_meas = j->have_prop = false;
   return AFQ_OK;
@@ -1370,9 +1380,8 @@ int afq_build_measurement_intermediates(afq_job_t j, void* stream) {
     r.ldc = N;
     r.sC = (long)O * N;
     AFQ_TRY(gemm_f64(r, st));
-    j->rc_set[s] = true;
-    if (x_f64(j, s)) AFQ_TRY(x_f64_chol(j, s, st));
   }
+  AFQ_TRY(x_f64_chol(j, 3, st));
   AFQ_TRY(small_pack_rc(j, st));
   if (j->lp)
     for (int s = 0; s < nsp; ++s) {
@@ -1503,8 +1512,7 @@ int afq_set_intermediate(afq_job_t j, int which, int spin, const void* src, void
     case AFQ_INT_ROT_H1: j->have_rot_h1[spin] = true; break;
     case AFQ_INT_ROT_CHOL:
       j->have_rot_chol[spin] = true;
-      j->rc_set[spin] = true;
-      if (x_f64(j, spin) && j->have_trial) AFQ_TRY(x_f64_chol(j, spin, S(stream)));
+      if (j->have_trial) AFQ_TRY(x_f64_chol(j, 1 << spin, S(stream)));
       AFQ_TRY(small_pack_rc(j, S(stream)));
       if (j->lp) AFQ_TRY(k_to_f32(j->rot_chol[spin], j->rot_chol32[spin], G * O * N, S(stream)));
       if (j->rct32[spin])

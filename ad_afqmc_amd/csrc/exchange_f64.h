@@ -24,7 +24,7 @@ struct ExF64 {
 };
 
 // Sizes of the packed rot_chol Q (doubles), of the packed theta (complex) and
-// of the setup workspace (doubles).
+// of the setup workspace (doubles, for two spins of O).
 long exchange_f64_a_elems(int O, int N, int G);
 long exchange_f64_b_elems(int O, int N, int W);
 long exchange_f64_tmp_elems(int O, int N, int G);
@@ -37,10 +37,15 @@ struct ExTrial {
   double* P;
 };
 int exchange_f64_set_trial(const ExTrial* sets, int nsets, int N, double* tmp, hipStream_t st);
-// From rot_chol (G, O, N): a, c0 (G,), mt (O, N - O), k0 (1,); kg (G,) scratch.
-int exchange_f64_set_chol(const double* rc, const double* Q, const double* P, int N, int O, int G, double* a,
-                          double* c0, double* mt, double* k0, double* kg, double* tmp, double* ws, long ws_elems,
-                          hipStream_t st);
+// From rot_chol (G, O, N) of up to two spins: a, c0 (G,), mt (O, N - O), k0 (1,);
+// kg (2 G,) scratch.
+struct ExChol {
+  const double *rc, *Q, *P;
+  int O;
+  double *a, *c0, *mt, *k0;
+};
+int exchange_f64_set_chol(const ExChol* sets, int nsets, int N, int G, double* kg, double* tmp, double* ws,
+                          long ws_elems, hipStream_t st);
 // Rows (k pairs) of the packed theta of one walker group.
 int exchange_f64_npairs(int Nv);
 // green null: the caller has filled thetap and the last partial K already.

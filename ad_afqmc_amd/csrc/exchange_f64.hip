@@ -372,12 +372,33 @@ __global__ __launch_bounds__(1024) void householder_kernel(TrialQR2 sets, int N)
 }
 
 // Column blockIdx.x of H_0 ... H_{O-1}: the first O are Q1, the others Q.  One
-// wave each (a lane owns the rows r = lane mod 64).
+// wave each, a lane owning the rows lane + 64 t: R of them in registers, or in
+// memory where R = 0.
+template <int R>
 __global__ __launch_bounds__(64) void basis_kernel(TrialQR2 sets, int N) {
   const TrialQR& q = sets.s[blockIdx.y];
   const int a = blockIdx.x, lane = threadIdx.x, O = q.O;
   const int ld = a < O ? O : N - O;
   double* x = a < O ? q.Q1 + a : q.Q + (a - O);
+  if constexpr (R > 0) {
+    double y[R];
+#pragma unroll
+    for (int t = 0; t < R; ++t) y[t] = lane + 64 * t == a ? 1.0 : 0.0;
+    for (int k = O - 1; k >= 0; --k) {
+      double v[R], d = 0.0;
+#pragma unroll
+      for (int t = 0; t < R; ++t) v[t] = lane + 64 * t < N ? q.V[(long)k * N + lane + 64 * t] : 0.0;  // 0 above k
+#pragma unroll
+      for (int t = 0; t < R; ++t) d += v[t] * y[t];
+      d = q.tau[k] * wave_sum(d);
+#pragma unroll
+      for (int t = 0; t < R; ++t) y[t] -= d * v[t];
+    }
+#pragma unroll
+    for (int t = 0; t < R; ++t)
+      if (lane + 64 * t < N) x[(long)(lane + 64 * t) * ld] = y[t];
+    return;
+  }
   for (int r = lane; r < N; r += 64) x[(long)r * ld] = r == a ? 1.0 : 0.0;
   for (int k = O - 1; k >= 0; --k) {
     const double* v = q.V + (long)k * N;
@@ -405,8 +426,8 @@ __global__ __launch_bounds__(64) void dual_kernel(TrialQR2 sets) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int i = lane + 64 * h;
-      if (i < j) x[h] -= c[i] * pj;
-      if (i == j) x[h] = pj;
+      const double ci = i < j ? c[i] : 0.0;
+      x[h] = i == j ? pj : i < j ? x[h] - ci * pj : x[h];
     }
   }
 #pragma unroll
@@ -463,23 +484,134 @@ __global__ __launch_bounds__(256) void occ_terms_kernel(const double* __restrict
   }
 }
 
-// out[e] = sum_s part[s][e] in the order of s
-__global__ void sum_slices_kernel(const double* __restrict__ part, int ns, long n, double* __restrict__ out) {
-  const long e = blockIdx.x * 256L + threadIdx.x;
-  if (e >= n) return;
+// Sums of the set-up: mt[e] = sum_i part[i][e] over ns slices of n, and k0 = sum_g
+// kg[g] (the last work-group); 16 waves take every 16th slice each, added in order.
+struct SetupSum {
+  const double* part;
+  const double* kg;
+  int ns;
+  long n;
+  double* mt;
+  double* k0;
+};
+struct SetupSum2 {
+  SetupSum s[2];
+};
+__global__ __launch_bounds__(1024) void setup_sum_kernel(SetupSum2 sets, int G) {
+  __shared__ double red[16][64];
+  const SetupSum& p = sets.s[blockIdx.y];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool last = blockIdx.x == gridDim.x - 1;
+  const long e = blockIdx.x * 64L + lane;
   double s = 0.0;
-  for (int i = 0; i < ns; ++i) s += part[i * n + e];
-  out[e] = s;
+  if (last) {
+    for (int g = threadIdx.x; g < G; g += 1024) s += p.kg[g];
+    s = wave_sum(s);
+  } else if (e < p.n) {
+#pragma unroll 4
+    for (int i = wave; i < p.ns; i += 16) s += p.part[i * p.n + e];
+  }
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave > 0) return;
+  double t = 0.0;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) t += red[i][lane];
+  if (last) {
+    if (lane == 0) *p.k0 = t;
+  } else if (e < p.n) {
+    p.mt[e] = t;
+  }
 }
 
-__global__ __launch_bounds__(256) void sum_kernel(const double* __restrict__ x, int n, double* __restrict__ out) {
-  __shared__ double red[4];
-  double s = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) s += x[i];
-  s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+// The set-up of a few occupied orbitals, one work-group a Cholesky index g: f0 and
+// rot_chol_g Q in LDS, then c0, tr(f0 f0), this g's part of M and its rows of the
+// packed A (zero in the tile rows past the chunk's last g).  Thread (c, i0) forms
+// column c of rows i0, i0 + ni, ...  Bound: launches, of which the general products
+// take seven a spin.  Intermediates and job of a run (UHF N = 20, O = 6 / 5, G = 80,
+// 100 walkers): 1.27 ms before, 0.96 now; RHF N = 10, O = 5, G = 27, which needs no
+// factors at all: 0.76 and 0.55.
+constexpr int kSetupMaxN = 128, kSetupMaxO = 24;
+struct SetupSmall {
+  const double *rc, *Q, *P;
+  int O, gw, RB, n8;
+  double *c0, *kg, *part;
+  double2* a;
+};
+struct SetupSmall2 {
+  SetupSmall s[2];
+};
+__global__ __launch_bounds__(256) void setup_small_kernel(SetupSmall2 sets, int N, int G) {
+  extern __shared__ double sh[];
+  __shared__ double red[8];
+  const SetupSmall& p = sets.s[blockIdx.y];
+  const int O = p.O, Nv = N - O, tid = threadIdx.x, g = blockIdx.x;
+  double* rc = sh;           // (O, N)
+  double* rv = rc + O * N;   // (O, Nv)
+  double* f = rv + O * Nv;   // (O, O)
+  for (int e = tid; e < O * N; e += 256) rc[e] = p.rc[(long)g * O * N + e];
   __syncthreads();
-  if (threadIdx.x == 0) *out = red[0] + red[1] + red[2] + red[3];
+  const int ni = 256 / N, i0 = tid / N, c = tid - i0 * N;  // ni >= 2
+  if (i0 < ni) {
+    const double* b = c < O ? p.P + c : p.Q + (c - O);
+    const int ld = c < O ? O : Nv;
+    double acc[kSetupMaxO / 2];
+#pragma unroll
+    for (int k = 0; k < kSetupMaxO / 2; ++k) acc[k] = 0.0;
+#pragma unroll 8
+    for (int r = 0; r < N; ++r) {
+      const double x = b[(long)r * ld];
+#pragma unroll
+      for (int k = 0; k < kSetupMaxO / 2; ++k)
+        if (i0 + k * ni < O) acc[k] += rc[(i0 + k * ni) * N + r] * x;
+    }
+#pragma unroll
+    for (int k = 0; k < kSetupMaxO / 2; ++k) {
+      const int i = i0 + k * ni;
+      if (i >= O) continue;
+      if (c < O)
+        f[i * O + c] = acc[k];
+      else
+        rv[i * Nv + c - O] = acc[k];
+    }
+  }
+  __syncthreads();
+  double t = 0.0, kk = 0.0;
+  for (int e = tid; e < O * O; e += 256) {
+    const int i = e / O, j = e - i * O;
+    kk += f[e] * f[j * O + i];
+    if (i == j) t += f[e];
+  }
+  t = wave_sum(t);
+  kk = wave_sum(kk);
+  if ((tid & 63) == 0) {
+    red[tid >> 6] = t;
+    red[4 + (tid >> 6)] = kk;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    p.c0[g] = red[0] + red[1] + red[2] + red[3];
+    p.kg[g] = red[4] + red[5] + red[6] + red[7];
+  }
+  for (int e = tid; e < O * Nv; e += 256) {
+    const int i = e / Nv, v = e - i * Nv;
+    double m = 0.0;
+    for (int k = 0; k < O; ++k) m += f[i * O + k] * rv[k * Nv + v];
+    p.part[(long)g * O * Nv + e] = m;
+  }
+  const int ck = g / p.gw, row0 = (g - ck * p.gw) * O;
+  const bool fill = g == G - 1 || g == ck * p.gw + p.gw - 1;
+  const int rows = fill ? 16 * p.RB - row0 : O, nk = 4 * p.n8;
+  double2* out = p.a + (long)ck * p.RB * p.n8 * 64;
+  for (int e = tid; e < rows * nk; e += 256) {
+    const int i = e / nk, sq = e - i * nk, k = 2 * sq, row = row0 + i;
+    double2 v = {0.0, 0.0};
+    if (i < O) {
+      if (k < Nv) v.x = rv[i * Nv + k];
+      if (k + 1 < Nv) v.y = rv[i * Nv + k + 1];
+    }
+    out[((row >> 4) * p.n8 + (sq >> 2)) * 64 + (sq & 3) * 16 + (row & 15)] = v;
+  }
 }
 
 unsigned blocks(long n) { return (unsigned)((n + 255) / 256); }
@@ -582,11 +714,16 @@ static Setup setup_pass(int O, int N, int G) {
   return u;
 }
 
+// Sizes of setup_small_kernel (48 KB of LDS at most).
+static bool setup_small(int O, int N) { return N <= kSetupMaxN && O <= kSetupMaxO; }
+
 static long trial_elems(int O, int N) { return 2L * O * N + O + (long)O * O; }
 
 long exchange_f64_tmp_elems(int O, int N, int G) {
   const Setup u = setup_pass(O, N, G);
-  return std::max((long)u.gc * O * (N - O) + 2L * u.gc * O * O + (long)u.ns * O * (N - O), 2 * trial_elems(O, N));
+  const long chol = setup_small(O, N) ? 2L * G * O * (N - O)
+                                      : (long)u.gc * O * (N - O) + 2L * u.gc * O * O + (long)u.ns * O * (N - O);
+  return std::max(chol, 2 * trial_elems(O, N));
 }
 
 int exchange_f64_set_trial(const ExTrial* sets, int nsets, int N, double* tmp, hipStream_t st) {
@@ -613,15 +750,25 @@ int exchange_f64_set_trial(const ExTrial* sets, int nsets, int N, double* tmp, h
     hipLaunchKernelGGL(householder_kernel<false>, dim3(1, nsets), dim3(1024), 0, st, q, N);
   }
   AFQ_TRY(launch_status("householder_kernel"));
-  hipLaunchKernelGGL(basis_kernel, dim3(N, nsets), dim3(64), 0, st, q, N);
+  const dim3 grid(N, nsets);
+  if (N <= 64)
+    hipLaunchKernelGGL(basis_kernel<1>, grid, dim3(64), 0, st, q, N);
+  else if (N <= 128)
+    hipLaunchKernelGGL(basis_kernel<2>, grid, dim3(64), 0, st, q, N);
+  else if (N <= 512)
+    hipLaunchKernelGGL(basis_kernel<8>, grid, dim3(64), 0, st, q, N);
+  else
+    hipLaunchKernelGGL(basis_kernel<0>, grid, dim3(64), 0, st, q, N);
   AFQ_TRY(launch_status("basis_kernel"));
   hipLaunchKernelGGL(dual_kernel, dim3(N, nsets), dim3(64), 0, st, q);
   return launch_status("dual_kernel");
 }
 
-int exchange_f64_set_chol(const double* rc, const double* Q, const double* P, int N, int O, int G, double* a,
-                          double* c0, double* mt, double* k0, double* kg, double* tmp, double* ws, long ws_elems,
-                          hipStream_t st) {
+// One spin by general products, passes of gc g's at a time; leaves ns slices of M
+// in *part_out and tr(f0 f0) in kg.
+static int set_chol_general(const ExChol& x, int N, int G, double* kg, double* tmp, double* ws, long ws_elems,
+                            double** part_out, hipStream_t st) {
+  const int O = x.O;
   const ExF64Tile t = exchange_f64_tile(O);
   const int Nv = N - O, n8 = (Nv + 7) / 8, RB = t.MB * t.WR;
   const Setup u = setup_pass(O, N, G);
@@ -630,14 +777,15 @@ int exchange_f64_set_chol(const double* rc, const double* Q, const double* P, in
   double* f0 = rcv + (long)gc * O * Nv;
   double* ft = f0 + (long)gc * O * O;
   double* part = ft + (long)gc * O * O;
+  *part_out = part;
   for (int g0 = 0; g0 < G; g0 += gc) {
     const int gn = std::min(gc, G - g0);
-    const double* r = rc + (long)g0 * O * N;
-    AFQ_TRY(mm(st, gn * O, O, N, r, N, false, P, O, f0, O, 1.0, 0.0, nullptr, 0));
-    hipLaunchKernelGGL(occ_terms_kernel, dim3(gn), dim3(256), 0, st, f0, O, c0 + g0, kg + g0, ft);
+    const double* r = x.rc + (long)g0 * O * N;
+    AFQ_TRY(mm(st, gn * O, O, N, r, N, false, x.P, O, f0, O, 1.0, 0.0, nullptr, 0));
+    hipLaunchKernelGGL(occ_terms_kernel, dim3(gn), dim3(256), 0, st, f0, O, x.c0 + g0, kg + g0, ft);
     AFQ_TRY(launch_status("occ_terms_kernel"));
     if (Nv == 0) continue;
-    AFQ_TRY(mm(st, gn * O, Nv, N, r, N, false, Q, Nv, rcv, Nv, 1.0, 0.0, nullptr, 0));
+    AFQ_TRY(mm(st, gn * O, Nv, N, r, N, false, x.Q, Nv, rcv, Nv, 1.0, 0.0, nullptr, 0));
     Gemm m;  // slice i of M: the g's [i gs, (i + 1) gs) of every pass
     m.M = O;
     m.N = Nv;
@@ -662,16 +810,51 @@ int exchange_f64_set_chol(const double* rc, const double* Q, const double* P, in
     const long nck = (gn + t.gw - 1) / t.gw;
     const long n = nck * RB * n8 * 64;
     hipLaunchKernelGGL(pack_a_kernel, dim3(blocks(n)), dim3(256), 0, st, rcv, O, Nv, t.gw, gn, RB, n8, nck,
-                       reinterpret_cast<double2*>(a + (long)(g0 / t.gw) * RB * n8 * 128));
+                       reinterpret_cast<double2*>(x.a + (long)(g0 / t.gw) * RB * n8 * 128));
     AFQ_TRY(launch_status("pack_a_kernel"));
   }
-  const long n = (long)O * Nv;
-  if (n > 0) {
-    hipLaunchKernelGGL(sum_slices_kernel, dim3(blocks(n)), dim3(256), 0, st, part, u.ns, n, mt);
-    AFQ_TRY(launch_status("sum_slices_kernel"));
+  return AFQ_OK;
+}
+
+static int set_sums(const SetupSum2& q, int nsets, int G, hipStream_t st) {
+  const long n = std::max(q.s[0].n, q.s[1].n);
+  hipLaunchKernelGGL(setup_sum_kernel, dim3((unsigned)((n + 63) / 64 + 1), nsets), dim3(1024), 0, st, q, G);
+  return launch_status("setup_sum_kernel");
+}
+
+int exchange_f64_set_chol(const ExChol* sets, int nsets, int N, int G, double* kg, double* tmp, double* ws,
+                          long ws_elems, hipStream_t st) {
+  SetupSmall2 p{};
+  SetupSum2 q{};
+  int ns = 0;
+  double* part = tmp;
+  size_t lds = 0;
+  for (int i = 0; i < nsets; ++i) {
+    const ExChol& x = sets[i];
+    if (!setup_small(x.O, N)) continue;
+    const ExF64Tile t = exchange_f64_tile(x.O);
+    const long n = (long)x.O * (N - x.O);
+    double* k = kg + ns * (long)G;
+    p.s[ns] = SetupSmall{x.rc, x.Q, x.P, x.O, t.gw, t.MB * t.WR, (N - x.O + 7) / 8, x.c0, k, part,
+                         reinterpret_cast<double2*>(x.a)};
+    q.s[ns++] = SetupSum{part, k, G, n, x.mt, x.k0};
+    part += G * n;
+    lds = std::max(lds, sizeof(double) * (2 * (size_t)x.O * N));
   }
-  hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(256), 0, st, kg, G, k0);
-  return launch_status("sum_kernel");
+  if (ns > 0) {
+    hipLaunchKernelGGL(setup_small_kernel, dim3(G, ns), dim3(256), lds, st, p, N, G);
+    AFQ_TRY(launch_status("setup_small_kernel"));
+    AFQ_TRY(set_sums(q, ns, G, st));
+  }
+  for (int i = 0; i < nsets; ++i) {
+    const ExChol& x = sets[i];
+    if (setup_small(x.O, N)) continue;
+    AFQ_TRY(set_chol_general(x, N, G, kg, tmp, ws, ws_elems, &part, st));
+    SetupSum2 one{};
+    one.s[0] = SetupSum{part, kg, setup_pass(x.O, N, G).ns, (long)x.O * (N - x.O), x.mt, x.k0};
+    AFQ_TRY(set_sums(one, 1, G, st));
+  }
+  return AFQ_OK;
 }
 
 int k_exchange_f64(const double* a, const double* Q, const double* c0, const double* mt, const double* k0,
