@@ -258,6 +258,7 @@ struct afq_job {
   double2* small_l = nullptr;             // L and rot_chol packed for the steps of a small job
   double2* small_rc = nullptr;
   double* h_step = nullptr;               // (steps, W) phaseless factors of a small job's block
+  double* h_own = nullptr;                // its allocation, once it has grown
   long h_cap = 0;
   double* xq_kg = nullptr;                // (2 G,) setup scratch
   double* xq_tmp = nullptr;               // setup scratch
@@ -272,8 +273,8 @@ struct afq_job {
   double* cholp = nullptr;                // (G, npk) FP64 packed L
   double2* vhsp = nullptr;                // (W, npk) FP64 packed VHS, or by blocks (vhs_f64) with ep
   float2* vhsp32 = nullptr;               // (W, npk) reduced-precision packed VHS
-  char* slab = nullptr;                   // the allocation that holds the job's buffers
-  size_t slab_bytes = 0;
+  std::vector<char*> mem;                 // the allocations that hold the job's buffers
+  size_t mem_bytes = 0;                   // their size, but for what ends of pieces leave unused
   double* fb_ws = nullptr;                // partial sums of the FP64 force bias
   long fb_ws_elems = 0;
   double* gemm_ws = nullptr;              // split-K workspace

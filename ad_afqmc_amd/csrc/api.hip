@@ -45,18 +45,13 @@ int dalloc(void** p, size_t bytes) {
   return AFQ_OK;
 }
 
-inline bool in_slab(const afq_job* j, const void* p) {
-  const char* c = static_cast<const char*>(p);
-  return c >= j->slab && c < j->slab + j->slab_bytes;
-}
-
 void release(afq_job* j) {
   auto fr = [](void* p) {
     if (p) (void)hipFree(p);
   };
-  if (!in_slab(j, j->h_step)) fr(j->h_step);
+  fr(j->h_own);
   fr(j->fields);
-  fr(j->slab);
+  for (char* p : j->mem) fr(p);
   for (auto& p : j->prof) {
     for (auto& sp : p.spans) {
       (void)hipEventDestroy(sp.first);
@@ -1036,29 +1031,50 @@ void init_job(afq_job* j, const afq_job_desc* d) {
     if (x_f64(j, s)) j->kchunk_max = std::max(j->kchunk_max, exchange_f64_nchunk(j->nocc[s], j->G) + 1);
 }
 
-// Places every device buffer of the job in one allocation (dry: only sums the
-// bytes): creating and destroying a job of some 60 buffers takes 0.4-0.9 and
-// 2.8 ms at N=100, G=500, 256 walkers with an allocation for each, and 0.06 and
-// 0.25 ms with one, and a gradient makes a job for each call.
+// Places every device buffer of the job (dry: only sums the bytes).  Above
+// kSegmentedJob in one allocation: creating and destroying a job of some 60
+// buffers takes 0.4-0.9 and 2.8 ms at N=100, G=500, 256 walkers (340 MB) with an
+// allocation for each, and 0.06 and 0.25 ms with one, and a gradient makes a job
+// for each call.  Below, in allocations of kSegment: where jobs of several sizes
+// follow each other, as the facade's do, one of 16 to 48 MB takes 0.3 ms (RHF
+// N=48, O=16, G=200, 64 walkers, 40 MB: 0.28 ms, 0.07 with an allocation for
+// each buffer, 0.05 in pieces of 16 MB, 0.08 of 8; at 50-70 MB pieces are slower
+// again, 0.08 and 0.34 against 0.04 and 0.05 to create and destroy one of 52 MB).
+constexpr size_t kSegment = size_t(16) << 20, kSegmentedJob = size_t(48) << 20;
 int alloc_job(afq_job* j, bool dry, int64_t* total) {
   const long N = j->N, G = j->G, W = j->W;
   const long wmax = std::max(j->wcols, std::max(j->nocc[0], j->nocc[1]));
   // propagation panel: both spins' columns side by side for unrestricted walkers
   const long wprop = j->restricted ? j->wcols : (long)j->nocc[0] + j->nocc[1];
   const int kch = j->kchunk_max;
-  if (!dry) {
-    AFQ_TRY(alloc_job(j, true, total));
-    AFQ_TRY(dalloc_n(&j->slab, j->slab_bytes));
-  }
-  size_t off = 0;
+  size_t placed = 0, left = 0;
+  char* at = nullptr;
+  // Page-aligned room for `bytes` in the current allocation, or in a new one.
+  auto place = [&](size_t bytes) -> int {
+    const size_t room = (std::max(bytes, size_t(1)) + 4095) & ~size_t(4095);
+    if (!dry && room > left) {
+      const size_t rest = j->mem_bytes - placed;
+      const size_t want = j->mem_bytes > kSegmentedJob ? rest : std::max(room, std::min(kSegment, rest));
+      AFQ_TRY(dalloc_n(&at, want));
+      j->mem.push_back(at);
+      left = want;
+    }
+    placed += room;
+    if (!dry) left -= room;
+    return AFQ_OK;
+  };
+  if (!dry) AFQ_TRY(alloc_job(j, true, total));
   *total = 0;
-  // page-aligned, as separate allocations are
-#define A_(p, n)                                                                        \
-  do {                                                                                  \
-    const size_t bytes_ = (size_t)(n) * sizeof(*(p));                                   \
-    *total += (int64_t)bytes_;                                                          \
-    if (!dry) (p) = reinterpret_cast<std::remove_reference_t<decltype(p)>>(j->slab + off); \
-    off += (std::max(bytes_, size_t(1)) + 4095) & ~size_t(4095);                         \
+#define A_(p, n)                                                          \
+  do {                                                                    \
+    const size_t bytes_ = (size_t)(n) * sizeof(*(p));                     \
+    *total += (int64_t)bytes_;                                            \
+    const size_t before_ = placed;                                        \
+    AFQ_TRY(place(bytes_));                                               \
+    if (!dry) {                                                           \
+      (p) = reinterpret_cast<std::remove_reference_t<decltype(p)>>(at);   \
+      at += placed - before_;                                             \
+    }                                                                     \
   } while (0)
   A_(j->h1, 2 * N * N);
   A_(j->chol, G * N * N);
@@ -1199,7 +1215,7 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
     A_(j->small_rc, G * small_rc_pairs((int)N, small_osum(j)));
   }
 #undef A_
-  if (dry) j->slab_bytes = off;
+  if (dry) j->mem_bytes = placed;
   return AFQ_OK;
 }
 
@@ -1653,8 +1669,8 @@ int reserve_fields(afq_job* j, long need, hipStream_t st) {
   if (hneed > j->h_cap) {
     double* h = nullptr;
     AFQ_TRY(dalloc_n(&h, (size_t)hneed));
-    if (!in_slab(j, j->h_step)) (void)hipFree(j->h_step);
-    j->h_step = h;
+    if (j->h_own) (void)hipFree(j->h_own);
+    j->h_step = j->h_own = h;
     j->h_cap = hneed;
   }
   return AFQ_OK;
