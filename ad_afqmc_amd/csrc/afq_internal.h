@@ -274,7 +274,7 @@ struct afq_job {
   double2* vhsp = nullptr;                // (W, npk) FP64 packed VHS, or by blocks (vhs_f64) with ep
   float2* vhsp32 = nullptr;               // (W, npk) reduced-precision packed VHS
   std::vector<char*> mem;                 // the allocations that hold the job's buffers
-  size_t mem_bytes = 0;                   // their size, but for what ends of pieces leave unused
+  size_t mem_bytes = 0, mem_large = 0;    // what the buffers take, and the large ones of them
   double* fb_ws = nullptr;                // partial sums of the FP64 force bias
   long fb_ws_elems = 0;
   double* gemm_ws = nullptr;              // split-K workspace

@@ -1031,36 +1031,45 @@ void init_job(afq_job* j, const afq_job_desc* d) {
     if (x_f64(j, s)) j->kchunk_max = std::max(j->kchunk_max, exchange_f64_nchunk(j->nocc[s], j->G) + 1);
 }
 
-// Places every device buffer of the job (dry: only sums the bytes).  Above
-// kSegmentedJob in one allocation: creating and destroying a job of some 60
-// buffers takes 0.4-0.9 and 2.8 ms at N=100, G=500, 256 walkers (340 MB) with an
-// allocation for each, and 0.06 and 0.25 ms with one, and a gradient makes a job
-// for each call.  Below, in allocations of kSegment: where jobs of several sizes
-// follow each other, as the facade's do, one of 16 to 48 MB takes 0.3 ms (RHF
-// N=48, O=16, G=200, 64 walkers, 40 MB: 0.28 ms, 0.07 with an allocation for
-// each buffer, 0.05 in pieces of 16 MB, 0.08 of 8; at 50-70 MB pieces are slower
-// again, 0.08 and 0.34 against 0.04 and 0.05 to create and destroy one of 52 MB).
-constexpr size_t kSegment = size_t(16) << 20, kSegmentedJob = size_t(48) << 20;
+// Places every device buffer of the job (dry: only sums the bytes).  An allocation
+// of more than 2 MB is mapped for itself; the runtime keeps up to 64 MB of freed
+// ones, and past that each costs 0.24 ms to free.  Smaller ones come from blocks
+// that the runtime holds.  So a job makes one allocation of its large buffers (a
+// gradient makes a job for each call; N=100, G=500, 256 walkers, 340 MB: created
+// in 0.06 and destroyed in 0.25 ms, 0.4-0.9 and 2.8 with an allocation for each of
+// its 60 buffers), and a small job takes its small buffers in pieces below 2 MB
+// (as the facade sets a job up, intermediates and inputs included: UHF N=37,
+// O=9/7, G=149, 101 walkers 3.1 ms in one allocation, 2.9 in pieces of 16 MB,
+// 2.3 so, 2.45 with an allocation for each buffer; RHF N=30, O=17, G=120, 64
+// walkers 2.2-2.4, 2.2, 1.65 and 1.7).
+constexpr size_t kPiece = size_t(1920) << 10, kPiecedJob = size_t(48) << 20;
 int alloc_job(afq_job* j, bool dry, int64_t* total) {
   const long N = j->N, G = j->G, W = j->W;
   const long wmax = std::max(j->wcols, std::max(j->nocc[0], j->nocc[1]));
   // propagation panel: both spins' columns side by side for unrestricted walkers
   const long wprop = j->restricted ? j->wcols : (long)j->nocc[0] + j->nocc[1];
   const int kch = j->kchunk_max;
-  size_t placed = 0, left = 0;
-  char* at = nullptr;
-  // Page-aligned room for `bytes` in the current allocation, or in a new one.
-  auto place = [&](size_t bytes) -> int {
+  // Page-aligned room in the large buffers' allocation, or in a piece for small ones.
+  size_t all = 0, large = 0, left = 0;
+  char *big = nullptr, *piece = nullptr;
+  auto place = [&](size_t bytes, char** at) -> int {
     const size_t room = (std::max(bytes, size_t(1)) + 4095) & ~size_t(4095);
-    if (!dry && room > left) {
-      const size_t rest = j->mem_bytes - placed;
-      const size_t want = j->mem_bytes > kSegmentedJob ? rest : std::max(room, std::min(kSegment, rest));
-      AFQ_TRY(dalloc_n(&at, want));
-      j->mem.push_back(at);
-      left = want;
+    const bool small = room <= kPiece && (dry || j->mem_bytes <= kPiecedJob);
+    all += room;
+    if (!small) large += room;
+    if (dry) return AFQ_OK;
+    if (small && room > left) {
+      AFQ_TRY(dalloc_n(&piece, kPiece));
+      j->mem.push_back(piece);
+      left = kPiece;
     }
-    placed += room;
-    if (!dry) left -= room;
+    if (!small && !big) {
+      AFQ_TRY(dalloc_n(&big, j->mem_bytes <= kPiecedJob ? j->mem_large : j->mem_bytes));
+      j->mem.push_back(big);
+    }
+    *at = small ? piece : big;
+    (small ? piece : big) += room;
+    if (small) left -= room;
     return AFQ_OK;
   };
   if (!dry) AFQ_TRY(alloc_job(j, true, total));
@@ -1069,12 +1078,9 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
   do {                                                                    \
     const size_t bytes_ = (size_t)(n) * sizeof(*(p));                     \
     *total += (int64_t)bytes_;                                            \
-    const size_t before_ = placed;                                        \
-    AFQ_TRY(place(bytes_));                                               \
-    if (!dry) {                                                           \
-      (p) = reinterpret_cast<std::remove_reference_t<decltype(p)>>(at);   \
-      at += placed - before_;                                             \
-    }                                                                     \
+    char* at_ = nullptr;                                                  \
+    AFQ_TRY(place(bytes_, &at_));                                         \
+    if (!dry) (p) = reinterpret_cast<std::remove_reference_t<decltype(p)>>(at_); \
   } while (0)
   A_(j->h1, 2 * N * N);
   A_(j->chol, G * N * N);
@@ -1215,7 +1221,10 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
     A_(j->small_rc, G * small_rc_pairs((int)N, small_osum(j)));
   }
 #undef A_
-  if (dry) j->mem_bytes = placed;
+  if (dry) {
+    j->mem_bytes = all;
+    j->mem_large = large;
+  }
   return AFQ_OK;
 }
 

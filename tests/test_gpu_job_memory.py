@@ -1,7 +1,8 @@
-"""A job's buffers lie in pieces of 16 MB, or above 48 MB in one allocation: jobs
-on both sides of that line give the oracle's step and energy (each buffer in a
-place of its own; 1e-10 of the largest value, the repository's FP64 parity), and
-creating and closing them over and over leaves no memory behind."""
+"""A job's small buffers lie in pieces below 2 MB and its large ones in one
+allocation, or above 48 MB all in one: jobs without large buffers, with both and
+past that line give the oracle's step and energy (each buffer in a place of its
+own; 1e-10 of the largest value, the repository's FP64 parity), and creating and
+closing them over and over leaves no memory behind."""
 import ctypes as C
 import math
 
