@@ -894,11 +894,16 @@ int compute_v0(afq_job* j, double* v0, hipStream_t st) {
   const int N = j->N, G = j->G;
   const long NN = (long)N * N;
   // accumulated over gamma chunks of a permuted copy: v0 = perm (N x nN) . L_chunk (nN x N)
-  const long gch = std::max(1L, std::min((long)G, (64L << 20) / (long)(sizeof(double) * NN)));
-  // the copy goes into the VHS buffer, which nothing uses between steps, where that holds it
+  long gch = std::max(1L, std::min((long)G, (64L << 20) / (long)(sizeof(double) * NN)));
+  // The copy goes into the VHS buffer, which nothing uses between steps, where that
+  // holds an eighth of it: a chunk more costs some 25 us, an allocation and its
+  // release 0.1 to 0.4 ms (RHF N=48, G=200, 64 walkers: two chunks instead).
   double* own = nullptr;
   double* perm = reinterpret_cast<double*>(j->vhs);
-  if (!perm || 2L * j->Wcap < gch) {
+  const long held = 2L * j->Wcap;
+  if (perm && 8 * held >= gch) {
+    gch = std::min(gch, held);
+  } else {
     AFQ_TRY(dalloc_n(&own, (size_t)(gch * NN)));
     perm = own;
   }
