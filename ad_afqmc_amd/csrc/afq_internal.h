@@ -254,7 +254,7 @@ struct afq_job {
   double* xq_c0[2] = {nullptr, nullptr};  // (G,)
   double* xq_mt[2] = {nullptr, nullptr};  // (nocc, N - nocc)
   double* xq_k0[2] = {nullptr, nullptr};  // (1,)
-  double2* xq_b[2] = {nullptr, nullptr};  // packed theta (one buffer for both spins unless the job is small)
+  double2* xq_b[2] = {nullptr, nullptr};  // packed theta (xq_theta)
   double2* small_l = nullptr;             // L and rot_chol packed for the steps of a small job
   double2* small_rc = nullptr;
   double* h_step = nullptr;               // (steps, W) phaseless factors of a small job's block

@@ -281,6 +281,12 @@ bool x_f64(const afq_job* j, int s) {
 // energies without them (small_whole).
 bool x_set(const afq_job* j, int s) { return x_f64(j, s) && !(small_meas(j) && small_whole(j)); }
 
+// Packed theta of a spin: a buffer of its own where both spins' are filled at once.
+double2* xq_theta(const afq_job* j, int s) {
+  const bool both = small_meas(j) || exchange_f64_few(j->nocc[s], j->N, j->W);
+  return s == 1 && both ? j->xq_b[1] : j->xq_b[0];
+}
+
 // Rebuilds the parts of that exchange that follow from the trial, and from
 // rot_chol (of the spins in `which`, a mask).
 int x_f64_trial(afq_job* j, hipStream_t st) {
@@ -308,7 +314,7 @@ int small_cols(const afq_job* j) { return j->restricted ? j->wcols : j->nocc[0] 
 bool small_occ(const afq_job* j) {
   return !j->lp && std::max(j->nocc[0], j->nocc[1]) <= kSmallMaxO && j->wcols <= kSmallMaxO;
 }
-bool small_meas(const afq_job* j) { return small_occ(j) && small_measure_lds(j->N, small_cols(j), small_osum(j)) > 0; }
+bool small_meas(const afq_job* j) { return small_occ(j) && small_measure_lds(j->N, small_cols(j), small_osum(j), j->nspin_meas) > 0; }
 bool small_whole(const afq_job* j) {
   return small_energy_whole(j->N, j->G, j->nocc[0], j->nspin_meas > 1 ? j->nocc[1] : 0);
 }
@@ -393,14 +399,14 @@ int measure_small(afq_job* j, const void* up, const void* dn, bool qr, bool inve
   p.overlaps = overlaps;
   p.ene1 = j->ene1;
   for (int s = 0; s < j->nspin_meas; ++s) {
-    const ExF64Tile t = exchange_f64_tile(j->nocc[s]);
+    const ExF64Tile t = exchange_f64_tile(j->nocc[s], j->W, j->G);
     p.green[s] = j->green[s];
     p.rh1[s] = j->rot_h1[s];
     p.rc[s] = j->rot_chol[s];
     p.q[s] = j->xq_q[s];
     p.mt[s] = j->xq_mt[s];
     p.k0[s] = j->xq_k0[s];
-    p.thetap[s] = j->xq_b[s];
+    p.thetap[s] = exchange_f64_few(j->nocc[s], j->N, j->W) ? nullptr : xq_theta(j, s);
     p.kpart[s] = j->kpart + (long)s * j->W * j->kchunk_max;
     p.wn[s] = t.wn;
     p.c2[s] = 8 * t.NB * t.WC;
@@ -417,7 +423,19 @@ int energy_pipeline(afq_job* j, const void* up, const void* dn, double2* out, hi
   if (small && small_whole(j)) return AFQ_OK;  // the energies are in out already
   if (!small && !have_green) AFQ_TRY(green_pipeline(j, up, dn, true, true, st));
   const bool two = !j->one_spin;
-  if (!small) {
+  // theta of the spins with few walkers, and then the one-body energies along with it
+  ExTheta th[2];
+  int nth = 0;
+  for (int s = 0; s < j->nspin_meas; ++s)
+    if (x_f64(j, s) && exchange_f64_few(j->nocc[s], j->N, j->W))
+      th[nth++] = ExTheta{j->green[s], j->xq_q[s], j->xq_mt[s], j->xq_k0[s], j->rot_h1[s], j->nocc[s], xq_theta(j, s),
+                          j->kpart + (long)s * j->W * j->kchunk_max};
+  const bool ene1_too = !small && nth == j->nspin_meas;
+  if (nth > 0) {
+    ProfScope ps(j, AFQ_K_EXCHANGE, st);
+    AFQ_TRY(exchange_f64_theta(th, nth, j->N, j->G, j->W, two ? 1.0 : 2.0, ene1_too ? j->ene1 : nullptr, st));
+  }
+  if (!small && !ene1_too) {
     ProfScope ps(j, AFQ_K_ENERGY_MISC, st);
     AFQ_TRY(k_ene1(j->green[0], j->rot_h1[0], j->nocc[0], two ? j->green[1] : nullptr, two ? j->rot_h1[1] : nullptr,
                    j->nocc[1], j->N, two ? 1.0 : 2.0, j->ene1, j->W, st));
@@ -448,8 +466,8 @@ int energy_pipeline(afq_job* j, const void* up, const void* dn, double2* out, hi
     ProfScope ps(j, AFQ_K_EXCHANGE, st);
     if (x_f64(j, s))  // theta in the SR gather buffer
       AFQ_TRY(k_exchange_f64(j->xq_a[s], j->xq_q[s], j->xq_c0[s], j->xq_mt[s], j->xq_k0[s],
-                             small ? nullptr : j->green[s], j->wgather,
-                             j->xq_b[s], j->nocc[s], j->N, j->G, j->W, coul, kpart, &nch[s], st));
+                             small || exchange_f64_few(j->nocc[s], j->N, j->W) ? nullptr : j->green[s], j->wgather,
+                             xq_theta(j, s), j->nocc[s], j->N, j->G, j->W, coul, kpart, &nch[s], st));
     else
       AFQ_TRY(k_exchange_wide(j->rot_chol[s], j->green[s], j->nocc[s], j->N, j->G, j->W, j->xwide, j->xwide_elems,
                               coul, kpart, &nch[s], st));
@@ -1033,7 +1051,7 @@ void init_job(afq_job* j, const afq_job_desc* d) {
   j->bf16x3 = d->precision == AFQ_PREC_BF16X3;
   j->kchunk_max = exchange_nchunk(j->G);
   for (int s = 0; s < 2; ++s)
-    if (x_f64(j, s)) j->kchunk_max = std::max(j->kchunk_max, exchange_f64_nchunk(j->nocc[s], j->G) + 1);
+    if (x_f64(j, s)) j->kchunk_max = std::max(j->kchunk_max, exchange_f64_slots(j->nocc[s], j->N, j->G));
 }
 
 // Places every device buffer of the job (dry: only sums the bytes).  An allocation
@@ -1125,7 +1143,10 @@ int alloc_job(afq_job* j, bool dry, int64_t* total) {
     }
     if (tmp > 0) {
       A_(j->xq_b[0], nb);
-      if (small_meas(j) && j->nspin_meas > 1) A_(j->xq_b[1], nb);
+      // both spins' at once: in a small job's measurement, and for few walkers
+      const int O = j->nocc[1];
+      const long w = small_meas(j) ? W : std::min(W, exchange_f64_most_few(O, (int)N));
+      if (j->nspin_meas > 1 && x_f64(j, 1) && w > 0) A_(j->xq_b[1], exchange_f64_b_elems(O, (int)N, (int)w));
       A_(j->xq_kg, 2 * G);
       A_(j->xq_tmp, tmp);
     }
@@ -1270,7 +1291,6 @@ int afq_job_create(afq_job_t* out, const afq_job_desc* d) {
       return fail(AFQ_E_HIP, std::string("hipMemset: ") + hipGetErrorString(e));
     }
   }
-  if (!j->xq_b[1]) j->xq_b[1] = j->xq_b[0];
   if (j->rhf) {
     j->mo[1] = j->mo[0];
     j->rot_h1[1] = j->rot_h1[0];

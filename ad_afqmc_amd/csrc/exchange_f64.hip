@@ -239,7 +239,7 @@ __global__ __launch_bounds__(64 * WR * WC, (waves_per_simd(MB, NB, WR * WC))) vo
     }
     sr = wave_sum(sr);
     si = wave_sum(si);
-    if (lane == 0) p.kpart[(long)(w0 + w) * (p.nchunk + 1) + chunk] = double2{sr, si};
+    if (lane == 0) p.kpart[(long)(w0 + w) * p.kstride + chunk] = double2{sr, si};
   }
 }
 
@@ -272,6 +272,124 @@ __global__ void pack_b_kernel(const double2* __restrict__ theta, int O, int Nv, 
 long exchange_thetap_elems(const ExF64Tile& t, int Nv, int W) {
   const int nslab = ((Nv + 7) / 8 + kSteps - 1) / kSteps;
   return (long)((W + t.wn - 1) / t.wn) * nslab * kPairs * 16 * t.NB * t.WC;
+}
+
+// The same for few walkers, straight from their Green's functions, in one launch
+// for both spins: theta_w of rows j0 .. j0 + 3 and 64 k's, each wave an eighth of
+// the sum over the orbitals, and these elements' part of 2 sum_ja M_ja theta_aj
+// (with K0, the first one's) in a slot of its own; and the one-body energies, a
+// work-group a walker.  Zero past Nv; columns of walkers past W stay unread.
+// Bound: the reads of Q, which each walker repeats (exchange_f64_few).
+constexpr int kThetaRows = 4, kThetaWaves = 8;
+struct ThetaSet {
+  const double2* green;
+  const double *Q, *mt, *k0, *rh1;
+  int O, nx, wn, C2, npr, nchunk, kstride;  // nx: blocks of 64 k's
+  double2* out;
+  double2* kpart;
+};
+struct ThetaArgs {
+  ThetaSet s[2];
+  int nsets, N;
+  double fac;
+  double2* ene1;
+};
+__global__ __launch_bounds__(64 * kThetaWaves) void theta_kernel(ThetaArgs a) {
+  __shared__ double2 part[kThetaWaves][kThetaRows][64];
+  __shared__ double2 red[kThetaWaves];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int N = a.N;
+  const long w = blockIdx.z;
+  int x = blockIdx.x;
+  if (x == a.s[0].nx + a.s[1].nx) {
+    if (blockIdx.y > 0) return;
+    double er = 0.0, ei = 0.0;
+    for (int s = 0; s < a.nsets; ++s) {
+      const int n = a.s[s].O * N;
+      const double2* g = a.s[s].green + w * n;
+      for (int e = threadIdx.x; e < n; e += 64 * kThetaWaves) {
+        const double h = a.fac * a.s[s].rh1[e];
+        er += h * g[e].x;
+        ei += h * g[e].y;
+      }
+    }
+    er = wave_sum(er);
+    ei = wave_sum(ei);
+    if (lane == 0) red[wave] = double2{er, ei};
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double2 s = red[0];
+      for (int i = 1; i < kThetaWaves; ++i) {
+        s.x += red[i].x;
+        s.y += red[i].y;
+      }
+      a.ene1[w] = s;
+    }
+    return;
+  }
+  const bool second = x >= a.s[0].nx;
+  const ThetaSet& p = a.s[second ? 1 : 0];
+  if (second) x -= a.s[0].nx;
+  const int j0 = kThetaRows * blockIdx.y, k = 64 * x + lane, Nv = N - p.O;
+  if (j0 >= p.O) return;
+  const int rs = (N + kThetaWaves - 1) / kThetaWaves, r0 = min(N, wave * rs), r1 = min(N, r0 + rs);
+  const double* q = p.Q + min(k, Nv - 1);
+  const double2* g[kThetaRows];
+  double2 acc[kThetaRows];
+#pragma unroll
+  for (int j = 0; j < kThetaRows; ++j) {
+    g[j] = p.green + (w * p.O + min(j0 + j, p.O - 1)) * N;
+    acc[j] = double2{0.0, 0.0};
+  }
+#pragma unroll 8
+  for (int r = r0; r < r1; ++r) {
+    const double b = q[(long)r * Nv];
+#pragma unroll
+    for (int j = 0; j < kThetaRows; ++j) {
+      const double2 z = g[j][r];
+      acc[j].x += b * z.x;
+      acc[j].y += b * z.y;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kThetaRows; ++j) part[wave][j][lane] = acc[j];
+  __syncthreads();
+  static_assert(kThetaRows <= kThetaWaves, "a wave finishes a row");
+  const int j = j0 + wave;
+  double2 t = {0.0, 0.0};
+  if (wave < kThetaRows && k < Nv) {
+#pragma unroll
+    for (int i = 0; i < kThetaWaves; ++i) {
+      t.x += part[i][wave][lane].x;
+      t.y += part[i][wave][lane].y;
+    }
+  }
+  double sr = 0.0, si = 0.0;
+  if (wave < kThetaRows && j < p.O && k < 2 * p.npr) {
+    const long grp = w / p.wn;
+    double* o = reinterpret_cast<double*>(p.out) +
+                (((grp * p.npr + (k >> 1)) * 2 * p.C2 + 2 * ((w - grp * p.wn) * p.O + j)) * 2 + (k & 1));
+    o[0] = t.x;
+    o[2] = t.y;
+    if (k < Nv) {
+      const double m = p.mt[(long)j * Nv + k];
+      sr = m * t.x;
+      si = m * t.y;
+    }
+  }
+  sr = wave_sum(sr);
+  si = wave_sum(si);
+  if (lane == 0) red[wave] = double2{sr, si};
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double2 s = {0.0, 0.0};
+    for (int i = 0; i < kThetaRows; ++i) {
+      s.x += red[i].x;
+      s.y += red[i].y;
+    }
+    const int slot = blockIdx.y * p.nx + x;
+    p.kpart[w * p.kstride + p.nchunk + slot] = double2{2.0 * s.x + (slot == 0 ? *p.k0 : 0.0), 2.0 * s.y};
+  }
 }
 
 // kpart[w][nchunk] = K0 + 2 sum_ja M_ja theta_w,aj
@@ -649,6 +767,13 @@ int launch(const ExF64& p, long grid, hipStream_t st) {
 
 }  // namespace
 
+// Few walkers: up to what theta_kernel reads of Q, each walker anew.  An energy with
+// a product, a packing and a sum for theta, and with theta_kernel, at G = 400:
+// N = 80, O = 20, 1 walker (0.2 MB) 75 and 58 us; N = 100, O = 20, 64 (20 MB) 187
+// and 164, 512 (164 MB) 952 and 951; N = 200, O = 40, 128 (328 MB) 1233 and 1229,
+// 256 (655 MB) 2344 and 2371.
+constexpr double kFewBytes = 250.0e6;
+
 // The tile: gw g's in 16 MB WR rows and wn walkers in 16 NB WC columns, chosen
 // for the least padding.  One wave column up to O = 64 (all 2 O columns of a
 // walker in one wave's 8 blocks); above, a whole f block takes eight waves.
@@ -682,6 +807,55 @@ ExF64Tile exchange_f64_tile(int O) {
   return best;
 }
 
+// Few walkers leave most of the tile's columns, or of the CUs, idle: then the
+// widest of the narrower tiles that fills both, or else the narrowest (an energy at
+// N = 60, O = 12, G = 144, 4 walkers 42 -> 35 us; N = 96, O = 16, G = 400, 4 walkers
+// 62 -> 50).
+ExF64Tile exchange_f64_tile(int O, int W, int G) {
+  ExF64Tile t = exchange_f64_tile(O);
+  const long nchunk = exchange_f64_nchunk(O, G);
+  for (int nb = 4; nb >= 2; --nb) {
+    const bool full = W >= t.wn && nchunk * ((W + t.wn - 1) / t.wn) >= 256;
+    if (full || t.WC > 1 || 16 * nb < 2 * O) break;
+    t.NB = nb;
+    t.wn = 16 * nb / (2 * O);
+  }
+  return t;
+}
+
+long exchange_f64_most_few(int O, int N) {
+  if (N <= O) return 0;
+  const double bytes = 8.0 * N * (N - O) * ((O + kThetaRows - 1) / kThetaRows);
+  return (long)std::min(65535.0, kFewBytes / bytes);
+}
+bool exchange_f64_few(int O, int N, int W) { return W <= exchange_f64_most_few(O, N); }
+static int theta_blocks(int O, int N) { return (2 * exchange_f64_npairs(N - O) + 63) / 64; }
+int exchange_f64_slots(int O, int N, int G) {
+  return exchange_f64_nchunk(O, G) + std::max(1, (O + kThetaRows - 1) / kThetaRows * theta_blocks(O, N));
+}
+
+int exchange_f64_theta(const ExTheta* sets, int nsets, int N, int G, int W, double fac, double2* ene1,
+                       hipStream_t st) {
+  if (nsets < 1) return AFQ_OK;
+  ThetaArgs a{};
+  int rows = 0;
+  for (int i = 0; i < nsets; ++i) {
+    const ExTheta& x = sets[i];
+    const ExF64Tile t = exchange_f64_tile(x.O, W, G);
+    a.s[i] = ThetaSet{x.green, x.Q, x.mt, x.k0, x.rh1, x.O, theta_blocks(x.O, N), t.wn, 8 * t.NB * t.WC,
+                      exchange_f64_npairs(N - x.O), exchange_f64_nchunk(x.O, G), exchange_f64_slots(x.O, N, G),
+                      x.thetap, x.kpart};
+    rows = std::max(rows, x.O);
+  }
+  a.nsets = nsets;
+  a.N = N;
+  a.fac = fac;
+  a.ene1 = ene1;
+  const dim3 grid(a.s[0].nx + a.s[1].nx + (ene1 ? 1 : 0), (rows + kThetaRows - 1) / kThetaRows, W);
+  hipLaunchKernelGGL(theta_kernel, grid, dim3(64 * kThetaWaves), 0, st, a);
+  return launch_status("theta_kernel");
+}
+
 int exchange_f64_nchunk(int O, int G) {
   const ExF64Tile t = exchange_f64_tile(O);
   return (G + t.gw - 1) / t.gw;
@@ -689,7 +863,18 @@ int exchange_f64_nchunk(int O, int G) {
 
 int exchange_f64_npairs(int Nv) { return ((Nv + 7) / 8 + kSteps - 1) / kSteps * kPairs; }
 
-long exchange_f64_b_elems(int O, int N, int W) { return exchange_thetap_elems(exchange_f64_tile(O), N - O, W); }
+// For up to W walkers: the widest tile, and the narrower ones up to the walkers
+// (256 work-groups of the widest, at most) that take them.
+long exchange_f64_b_elems(int O, int N, int W) {
+  ExF64Tile t = exchange_f64_tile(O);
+  long n = exchange_thetap_elems(t, N - O, W);
+  const int few = std::min(W, 256 * t.wn);
+  for (t.NB = 4; t.WC == 1 && t.NB >= 2 && 16 * t.NB >= 2 * O; --t.NB) {
+    t.wn = 16 * t.NB / (2 * O);
+    n = std::max(n, exchange_thetap_elems(t, N - O, few));
+  }
+  return n;
+}
 
 long exchange_f64_a_elems(int O, int N, int G) {
   const ExF64Tile t = exchange_f64_tile(O);
@@ -861,7 +1046,7 @@ int k_exchange_f64(const double* a, const double* Q, const double* c0, const dou
                    const double2* green, double2* theta, double2* thetap, int O, int N, int G, int W, double2* coul,
                    double2* kpart, int* nch_out, hipStream_t st) {
   if (O < 1 || O > kExchangeF64MaxO) return fail(AFQ_E_UNSUPPORTED, "exchange kernel supports 1 <= nocc <= 128");
-  const ExF64Tile t = exchange_f64_tile(O);
+  const ExF64Tile t = exchange_f64_tile(O, W, G);
   ExF64 p;
   p.a = a;
   p.theta = thetap;
@@ -886,7 +1071,9 @@ int k_exchange_f64(const double* a, const double* Q, const double* c0, const dou
     p.strip = (int)((room - 2 * O) / (ld + 2 * O));
   }
   p.lds_elems = p.strip < O ? p.strip * ld + O * (2L * p.strip + 2) : p.gp * O * ld;
-  *nch_out = p.nchunk + 1;
+  const int nslab = (p.n8 + kSteps - 1) / kSteps;
+  p.kstride = exchange_f64_few(O, N, W) ? exchange_f64_slots(O, N, G) : p.nchunk + 1;
+  *nch_out = p.kstride;
   if (green && p.Nv > 0) {
     // theta^T: the rows (w, j) of all walkers' G times Q
     Gemm g;
@@ -901,7 +1088,6 @@ int k_exchange_f64(const double* a, const double* Q, const double* c0, const dou
     g.C = theta;
     g.ldc = p.Nv;
     AFQ_TRY(gemm_f64(g, st));
-    const int nslab = (p.n8 + kSteps - 1) / kSteps;
     const long n = (long)p.nwg * nslab * kPairs * 8 * t.NB * t.WC;
     hipLaunchKernelGGL(pack_b_kernel, dim3(blocks(n)), dim3(256), 0, st, theta, O, p.Nv, t.wn, W, 8 * t.NB * t.WC,
                        nslab, n, thetap);
@@ -924,6 +1110,12 @@ int k_exchange_f64(const double* a, const double* Q, const double* c0, const dou
   EXF64(2, 7, 4, 1);
   EXF64(2, 6, 4, 1);
   EXF64(2, 5, 4, 1);
+  EXF64(2, 4, 4, 1);
+  EXF64(2, 3, 4, 1);
+  EXF64(2, 2, 4, 1);
+  EXF64(3, 2, 4, 1);
+  EXF64(3, 3, 4, 1);
+  EXF64(3, 4, 4, 1);
   EXF64(3, 5, 4, 1);
   EXF64(3, 6, 4, 1);
   EXF64(2, 7, 8, 1);

@@ -50,7 +50,7 @@ struct SmallMeasure {
   const double* q[2];
   const double* mt[2];
   const double* k0[2];
-  double2* thetap[2];
+  double2* thetap[2];     // null: left to the exchange (exchange_f64_few)
   double2* kpart[2];
   int wn[2], c2[2], npr[2], nchunk[2];
   // or, with `whole`, the exchange and the energy here (small_energy_whole)
@@ -73,7 +73,7 @@ int k_small_pack_rc(const double* rc0, int n0, const double* rc1, int n1, int G,
 // LDS bytes of a step's and of a measurement's work-group; 0 if the sizes are
 // past the limits.
 size_t small_step_lds(int N, int G, int c, int osum, int nbuf);
-size_t small_measure_lds(int N, int c, int osum);
+size_t small_measure_lds(int N, int c, int osum, int nspin);
 // Whether a phaseless step of W walkers is better off in one work-group per
 // walker, which reads L and rot_chol for every walker, than in batched products.
 bool small_step_pays(int N, int G, int osum, int W, bool sym);

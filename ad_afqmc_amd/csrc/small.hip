@@ -661,6 +661,10 @@ __global__ __launch_bounds__(kMeasureThreads) void small_measure_kernel(SmallMea
     }
     // theta_w (columns j) = Q^T G_w^T in the exchange's packed layout, zero
     // past Nv, and the walker's part of K that is linear in it
+    if (!p.thetap[s]) {
+      Gm += n;
+      continue;
+    }
     const int grp = (int)(w / p.wn[s]), wl = (int)(w - (long)grp * p.wn[s]), np2 = 2 * p.npr[s];
     double* out = reinterpret_cast<double*>(p.thetap[s]);
     double2 kk = {0.0, 0.0};
@@ -753,13 +757,15 @@ bool small_energy_whole(int N, int G, int occ0, int occ1) {
   return (long)G * N * (occ0 * occ0 + occ1 * occ1) <= 50000;
 }
 
-// Past N osum = 1536 a work-group's theta product takes about as long as the
-// launches it saves (N = 96, O = 16, G = 300, 64 walkers: 118 us an energy
-// against 185 before, with the batched products for theta and the rest 152 at
-// N = 100, O = 20, 50 walkers).
-size_t small_measure_lds(int N, int c, int osum) {
+// One spin up to N osum = 1536, two spins, which save twice the launches, to 2400
+// (the LDS): an energy here and by separate launches, N = 120, O = 16, G = 400,
+// N osum = 1920: 1 walker 56 and 54 us, 32 walkers 107 and 103, 2048 walkers 3.08
+// and 2.73 ms; UHF N = 60, O = 14 / 13, G = 300, 1620: 52 and 68 us, 76 and 79, 1.42
+// and 1.52 ms; UHF N = 76, O = 16 / 15, G = 400, 2356: 55 and 68, 125 and 123, 4.12
+// and 4.17.
+size_t small_measure_lds(int N, int c, int osum, int nspin) {
   const size_t bytes = sizeof(double2) * (size_t)N * (c + osum) + sizeof(double) * (size_t)N * osum;
-  return N * osum <= 1536 && bytes <= kMeasureLds ? bytes : 0;
+  return N * osum <= (nspin > 1 ? 2400 : 1536) && bytes <= kMeasureLds ? bytes : 0;
 }
 
 long small_l_pairs(int N, bool sym) { return (vhs_entries(N, sym) + 1) / 2; }
@@ -808,7 +814,7 @@ int k_small_weights(const double* h, int nsteps, int W, double dt, double* weigh
 }
 
 int k_small_measure(const SmallMeasure& p, hipStream_t st) {
-  const size_t bytes = small_measure_lds(p.b.N, p.b.c, osum_of(p.b));
+  const size_t bytes = small_measure_lds(p.b.N, p.b.c, osum_of(p.b), p.b.nspin);
   if (bytes == 0) return fail(AFQ_E_UNSUPPORTED, "small measurement: sizes past the limits");
   static std::atomic<bool> raised{false};
   AFQ_TRY(raise_lds(reinterpret_cast<const void*>(small_measure_kernel), kMeasureLds, raised, "small measurement"));
