@@ -56,7 +56,10 @@ __device__ inline double2 crecip(double2 a) {
 // 30 -> 20 us; n=40, 512 57 -> 43; n=60 and 58, 2 x 256 84 -> 73; n=100, 40
 // matrices 210 -> 156 (950 in place in global memory, with a barrier and a round
 // trip to L2 for each column); n=82, 48 177 -> 127 (800).  The same steps as a
-// loop, one column after another through the registers, were 3-15% slower.
+// loop, one column after another through the registers, were 3-15% slower.  Up to
+// n = 16 a work-group is the two waves that have columns: with eight, a CU holds a
+// quarter of the matrices (overlaps of 2048 walkers, N=130, n=16: 106 us, and 97 in
+// panels of 16; 63 so).
 //
 // n > 128 (gj_det_inv_body, n <= 256): the matrix is factored in global memory,
 // in the inverse's buffer or the set's scratch (it stays in L2), with explicit
@@ -69,19 +72,22 @@ __device__ inline double2 crecip(double2 a) {
 // trailing rows and columns are eliminated (the pivots, hence the determinant,
 // are the same).  NMAX = kDetInvMaxN; each thread covers NMAX / 64 columns
 // (and pivot-search rows); n <= 64 matrices of such a launch use dynamic LDS.
-constexpr int kLdsN = 64;   // largest n of one register row a lane (and of the LDS Cholesky)
+constexpr int kTwoN = 16;    // largest n of two waves
+constexpr int kLdsN = 64;    // largest n of one register row a lane (and of the LDS Cholesky)
 constexpr int kReg2N = 128;  // largest n of two register rows a lane
 constexpr int kPanel = 8;    // columns of a wave
-constexpr size_t reg_lds(int h, int nmax) {
-  const size_t work = sizeof(double2) * h * 64 * (2 * kPanel + kPanel);
+constexpr size_t reg_lds(int h, int nw, int nmax) {
+  const size_t work = sizeof(double2) * (2 * kPanel * 64 * h + nw * kPanel * kPanel);
   return h == 1 ? std::max(work, sizeof(double2) * nmax * (nmax | 1)) : work;
 }
-constexpr int det_inv_threads(int nmax) { return nmax == kLdsN ? 512 : nmax == kReg2N ? 1024 : 256; }
+constexpr int det_inv_threads(int nmax) {
+  return nmax == kTwoN ? 128 : nmax == kLdsN ? 512 : nmax == kReg2N ? 1024 : 256;
+}
 
-// H rows a lane (n <= 64 H).  lds: reg_lds(H, n) bytes.
-template <int H>
+// H rows a lane, NW waves (n <= 64 H, 8 NW).  lds: reg_lds(H, NW, n) bytes.
+template <int H, int NW>
 __device__ __forceinline__ void gj_reg_body(const DetInvSet& set, long b, double2* __restrict__ lds) {
-  constexpr int ROWS = 64 * H, NW = ROWS / kPanel, NT = 64 * NW;
+  constexpr int ROWS = 64 * H, NT = 64 * NW;
   double2(*ubuf)[kPanel][ROWS] = reinterpret_cast<double2(*)[kPanel][ROWS]>(lds);  // [2]: U[t][row], by panel parity
   // [NW]: per wave, [column][t] of the panel's pivot rows before the panel
   double2(*prow)[kPanel][kPanel] = reinterpret_cast<double2(*)[kPanel][kPanel]>(lds + 2 * kPanel * ROWS);
@@ -348,10 +354,12 @@ __device__ __forceinline__ void gj_det_inv_body(const DetInvSet& set, long b, do
 template <int NMAX>
 __global__ __launch_bounds__(det_inv_threads(NMAX)) void gj_det_inv_kernel(DetInvSet s0, DetInvSet s1) {
   extern __shared__ double2 lds_gj[];
-  if constexpr (NMAX == kLdsN)
-    gj_reg_body<1>(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
+  if constexpr (NMAX == kTwoN)
+    gj_reg_body<1, 2>(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
+  else if constexpr (NMAX == kLdsN)
+    gj_reg_body<1, 8>(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
   else if constexpr (NMAX == kReg2N)
-    gj_reg_body<2>(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
+    gj_reg_body<2, 16>(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
   else
     gj_det_inv_body<NMAX>(blockIdx.y == 0 ? s0 : s1, blockIdx.x, lds_gj);
 }
@@ -364,10 +372,12 @@ __global__ __launch_bounds__(det_inv_threads(NMAX)) void gj_det_inv_grouped_kern
   const int item = blockIdx.x;
   const int j = group_find(prefix, njobs, item);
   const DetInvSet set = sets[j];
-  if constexpr (NMAX == kLdsN)
-    gj_reg_body<1>(set, item - prefix[j], lds_gj);
+  if constexpr (NMAX == kTwoN)
+    gj_reg_body<1, 2>(set, item - prefix[j], lds_gj);
+  else if constexpr (NMAX == kLdsN)
+    gj_reg_body<1, 8>(set, item - prefix[j], lds_gj);
   else if constexpr (NMAX == kReg2N)
-    gj_reg_body<2>(set, item - prefix[j], lds_gj);
+    gj_reg_body<2, 16>(set, item - prefix[j], lds_gj);
   else
     gj_det_inv_body<NMAX>(set, item - prefix[j], lds_gj);
 }
@@ -581,8 +591,9 @@ int batched_det_inv_sets(const DetInvSet* sets, int nsets, int count, hipStream_
   }
   if (count <= 0) return AFQ_OK;
   // n <= 128: the matrices stay in registers
-  return nmax <= kLdsN    ? launch_det_inv<kLdsN>(sets, nsets, count, reg_lds(1, nmax), stream)
-         : nmax <= kReg2N ? launch_det_inv<kReg2N>(sets, nsets, count, reg_lds(2, nmax), stream)
+  return nmax <= kTwoN    ? launch_det_inv<kTwoN>(sets, nsets, count, reg_lds(1, 2, nmax), stream)
+         : nmax <= kLdsN  ? launch_det_inv<kLdsN>(sets, nsets, count, reg_lds(1, 8, nmax), stream)
+         : nmax <= kReg2N ? launch_det_inv<kReg2N>(sets, nsets, count, reg_lds(2, 16, nmax), stream)
                           : launch_det_inv<kDetInvMaxN>(sets, nsets, count, matrix_lds_bytes(nmax), stream);
 }
 
@@ -599,8 +610,9 @@ int det_inv_grouped(const GroupTab<DetInvSet>& t, int nmax, hipStream_t stream) 
   if (t.njobs < 1 || t.total < 1) return AFQ_OK;
   if (nmax < 1 || nmax > kDetInvMaxN)
     return fail(AFQ_E_UNSUPPORTED, "det/inverse kernel supports 1 <= n <= " + std::to_string(kDetInvMaxN));
-  return nmax <= kLdsN    ? launch_det_inv_grouped<kLdsN>(t, reg_lds(1, nmax), stream)
-         : nmax <= kReg2N ? launch_det_inv_grouped<kReg2N>(t, reg_lds(2, nmax), stream)
+  return nmax <= kTwoN    ? launch_det_inv_grouped<kTwoN>(t, reg_lds(1, 2, nmax), stream)
+         : nmax <= kLdsN  ? launch_det_inv_grouped<kLdsN>(t, reg_lds(1, 8, nmax), stream)
+         : nmax <= kReg2N ? launch_det_inv_grouped<kReg2N>(t, reg_lds(2, 16, nmax), stream)
                           : launch_det_inv_grouped<kDetInvMaxN>(t, matrix_lds_bytes(nmax), stream);
 }
 
