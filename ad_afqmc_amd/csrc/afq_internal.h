@@ -131,8 +131,8 @@ int gemm_lp(LpKind kind, bool bf16x3, const Gemm& g, hipStream_t stream);
 // ---------------------------------------------------------------- small dense linear algebra
 // In-place Gauss-Jordan with partial pivoting (|re|+|im| pivot metric, first
 // maximum wins, as LAPACK's izamax) on `count` n x n complex matrices.  Writes
-// det (count,) and, if inv != nullptr, the inverse.  n <= 256: up to n = 64
-// the matrix is factored in LDS, above in global memory (in inv itself).
+// det (count,) and, if inv != nullptr, the inverse.  n <= 256: up to n = 128
+// the matrix is factored in registers, above in global memory (in inv itself).
 int batched_det_inv(const double2* S, long strideS, int n, int count, double2* det, double2* inv, long strideInv,
                     hipStream_t stream);
 // One launch over one or two sets of `count` matrices each (e.g. both spins).
@@ -143,7 +143,8 @@ struct DetInvSet {
   double2* det;
   double2* inv;  // nullptr: determinant only
   long strideInv;
-  // n > 64 without an inverse: global scratch of n x n per matrix, matrix
+  // n > 64 without an inverse (a launch with a set above 128 factors those in
+  // global memory too): global scratch of n x n per matrix, matrix
   // stride strideS (S itself may be given: it is then overwritten)
   double2* work = nullptr;
 };

@@ -117,7 +117,7 @@ int green_pipeline(afq_job* j, const void* up, const void* dn, bool want_inv, bo
       g.C = j->S[s];
       g.ldc = O;
       g.sC = (long)O * O;
-      // above n = 64 a determinant alone is factored in place in S
+      // S is the scratch of a determinant alone where that is factored in global memory
       sets[s] = DetInvSet{j->S[s], (long)O * O, O, j->det[s], want_inv ? j->Sinv[s] : nullptr, (long)O * O, j->S[s]};
     }
     {

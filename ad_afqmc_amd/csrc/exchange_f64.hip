@@ -781,6 +781,12 @@ constexpr double kFewBytes = 250.0e6;
 // on four waves with three work-groups a CU 12.2, with two 13.0; 3 x 5 on eight
 // waves 12.3; 1 x 5 on eight 12.8; 3 x 5 on four 13.6.  At O = 60: 2 x 8 on four
 // waves 67.2, 1 x 8 on eight 66.7, 2 x 8 on eight 68.5, 1 x 8 on four 74.0.
+// O = 49 to 51: five g's in the 256 rows of eight waves (N = 250, G = 600, 128
+// walkers 3.27 ms at O = 51, 3.95 with two in 128 rows).
+// Share of the tile that is not padding: O <= 25 0.84 or more; 26 0.75, rising to 1
+// at 32; 33 0.71, 38 0.94, 40 0.94, 43 0.80, 48 1; 49 0.84, 52 0.75, 57 0.79, 64 1;
+// above, where a tile holds one f block, 65 0.46, 82 0.73, 96 1, 97 0.57, 112 0.77,
+// 128 1.
 ExF64Tile exchange_f64_tile(int O) {
   ExF64Tile best{};
   double top = -1.0;
@@ -798,10 +804,9 @@ ExF64Tile exchange_f64_tile(int O) {
     for (int nb = 8; nb >= 5; --nb) consider(2, nb, 4, 1);
     consider(3, 5, 4, 1);
     consider(3, 6, 4, 1);
-    if (O > 48 && O < 54) consider(2, 7, 8, 1);
+    if (O > 48 && O <= 51) consider(2, 7, 8, 1);
   } else {
     consider(3, 3, 2, 4);
-    consider(4, 3, 2, 4);
     consider(4, 4, 2, 4);
   }
   return best;
@@ -1120,7 +1125,6 @@ int k_exchange_f64(const double* a, const double* Q, const double* c0, const dou
   EXF64(3, 6, 4, 1);
   EXF64(2, 7, 8, 1);
   EXF64(3, 3, 2, 4);
-  EXF64(4, 3, 2, 4);
   EXF64(4, 4, 2, 4);
 #undef EXF64
   return fail(AFQ_E_UNSUPPORTED, "exchange: no tile for this nocc");

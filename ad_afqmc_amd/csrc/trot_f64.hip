@@ -301,12 +301,12 @@ int trot_f64(const TrotF64& f, hipStream_t st) {
   const long grid = 8L * ((f.W + 7) / 8) * S;
   if (grid > 0x7fffffffL) return fail(AFQ_E_UNSUPPORTED, "fused FP64 propagator: grid too large");
   const size_t bytes = 16L * a.R * 16 * NB * 8;
-  const int XB = ((a.R % NWAVE % 4) * NB + NWAVE - 1) / NWAVE;  // 0, 1 or 2
-#define TROT(mb, nb)                                                      \
-  if (MB == mb && NB == nb)                                               \
-  return XB == 0   ? launch<mb, nb, 0>(a, grid, bytes, st)                \
-         : XB == 1 ? launch<mb, nb, 1>(a, grid, bytes, st)                \
-                   : launch<mb, nb, 2>(a, grid, bytes, st)
+  const int XB = ((a.R % NWAVE % 4) * NB + NWAVE - 1) / NWAVE;  // 0, 1 or, from NB = 3, 2
+#define TROT(mb, nb)                                       \
+  if (MB == mb && NB == nb)                                \
+  return XB == 0   ? launch<mb, nb, 0>(a, grid, bytes, st) \
+         : XB == 1 ? launch<mb, nb, 1>(a, grid, bytes, st) \
+                   : launch<mb, nb, (nb > 2 ? 2 : 1)>(a, grid, bytes, st)
   TROT(1, 1);
   TROT(1, 2);
   TROT(1, 3);
