@@ -21,6 +21,7 @@ CASES = [(110, 16, 0, 9, 5, 1), (110, 16, 0, 9, 5, 3), (110, 16, 15, 70, 9, 5), 
          (61, 20, 17, 13, 7, 2), (80, 25, 19, 6, 6, 1), (80, 32, 31, 9, 4, 2), (90, 40, 33, 7, 3, 3),
          (130, 64, 65, 3, 2, 2), (140, 97, 1, 3, 2, 1), (48, 16, 16, 60, 40, 7), (60, 12, 11, 50, 3, 2),
          (37, 9, 7, 300, 30, 30), (30, 17, 0, 2, 700, 700), (17, 17, 17, 5, 3, 2), (66, 66, 0, 3, 2, 2),
+         (140, 12, 0, 33, 180, 180),
          # past the few
          (300, 60, 58, 3, 34, 33), (260, 97, 0, 2, 33, 31), (250, 33, 20, 3, 160, 65), (250, 34, 33, 2, 71, 70),
          (76, 16, 15, 9, 3, 3), (75, 16, 16, 9, 3, 2), (150, 16, 0, 9, 3, 2)]
