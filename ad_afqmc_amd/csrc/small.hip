@@ -785,13 +785,22 @@ int k_small_pack_rc(const double* rc0, int n0, const double* rc1, int n1, int G,
   return launch_status("pack_rc_kernel");
 }
 
-// The bytes of L and rot_chol a CU reads for its walkers against the launches
-// saved: at 2.1 MB a CU (UHF N = 40, O = 10, G = 160, 300 walkers) 251 us against
-// 262 as separate launches, at 2.2 MB (N = 48, O = 16 / 16, G = 160) 241 against
-// 240, at 0.6 MB (N = 48, O = 5, G = 135) 65 against 150.
+// The bytes of L and rot_chol a CU reads for its walkers (work-groups over 256 CUs)
+// against the launches saved.  Where L is packed (sym), the launches are those of the
+// fused propagator, and the line lies at about 2.5 MB a CU (UHF, separate and here):
+//   N = 48, O = 9 / 9:    G = 60, 256 walkers (1.0 MB) 116 / 81 us; 512 (2.0) 155 / 147;
+//                         1024 (3.9) 255 / 278; G = 115, 257 (3.8) 161 / 158;
+//   N = 48, O = 16 / 16:  G = 115, 4 walkers (2.5 MB) 106 / 117, 256 149 / 125, 257
+//                         (5.0) 197 / 228; G = 160, 64 (3.5) 130 / 129, 512 (6.9) 216 / 250.
+// Where it is not, each product is a launch of the general kernel, and it lies near
+// 10 MB:
+//   N = 20, O = 6 / 6:    G = 450, 256 walkers (2.3 MB) 183 / 75, 1024 (9.2) 261 / 165;
+//   N = 30, O = 8 / 8:    G = 300, 256 (3.3) 168 / 88; G = 450, 257 (9.9) 198 / 195;
+//                         G = 300, 1024 (13.2) 278 / 299;
+//   N = 40, O = 10 / 10:  G = 300, 256 (5.8) 209 / 124; G = 300, 257 (11.5) 234 / 229.
 bool small_step_pays(int N, int G, int osum, int W, bool sym) {
   const double bytes = 8.0 * G * (vhs_entries(N, sym) + N * osum);
-  return bytes * ((W + 255) / 256) <= 2.5e6;
+  return bytes * ((W + 255) / 256) <= (sym ? 2.5e6 : 9.5e6);
 }
 
 int k_small_step(const SmallStep& p, hipStream_t st) {
