@@ -40,9 +40,11 @@ PEAKS = {  # MI355X published dense peaks
 }
 
 
-def flops_per_walker_step(N, Oa, Ob, G, m, one_spin, K=5):
+def flops_per_walker_step(N, Oa, Ob, G, m, one_spin, K=5, exchange_virtual=False):
     """Algorithmic real flops per walker-step (complex x real MAC = 4, complex x
-    complex MAC = 8), with the measurement (QR + energy) amortised over m steps."""
+    complex MAC = 8), with the measurement (QR + energy) amortised over m steps;
+    exchange_virtual: the FP64 exchange, which contracts over the N - O orbitals
+    that the trial leaves empty and not over all N."""
     occ = [Oa] if one_spin else [Oa, Ob]
     sumO = sum(occ)
     f = {}
@@ -53,7 +55,7 @@ def flops_per_walker_step(N, Oa, Ob, G, m, one_spin, K=5):
     f["green_fb"] = green
     f["force_bias"] = 4.0 * G * N * sumO
     f["overlap"] = sum(4.0 * o * o * N + 8.0 / 3.0 * o**3 for o in occ)
-    f["energy"] = (sum(4.0 * G * o * o * N + 8.0 * G * o * o for o in occ) + green) / m
+    f["energy"] = (sum(4.0 * G * o * o * (N - o if exchange_virtual else N) + 8.0 * G * o * o for o in occ) + green) / m
     f["qr"] = sum(8.0 * (2.0 * N * o * o - 2.0 / 3.0 * o**3) for o in occ) / m
     return sum(f.values()), f
 
@@ -65,7 +67,7 @@ def whole_step_roofline(N, Oa, Ob, G, m, one_spin, precision, value):
     the VHS, Taylor, force-bias and energy contractions run reduced; exp(-dt/2
     h1) runs on FP32 (on FP64 at 33..48 walker columns); the Green's function,
     overlap and QR stay FP64."""
-    f_total, f = flops_per_walker_step(N, Oa, Ob, G, m, one_spin)
+    f_total, f = flops_per_walker_step(N, Oa, Ob, G, m, one_spin, exchange_virtual=precision == "fp64")
     red = {"fp64": PEAKS["fp64"], "fp32": PEAKS["fp32"], "bf16x3": PEAKS["bf16"] / 3.0}[precision]
     cols = Oa if one_spin else Oa  # exp(-dt/2 h1) runs per spin buffer
     peaks = {"vhs": red, "taylor": red, "force_bias": red, "energy": red,
@@ -105,8 +107,8 @@ def launch_flops(cls, N, Oa, Ob, G, W, unrestricted=False, vhs_cols=None, exchan
     """Flops of one launch of a kernel class, as the kernel computes them,
     averaged over the launches of a block: the VHS product covers `vhs_cols`
     columns (N^2 by default); the FP64 exchange (`exchange_virtual`) contracts
-    over the N - O orbitals that the trial leaves empty; a Taylor launch covers the walker panel (both
-    spins' columns side by side for unrestricted walkers); the one-body,
+    over the N - O orbitals that the trial leaves empty; a Taylor launch covers
+    the walker panel (both spins' columns side by side for unrestricted walkers); the one-body,
     exchange, force-bias, Green's-function and overlap launches alternate
     between the spins of an unrestricted or UHF case."""
     occ = (Oa, Ob) if (unrestricted or Oa != Ob) else (Oa,)
@@ -783,7 +785,7 @@ def main():
     r["precision"] = args.precision
     value, elapsed, blocks = r["value"], r["elapsed"], r["blocks"]
     finite = bool(np.all(np.isfinite(blocks)))
-    f_total, _ = flops_per_walker_step(N, Oa, Ob, G, nsteps, not uhf)
+    f_total, _ = flops_per_walker_step(N, Oa, Ob, G, nsteps, not uhf, exchange_virtual=args.precision == "fp64")
     line = {
         "metric": "walker-steps/s at <=0.1 mHa vs FP64 oracle; p50/p99 job latency under load",
         "value": value,
