@@ -41,11 +41,11 @@ inline int launch_status(const char* what) {
 }
 
 // Raises a kernel's dynamic LDS limit to `bytes`, the most that any launch of it
-// takes, at its first launch (`done`: one flag a kernel).  The limit is a state
-// of the kernel and not of the launch: set to each launch's own need, another
+// takes, at its first launch on a device (`done`: one word a kernel, a bit a
+// device).  The limit is a state of the kernel and not of the launch: set to each launch's own need, another
 // host thread's smaller launch could lower it between this one's raise and its
 // launch.
-int raise_lds(const void* kernel, size_t bytes, std::atomic<bool>& done, const char* what);
+int raise_lds(const void* kernel, size_t bytes, std::atomic<uint64_t>& done, const char* what);
 
 // ---------------------------------------------------------------- GEMM
 // Batched C[b] = alpha * opA(A[b]) * opB(B[b]) + beta * C[b]   (and D[b] += result

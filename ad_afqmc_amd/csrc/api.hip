@@ -23,11 +23,14 @@ int fail(int code, const std::string& m) {
   return code;
 }
 
-int raise_lds(const void* kernel, size_t bytes, std::atomic<bool>& done, const char* what) {
-  if (done.load(std::memory_order_acquire)) return AFQ_OK;
+int raise_lds(const void* kernel, size_t bytes, std::atomic<uint64_t>& done, const char* what) {
+  int dev = 0;
+  AFQ_HIP(hipGetDevice(&dev));
+  const uint64_t bit = 1ull << (dev & 63);
+  if (done.load(std::memory_order_acquire) & bit) return AFQ_OK;
   const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
   if (e != hipSuccess) return fail(AFQ_E_HIP, std::string(what) + " LDS attribute: " + hipGetErrorString(e));
-  done.store(true, std::memory_order_release);
+  done.fetch_or(bit, std::memory_order_release);
   return AFQ_OK;
 }
 }  // namespace afq

@@ -758,7 +758,7 @@ template <int MB, int NB, int WR, int WC>
 int launch(const ExF64& p, long grid, hipStream_t st) {
   constexpr size_t stage = sizeof(double2) * 2 * kPairs * 16 * NB * WC;
   const size_t bytes = std::max(stage, sizeof(double) * p.lds_elems);
-  static std::atomic<bool> raised{false};
+  static std::atomic<uint64_t> raised{0};
   AFQ_TRY(raise_lds(reinterpret_cast<const void*>(exchange_f64_kernel<MB, NB, WR, WC>),
                     std::max(stage, tile_room(MB, NB, WR * WC)), raised, "exchange"));
   hipLaunchKernelGGL((exchange_f64_kernel<MB, NB, WR, WC>), dim3((unsigned)grid), dim3(64 * WR * WC), bytes, st, p);
@@ -933,7 +933,7 @@ int exchange_f64_set_trial(const ExTrial* sets, int nsets, int N, double* tmp, h
   const size_t bytes = sizeof(double) * N * omax;
   constexpr size_t most = 152 * 1024;
   if (bytes <= most) {
-    static std::atomic<bool> raised{false};
+    static std::atomic<uint64_t> raised{0};
     AFQ_TRY(raise_lds(reinterpret_cast<const void*>(householder_kernel<true>), most, raised, "householder"));
     hipLaunchKernelGGL(householder_kernel<true>, dim3(1, nsets), dim3(1024), bytes, st, q, N);
   } else {

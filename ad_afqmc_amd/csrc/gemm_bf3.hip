@@ -335,7 +335,7 @@ int launch_lds(const Bf3& p, hipStream_t s) {
     if (items > 0x7fffffffL) return fail(AFQ_E_UNSUPPORTED, "gemm_bf3: grid too large");
   }
   const size_t lds = sizeof(__bf16) * 2 * (BMR + BN) * 64;
-  static std::atomic<bool> raised{false};
+  static std::atomic<uint64_t> raised{0};
   if (lds > 65536)
     AFQ_TRY(raise_lds(reinterpret_cast<const void*>(gemm_bf3_lds_kernel<BMR, BN, WM, WN>), lds, raised, "gemm_bf3"));
   hipLaunchKernelGGL((gemm_bf3_lds_kernel<BMR, BN, WM, WN>), dim3((unsigned)items, p.batch), dim3(64 * WM * WN), lds,
@@ -479,7 +479,7 @@ int reduce_f32_grouped(const GroupTab<ReduceJob>& t, hipStream_t s) {
 int gemm_bf3_grouped(const GroupTab<Bf3Job>& t, hipStream_t s) {
   if (t.njobs < 1 || t.total < 1) return AFQ_OK;
   const size_t lds = sizeof(__bf16) * 2 * (128 + 128) * 64;
-  static std::atomic<bool> raised{false};
+  static std::atomic<uint64_t> raised{0};
   if (lds > 65536)
     AFQ_TRY(raise_lds(reinterpret_cast<const void*>(gemm_bf3_grouped_kernel), lds, raised, "gemm_bf3"));
   hipLaunchKernelGGL(gemm_bf3_grouped_kernel, dim3((unsigned)t.total), dim3(512), lds, s, t.params, t.prefix,

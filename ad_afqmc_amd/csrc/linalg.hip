@@ -575,7 +575,7 @@ static int check_det_inv_set(const DetInvSet& s) {
 
 template <int NMAX>
 static int launch_det_inv(const DetInvSet* sets, int nsets, int count, size_t lds, hipStream_t stream) {
-  static std::atomic<bool> raised{false};
+  static std::atomic<uint64_t> raised{0};
   AFQ_TRY(raise_lds(reinterpret_cast<const void*>(gj_det_inv_kernel<NMAX>), kLdsMax, raised, "det/inverse"));
   hipLaunchKernelGGL(gj_det_inv_kernel<NMAX>, dim3(count, nsets), dim3(det_inv_threads(NMAX)), lds, stream, sets[0],
                      sets[nsets > 1 ? 1 : 0]);
@@ -599,7 +599,7 @@ int batched_det_inv_sets(const DetInvSet* sets, int nsets, int count, hipStream_
 
 template <int NMAX>
 static int launch_det_inv_grouped(const GroupTab<DetInvSet>& t, size_t lds, hipStream_t stream) {
-  static std::atomic<bool> raised{false};
+  static std::atomic<uint64_t> raised{0};
   AFQ_TRY(raise_lds(reinterpret_cast<const void*>(gj_det_inv_grouped_kernel<NMAX>), kLdsMax, raised, "det/inverse"));
   hipLaunchKernelGGL(gj_det_inv_grouped_kernel<NMAX>, dim3((unsigned)t.total), dim3(det_inv_threads(NMAX)), lds, stream, t.params,
                      t.prefix, t.njobs);
@@ -624,7 +624,7 @@ int batched_det_inv(const double2* S, long strideS, int n, int count, double2* d
 
 template <int NMAX>
 static int launch_cholesky(const CholSet* sets, int nsets, int count, size_t lds, hipStream_t stream) {
-  static std::atomic<bool> raised{false};
+  static std::atomic<uint64_t> raised{0};
   AFQ_TRY(raise_lds(reinterpret_cast<const void*>(cholesky_upper_kernel<NMAX>), kLdsMax, raised, "Cholesky"));
   hipLaunchKernelGGL(cholesky_upper_kernel<NMAX>, dim3(count, nsets), dim3(256), lds, stream, sets[0],
                      sets[nsets > 1 ? 1 : 0]);
@@ -653,7 +653,7 @@ int batched_cholesky_upper(const double2* S, long strideS, int n, int count, dou
 
 template <int NMAX>
 static int launch_cholesky_grouped(const GroupTab<CholSet>& t, size_t lds, hipStream_t stream) {
-  static std::atomic<bool> raised{false};
+  static std::atomic<uint64_t> raised{0};
   AFQ_TRY(raise_lds(reinterpret_cast<const void*>(cholesky_grouped_kernel<NMAX>), kLdsMax, raised, "Cholesky"));
   hipLaunchKernelGGL(cholesky_grouped_kernel<NMAX>, dim3((unsigned)t.total), dim3(256), lds, stream, t.params,
                      t.prefix, t.njobs);

@@ -733,7 +733,7 @@ int osum_of(const SmallJob& b) { return b.occ[0] + (b.nspin > 1 ? b.occ[1] : 0);
 
 template <int NT, int TR, int TPT, bool RES>
 int launch_step(const SmallStep& p, size_t bytes, hipStream_t st) {
-  static std::atomic<bool> raised{false};
+  static std::atomic<uint64_t> raised{0};
   AFQ_TRY(raise_lds(reinterpret_cast<const void*>(small_step_kernel<NT, TR, TPT, RES>),
                     RES ? kResidentLds : kStepLds, raised, "small step"));
   hipLaunchKernelGGL((small_step_kernel<NT, TR, TPT, RES>), dim3(p.b.W), dim3(NT), bytes, st, p);
@@ -825,7 +825,7 @@ int k_small_weights(const double* h, int nsteps, int W, double dt, double* weigh
 int k_small_measure(const SmallMeasure& p, hipStream_t st) {
   const size_t bytes = small_measure_lds(p.b.N, p.b.c, osum_of(p.b), p.b.nspin);
   if (bytes == 0) return fail(AFQ_E_UNSUPPORTED, "small measurement: sizes past the limits");
-  static std::atomic<bool> raised{false};
+  static std::atomic<uint64_t> raised{0};
   AFQ_TRY(raise_lds(reinterpret_cast<const void*>(small_measure_kernel), kMeasureLds, raised, "small measurement"));
   hipLaunchKernelGGL(small_measure_kernel, dim3(p.b.W), dim3(kMeasureThreads), bytes, st, p);
   return launch_status("small_measure_kernel");

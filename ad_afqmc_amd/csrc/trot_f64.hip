@@ -252,7 +252,7 @@ int simd_blocks(int R, int NB) {
 
 template <int MB, int NB, int XB>
 int launch(const TrotArgs& a, long grid, size_t bytes, hipStream_t st) {
-  static std::atomic<bool> raised{false};
+  static std::atomic<uint64_t> raised{0};
   AFQ_TRY(raise_lds(reinterpret_cast<const void*>(trot_f64_kernel<MB, NB, XB>), kLdsMax, raised, "propagator"));
   hipLaunchKernelGGL((trot_f64_kernel<MB, NB, XB>), dim3((unsigned)grid), dim3(NT), bytes, st, a);
   return launch_status("trot_f64_kernel");

@@ -68,3 +68,30 @@ def test_singular_overlap(o):
     ref = O.det_overlap(up, sysm.mo_up) ** 2
     assert ov[1] == 0.0
     assert np.max(np.abs(np.delete(ov, 1) - np.delete(ref, 1))) < 1e-10 * np.max(np.abs(ref))
+
+
+def test_group_of_small_jobs():
+    """A group none of whose jobs has more than 16 electrons a spin: one block by
+    one launch per kernel against each job's own block."""
+    from ad_afqmc_amd.engine import JobGroup
+    from ad_afqmc_amd.serving import GpuExecutor, JobSpec
+
+    print("[det/inverse small] group", flush=True)
+    specs = [JobSpec(job_id=i, norb=n, nocc=o, nchol=g, n_walkers=w, n_steps=10, seed=20 + i, precision="bf16x3")
+             for i, (n, o, g, w) in enumerate([(30, 6, 60, 33), (60, 16, 120, 17), (40, 9, 80, 20)])]
+    single, grouped = (GpuExecutor(n_prop_steps=5, use_graphs=False) for _ in range(2))
+    hs, hg = ([ex.start(s) for s in specs] for ex in (single, grouped))
+    group = JobGroup([(h["job"], h["up"], h["weights"], h["overlaps"], h["scalars"], h["counter"], h["out"],
+                       h["spec"].seed) for h in hg], 5)
+    for h in hs:
+        single._block(h)
+    group.sr_block()
+    torch.cuda.synchronize()
+    for a, b in zip(hs, hg):
+        for k in ("out", "weights", "overlaps", "up", "scalars"):
+            x, y = b[k].cpu().numpy(), a[k].cpu().numpy()
+            assert np.all(np.isfinite(x)) and np.max(np.abs(x - y)) < 1e-10 * np.max(np.abs(y))
+    group.close()
+    for ex, h in ((single, hs), (grouped, hg)):
+        for x in h:
+            ex.release(x)

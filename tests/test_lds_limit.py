@@ -1,6 +1,6 @@
 """A kernel's dynamic LDS limit is state of the process, not of a launch, and jobs
 may run from several host threads: it is raised in one place, once per kernel
-and to the most that any launch takes, never to one launch's own size."""
+and device and to the most that any launch takes, never to one launch's own size."""
 import glob
 import os
 import re
@@ -24,5 +24,5 @@ def test_every_raise_has_a_flag_of_its_own_launcher():
     for name, s in _sources().items():
         for m in re.finditer(r"AFQ_TRY\(raise_lds\(", s):
             n += 1
-            assert re.search(r"static std::atomic<bool> raised\{false\};\s*(?:if \([^;{}]*\)\s*)?$", s[:m.start()]), name
+            assert re.search(r"static std::atomic<uint64_t> raised\{0\};\s*(?:if \([^;{}]*\)\s*)?$", s[:m.start()]), name
     assert n >= 10
