@@ -1691,24 +1691,25 @@ int afq_sr_zeta(double* out, uint64_t seed, uint64_t counter, void* stream) {
 
 namespace afq {
 
-// Room for `need` fields, and the phaseless factors of as many steps.
+// Room for `need` fields, and the phaseless factors of as many steps: those first,
+// since the room for fields is what a later call is checked against.
 int reserve_fields(afq_job* j, long need, hipStream_t st) {
   const long hneed = j->h_step ? (need + j->G - 1) / j->G : 0;
   if (need <= j->fields_cap && hneed <= j->h_cap) return AFQ_OK;
   AFQ_HIP(hipStreamSynchronize(st));
-  if (need > j->fields_cap) {
-    if (j->fields) (void)hipFree(j->fields);
-    j->fields = nullptr;
-    j->fields_cap = 0;
-    AFQ_TRY(dalloc_n(&j->fields, (size_t)need));
-    j->fields_cap = need;
-  }
   if (hneed > j->h_cap) {
     double* h = nullptr;
     AFQ_TRY(dalloc_n(&h, (size_t)hneed));
     if (j->h_own) (void)hipFree(j->h_own);
     j->h_step = j->h_own = h;
     j->h_cap = hneed;
+  }
+  if (need > j->fields_cap) {
+    if (j->fields) (void)hipFree(j->fields);
+    j->fields = nullptr;
+    j->fields_cap = 0;
+    AFQ_TRY(dalloc_n(&j->fields, (size_t)need));
+    j->fields_cap = need;
   }
   return AFQ_OK;
 }
