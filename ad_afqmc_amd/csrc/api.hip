@@ -317,7 +317,9 @@ int small_cols(const afq_job* j) { return j->restricted ? j->wcols : j->nocc[0] 
 bool small_occ(const afq_job* j) {
   return !j->lp && std::max(j->nocc[0], j->nocc[1]) <= kSmallMaxO && j->wcols <= kSmallMaxO;
 }
-bool small_meas(const afq_job* j) { return small_occ(j) && small_measure_lds(j->N, small_cols(j), small_osum(j), j->nspin_meas) > 0; }
+bool small_meas(const afq_job* j) {
+  return small_occ(j) && small_measure_lds(j->N, small_cols(j), small_osum(j), j->nspin_meas) > 0;
+}
 bool small_whole(const afq_job* j) {
   return small_energy_whole(j->N, j->G, j->nocc[0], j->nspin_meas > 1 ? j->nocc[1] : 0);
 }
@@ -435,7 +437,7 @@ int energy_pipeline(afq_job* j, const void* up, const void* dn, double2* out, hi
                           j->kpart + (long)s * j->W * j->kchunk_max};
   const bool ene1_too = !small && nth == j->nspin_meas;
   if (nth > 0) {
-    ProfScope ps(j, AFQ_K_EXCHANGE, st);
+    ProfScope ps(j, AFQ_K_ENERGY_MISC, st);
     AFQ_TRY(exchange_f64_theta(th, nth, j->N, j->G, j->W, two ? 1.0 : 2.0, ene1_too ? j->ene1 : nullptr, st));
   }
   if (!small && !ene1_too) {
